@@ -534,6 +534,67 @@ __global__ __launch_bounds__(256) void unpack_panel_kernel(const UnpackJob* __re
     }
 }
 
+// C panels of k slices: adds a job's nslice panels up and applies
+// alpha / beta through C's offsets.  A workgroup takes E consecutive elements
+// (row by row) of one job; its threads form SP sets that each add every
+// SP-th slice, and the sets' sums meet in LDS in slice-set order, so that the
+// result does not depend on which workgroup ran when.  Bound by the reads of
+// the panels, or, for a small C with many slices, by their latency: 16 sets
+// keep 16 x 4 loads in flight per element.
+template <typename TC, int SP>
+__global__ __launch_bounds__(SP == 16 ? 1024 : 256) void reduce_slices_kernel(
+    const UnpackJob* __restrict__ jobs, const UnpackChunk* __restrict__ chunks, const int64_t* __restrict__ pool,
+    const double* __restrict__ ws, TC* __restrict__ C, double alpha, double beta)
+{
+    constexpr int NT = SP == 16 ? 1024 : 256, E = NT / SP;
+    const UnpackChunk ch = chunks[blockIdx.x];
+    const UnpackJob j = jobs[ch.job];
+    const int set = threadIdx.x / E, el = threadIdx.x % E;
+    const int e = ch.r0 + el, n = j.nr * j.nc;
+    double sum = 0.0;
+    if (e < n)
+    {
+        const double* p = ws + j.panel + e;
+        int s = set;
+        for (; s + 3 * SP < j.nslice; s += 4 * SP)
+        {
+            const double x0 = p[(int64_t)s * j.sstride], x1 = p[(int64_t)(s + SP) * j.sstride];
+            const double x2 = p[(int64_t)(s + 2 * SP) * j.sstride], x3 = p[(int64_t)(s + 3 * SP) * j.sstride];
+            sum += (x0 + x1) + (x2 + x3);
+        }
+        for (; s < j.nslice; s += SP) sum += p[(int64_t)s * j.sstride];
+    }
+    if constexpr (SP > 1)
+    {
+        __shared__ double part[SP][E];
+        part[set][el] = sum;
+        __syncthreads();
+        if (set > 0) return;
+#pragma unroll
+        for (int q = 1; q < SP; q++) sum += part[q][el];
+    }
+    if (e >= n) return;
+    TC* c = C + j.dst + pool[j.rowmap + e / j.nc] + pool[j.colmap + e % j.nc];
+    double v = alpha * sum;
+    if (beta != 0.0) v += beta * (double)*c;
+    *c = (TC)v;
+}
+
+template <typename TC>
+void launch_reduce(const PanelLaunch& L)
+{
+    auto go = [&](auto* k, int threads) {
+        hipLaunchKernelGGL(k, dim3(L.nuchunks), dim3(threads), 0, L.stream, L.ujobs, L.uchunks, L.pool,
+                           (const double*)L.cws, (TC*)L.C, L.alpha, L.beta);
+    };
+    if (L.slices >= 32)
+        go(&reduce_slices_kernel<TC, 16>, 1024);
+    else if (L.slices >= 8)
+        go(&reduce_slices_kernel<TC, 4>, 256);
+    else
+        go(&reduce_slices_kernel<TC, 1>, 256);
+}
+
 // ------------------------------------------------------------------ fill
 
 // Pseudo-random values in [-1, 1) (a 64-bit mix of the index) so that
@@ -684,6 +745,7 @@ int panel_num_tiles(int family)
     return family == FAMILY_F64 ? kNumTiles + lds_num_tiles() : panel_bf16_num_tiles();
 }
 bool panel_tile_lds(int family, int t) { return family == FAMILY_F64 && t >= kNumTiles; }
+int panel_tile_k(int family, int t) { return panel_tile_lds(family, t) ? lds_tile_k(t - kNumTiles) : 0; }
 int panel_tile_m(int family, int t)
 {
     if (family == FAMILY_OZAKI) return 64;
@@ -733,9 +795,19 @@ hipError_t launch_fill_random(void* p, int64_t n, bool bf16, hipStream_t s)
     return hipGetLastError();
 }
 
+int reduce_chunk_elems(int slices) { return slices >= 8 ? 64 : 256; }
+
 hipError_t launch_panel_unpack(const PanelLaunch& L)
 {
     if (L.nuchunks == 0) return hipSuccess;
+    if (L.slices > 1)
+    {
+        if (L.dtype == 0)
+            launch_reduce<double>(L);
+        else
+            launch_reduce<float>(L);
+        return hipGetLastError();
+    }
     if (L.dtype == 0)
         hipLaunchKernelGGL(unpack_panel_kernel<double>, dim3(L.nuchunks), dim3(256), 0, L.stream,
                            L.ujobs, L.uchunks, L.pool, (const double*)L.cws, (double*)L.C, L.alpha,

@@ -31,6 +31,7 @@ int panel_tile_waves(int family, int tile);
 // FP64 tiles that stage both operands through LDS (every operand read from
 // the tensors, single-block GEMMs only)
 bool panel_tile_lds(int family, int tile);
+int panel_tile_k(int family, int tile);  // gather tiles: k per stage
 struct PanelLaunch
 {
     const PackChunk* chunks;
@@ -52,11 +53,16 @@ struct PanelLaunch
     int family;  // FAMILY_F64 or a split-BF16 family
     int tile;
     bool direct_a, direct_b;  // FP64: operand read from the tensor (PanelTask)
+    int group;                // gather tiles: lanes along k, 1 A + 2 B
+    bool scaled;              // gather tiles: per-k scales (PanelTask::a_kt)
+    int slices;               // most k slices of one GEMM (C panels to add up)
     hipStream_t stream;
 };
 hipError_t launch_panel_pack(const PanelLaunch& L);
 hipError_t launch_panel_gemm(const PanelLaunch& L);
 hipError_t launch_panel_unpack(const PanelLaunch& L);
+// C elements per chunk of a plan with k slices
+int reduce_chunk_elems(int slices);
 // n pseudo-random values in [-1, 1) (double, or BF16 when bf16) at p
 hipError_t launch_fill_random(void* p, int64_t n, bool bf16, hipStream_t s);
 // split-BF16 panels (gemm_panel_bf16.hip)
@@ -66,9 +72,10 @@ int panel_bf16_tile_n(int tile);
 int panel_bf16_tile_waves(int tile);
 bool panel_bf16_tile_fast_only(int tile);
 bool panel_bf16_tile_direct(int tile);  // has variants reading FP32 operands directly
-// FP64 GEMM reading both operands from the tensors through LDS
+// FP64 GEMM gathering both operands from the tensors through LDS
 // (gemm_lds.hip); its tiles follow the register-fed FP64 tiles.
 int lds_num_tiles();
+int lds_tile_k(int lt);  // k per stage
 int lds_tile_m(int lt);
 int lds_tile_n(int lt);
 hipError_t launch_gemm_lds(const PanelLaunch& L, int lt);

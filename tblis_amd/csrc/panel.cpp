@@ -278,6 +278,117 @@ double tile_cost(const std::vector<PanelGemm>& gemms, const TileModel& tm, int c
     return std::max(total / (busy * per_simd), maxtask / (W * simd * tm.eff));
 }
 
+int64_t total_k(const PanelGemm& g)
+{
+    int64_t k = 0;
+    for (auto x : g.klen) k += x;
+    return k;
+}
+
+// Adding the k slices of a plan up: one launch, and the C panels written
+// and read once.
+double reduce_us(double panel_bytes) { return 4.0 + 2.0 * panel_bytes / 4.2e6; }
+
+struct GatherChoice
+{
+    int tile = -1;
+    int slices = 1;
+    double us = 0;
+};
+
+// Best gather tile (gemm_lds.hip; only: that one) and number of k slices
+// for these GEMMs, from a model of a CU that holds up to occ workgroups: a stage takes the
+// MFMA and issue cycles of every resident workgroup's stage, at least the
+// memory latency of the one stage of loads in flight, and a task 1.5 stages
+// more than its k (filling, epilogue).  Cycles per stage and latency fitted
+// to (us, model / measured): 24^4 on tile 10 whole 36 / 34.1, in 3 slices
+// 19 / 20.2, on tile 11 21 / 21.9; the permuted 64/32 contraction 566 / 564,
+// the 8-irrep DPD GEMMs 58 / 59.
+GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int src_elem, int cus, int only = -1)
+{
+    struct Model
+    {
+        int lt, occ;
+        double stage;  // cycles of one workgroup's stage on a CU
+    };
+    constexpr Model models[] = {{1, 4, 1170}, {2, 3, 800}};
+    constexpr double kLatency = 2000, kGHz = 2.15;
+    GatherChoice best;
+    const int first = panel_num_tiles(family) - lds_num_tiles();
+    for (const Model& md : models)
+    {
+        const int tile = first + md.lt;
+        if (only >= 0 && tile != only) continue;
+        const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
+        const int64_t bk = panel_tile_k(family, tile);
+        int64_t kmax = 1;
+        double bytes = 0;
+        for (const PanelGemm& g : gemms)
+        {
+            const int64_t k = total_k(g);
+            kmax = std::max(kmax, k);
+            bytes += (double)src_elem * ((double)g.mlen[0] * k + (double)g.nlen[0] * k + (double)g.mlen[0] * g.nlen[0]);
+        }
+        for (int64_t S = 1; S <= std::min<int64_t>(ceil_div(kmax, 2 * bk), 1024); S += S < 4 ? 1 : S / 4)
+        {
+            const int64_t kslice = ceil_div(ceil_div(kmax, S), bk) * bk;
+            int64_t ntask = 0;
+            double work = 0, panels = 0;
+            for (const PanelGemm& g : gemms)
+            {
+                const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g), s = std::max<int64_t>(1, ceil_div(k, kslice));
+                const int64_t nt = ceil_div(m, BM) * ceil_div(n, BN) * s;
+                ntask += nt;
+                work += (double)nt * (std::min((double)kslice, (double)k) / (double)bk + 1.5) * md.stage;
+                if (s > 1) panels += 8.0 * (double)s * (double)m * (double)n;
+            }
+            if (S > 1 && (panels > (double)(64 << 20) || ntask > 8 * cus)) break;
+            const double st = (double)kslice / (double)bk + 1.5;
+            const int64_t res = std::min<int64_t>(md.occ, ceil_div(ntask, cus));
+            double cyc = st * std::max(res * md.stage, kLatency);
+            if (ntask > md.occ * cus) cyc = std::max(cyc, 1.05 * work / cus);
+            double us = std::max(cyc / (kGHz * 1e3), bytes / 4.2e6) + 3.0;
+            if (panels > 0) us += reduce_us(panels);
+            if (best.tile < 0 || us < best.us) best = GatherChoice{tile, (int)S, us};
+        }
+    }
+    return best;
+}
+
+// Plans that take a gather tile without a measurement: GEMMs whose operands
+// have unit-stride rows or k (others are packed once instead of gathered by
+// every tile) and that the register-fed tiles serve badly (us, register tile
+// / gather tile, same box).
+//   Long k and few C tiles (under two 32 x 32 tiles per CU): without k
+//   slices the chip is idle.  32 x 32 x 131072 3125 / 22.6, 50 x 50 x 22785
+//   558 / 15.3, 16 x 16 x 2560 41 / 8.2.
+//   One to two 32 x 32 tiles per CU: the register tile runs a second,
+//   nearly empty round.  24^4 (324 tiles) 27.3 / 22.0; up to one round it
+//   is the better one at this k (22^4, 256 tiles: 13.4 / 17.4; 10^4 6.7 / 6.8).
+//   Short k (up to 64): packing an operand moves as many bytes as the
+//   contraction itself.  64 x 65536 x 32 34.2 / 20.4, 70 x 112000 x 40 75 /
+//   55; not where the 64 x 64 tile is mostly padding (33 x 14553 x 21 13.3 /
+//   13.9).
+bool gather_preferred(const std::vector<PanelGemm>& gemms, int cus)
+{
+    int64_t tiles = 0, kmax = 0;
+    double area = 0, padded = 0;
+    for (const PanelGemm& g : gemms)
+    {
+        const int64_t m = g.mlen[0], n = g.nlen[0];
+        tiles += ceil_div(m, 32) * ceil_div(n, 32);
+        area += (double)m * (double)n;
+        padded += 4096.0 * (double)(ceil_div(m, 64) * ceil_div(n, 64));
+        kmax = std::max(kmax, total_k(g));
+        for (const std::vector<PBlock>* bl : {&g.a, &g.b})
+            for (const PBlock& b : *bl)
+                if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1)
+                    return false;
+    }
+    if (tiles < 2 * cus) return tiles > cus || kmax >= 1024;
+    return kmax <= 64 && padded <= 1.6 * area;
+}
+
 }  // namespace
 
 void debug_side_tables(const Side& s, int64_t G, int64_t r0, std::vector<int64_t>& offs,
@@ -461,6 +572,9 @@ namespace
 // operands)
 bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T,
                      const bool allow_direct[2], int src_elem);
+int ksplit_forced();
+bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
+                   int64_t kslice);
 // tables_for_tile with the tasks grouped by which operands they read
 // directly (one kernel variant per launch); packed: every operand packed
 bool tables_uniform(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
@@ -530,15 +644,25 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         if (family == FAMILY_BF16X3 && panel_bf16_tile_fast_only(tm.tile)) continue;
         if (panel_tile_lds(family, tm.tile) && !lds_applicable(gemms, dtype == 0 ? 8 : 4)) continue;
         cands.push_back(tm.tile);
-        // the LDS-staged tiles measured slower than the register tiles on
-        // every workload (permuted 64/32, 8-irrep DPD, 4096-instance batch):
-        // the tuner times them, the cost model does not pick them
-        if (panel_tile_lds(family, tm.tile)) continue;
+        if (panel_tile_lds(family, tm.tile)) continue;  // gather tiles have a model of their own
         double c = tile_cost(gemms, tm, cus, family);
         if (best < 0 || c < best)
         {
             best = c;
             tile = tm.tile;
+        }
+    }
+    // Gather tiles: chosen by their model where the register-fed tiles do
+    // badly; not for plans in caller storage, whose size limit a plan's
+    // panels are held against.
+    {
+        char* sbase = nullptr;
+        size_t sbytes = 0;
+        static_storage(sbase, sbytes);
+        if (family == FAMILY_F64 && !sbase && lds_applicable(gemms, dtype == 0 ? 8 : 4) && gather_preferred(gemms, cus))
+        {
+            const GatherChoice c = gather_choice(gemms, family, dtype == 0 ? 8 : 4, cus);
+            tile = c.tile;
         }
     }
     bool packed = false;
@@ -575,6 +699,15 @@ bool tables_uniform(const std::vector<PanelGemm>& gemms, int family, int tile, P
 {
     const bool allow[2] = {!packed, !packed};
     T = PanelTables();
+    if (panel_tile_lds(family, tile))
+    {
+        int64_t kmax = 1;
+        for (const PanelGemm& g : gemms) kmax = std::max(kmax, total_k(g));
+        const int64_t bk = panel_tile_k(family, tile);
+        int64_t S = ksplit_forced();
+        if (!S) S = gather_choice(gemms, family, src_elem, device_cu_count(), tile).slices;
+        return gather_tables(gemms, family, tile, T, src_elem, ceil_div(ceil_div(kmax, S), bk) * bk);
+    }
     if (!tables_for_tile(gemms, family, tile, T, allow, src_elem)) return false;
     auto group = [](const PanelTask& t) {
         return (t.a_src != PANEL_MISSING ? 1 : 0) + (t.b_src != PANEL_MISSING ? 2 : 0);
@@ -618,31 +751,33 @@ void side_range(const Side& s, int64_t& lo, int64_t& hi)
     }
 }
 
+bool same_side(const Side& a, const Side& b) { return a.len == b.len && a.stride == b.stride && a.offs == b.offs; }
+
 }  // namespace
 
-// Can the LDS-staged tiles run these GEMMs: direct reads enabled, single
-// A, B and C blocks, k > 0, unscaled, both operands within a buffer
-// resource's reach (non-negative offsets, under 2 GiB from the block's
-// base).
 bool lds_applicable(const std::vector<PanelGemm>& gemms, int src_elem)
 {
     if (!direct_enabled()) return false;
     for (const PanelGemm& g : gemms)
     {
-        if (g.mlen.size() != 1 || g.nlen.size() != 1 || g.klen.size() != 1 || g.c.size() != 1) return false;
-        if (g.klen[0] <= 0) return false;
+        if (g.mlen.size() != 1 || g.nlen.size() != 1 || g.c.size() != 1) return false;
         if (g.a.size() != g.klen.size() || g.b.size() != g.klen.size()) return false;
-        for (double x : g.kscale)
-            if (x != 1.0) return false;
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
+        {
+            if (bl->empty()) continue;
+            // rows and k offsets (block bases included) in 32-bit bytes
+            int64_t rlo, rhi, klo = 0, khi = 0;
+            side_range((*bl)[0].rows, rlo, rhi);
             for (const PBlock& b : *bl)
             {
-                if (b.base == PANEL_MISSING) return false;
-                int64_t rlo, rhi, klo, khi;
-                side_range(b.rows, rlo, rhi);
-                side_range(b.k, klo, khi);
-                if (rlo < 0 || klo < 0 || (rhi + khi + 1) * src_elem >= ((int64_t)1 << 31)) return false;
+                if (b.base == PANEL_MISSING || !same_side(b.rows, (*bl)[0].rows)) return false;
+                int64_t lo, hi;
+                side_range(b.k, lo, hi);
+                klo = std::min(klo, b.base - (*bl)[0].base + lo);
+                khi = std::max(khi, b.base - (*bl)[0].base + hi);
             }
+            if ((rhi - rlo + khi - klo + 1) * src_elem >= ((int64_t)1 << 32)) return false;
+        }
     }
     return true;
 }
@@ -662,15 +797,235 @@ bool direct_all(const std::vector<PanelGemm>& gemms)
     return e && e[0] == '1' && gemms.size() > 1;
 }
 
+// The tile grid of one GEMM in task order.
+// XCD regions: the grid cut into RM x RN rectangles (RM * RN <= 8), the cut
+// that loads the fewest panel rows per region.  In plans of many GEMMs
+// (batches) each GEMM is one region: its tiles then share one XCD's L2,
+// where a cut GEMM has each XCD fetch its own copy of the operands, and the
+// many GEMMs balance the XCDs.
+// Tiles in groups of G rows, columns walked with the rows fastest: the tiles
+// an XCD runs at once then share G row panels of A' and a few column panels
+// of B' in its L2, where a row-major walk would share one A' panel and
+// stream a new B' panel per tile.
+struct TileWalk
+{
+    int64_t MT, NT, RM = 1, RN = 1, GR;
+    TileWalk(int64_t mt, int64_t nt, int64_t mp, int64_t np, size_t ngemms)
+        : MT(mt), NT(nt), GR(std::max<int64_t>(1, tile_group_rows()))
+    {
+        if ((int64_t)ngemms >= whole_gemm_regions()) return;
+        int64_t best = -1;
+        for (int64_t rm = 1; rm <= kXcds; rm *= 2)
+        {
+            const int64_t rn = kXcds / rm;
+            if (rm > MT || rn > NT) continue;
+            const int64_t load = mp / rm + np / rn;
+            if (best < 0 || rm * rn > RM * RN || (rm * rn == RM * RN && load < best))
+            {
+                best = load;
+                RM = rm;
+                RN = rn;
+            }
+        }
+    }
+    void at(int64_t pid, int64_t& tm, int64_t& tn) const
+    {
+        const int64_t first = pid / (GR * NT) * GR, gm = std::min(GR, MT - first);
+        const int64_t local = pid % (GR * NT);  // < gm * NT
+        tm = first + local % gm;
+        tn = local / gm;
+    }
+    int64_t region(int64_t tm, int64_t tn) const { return (tm * RM / MT) * RN + tn * RN / NT; }
+};
+
+// Share of neighbouring offsets that are one element apart.
+double unit_share(const std::vector<int64_t>& off)
+{
+    int64_t c = 0;
+    const int64_t n = (int64_t)off.size();
+    for (int64_t i = 0; i + 1 < n; i++) c += off[i + 1] - off[i] == 1;
+    return n > 1 ? (double)c / (double)(n - 1) : 0.0;
+}
+
+// Offsets of a side in odometer order.
+std::vector<int64_t> side_offsets(const Side& s)
+{
+    if (!s.offs.empty()) return s.offs;
+    Pool p;
+    const int64_t at = p.offsets(s);
+    return std::vector<int64_t>(p.data().begin() + at, p.data().begin() + at + side_len(s));
+}
+
+// k slices per GEMM forced by TBLIS_HIP_KSPLIT (read at every plan build), or 0.
+int ksplit_forced()
+{
+    const char* e = std::getenv("TBLIS_HIP_KSPLIT");
+    const int v = e ? std::atoi(e) : 0;
+    return v >= 1 ? std::min(v, 4096) : 0;
+}
+
+// Tables of a plan on a gather tile (gemm_lds.hip): tasks and, for GEMMs cut
+// along k, the jobs that add their C panels up.  kslice: k per task.
+bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
+                   int64_t kslice)
+{
+    const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
+    Pool pool;
+    std::vector<int64_t> cost, region;
+    std::vector<int> group;
+    std::vector<PanelTask> all;
+    int64_t nregions = 0, wsc = 0;
+    for (const PanelGemm& g : gemms)
+        for (double x : g.kscale) T.scaled |= x != 1.0;
+    for (const PanelGemm& g : gemms)
+    {
+        const int64_t m = g.mlen[0], n = g.nlen[0];
+        int64_t k = 0;
+        for (auto x : g.klen) k += x;
+        if (m == 0 || n == 0) continue;
+        const int64_t MT = ceil_div(m, BM), NT = ceil_div(n, BN), mp = MT * BM, np = NT * BN;
+        if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX / 2) fail("contraction too large for one GEMM");
+        T.useful_flops += 2 * m * n * k;
+        T.mfma_flops += 2 * mp * np * (ceil_div(k, 4) * 4);
+        if (k > 0) T.reads_ab = true;
+        int64_t rt[2] = {0, 0}, km[2] = {0, 0}, src[2] = {0, 0}, scales = 0;
+        int kl = 0;
+        if (k > 0)
+        {
+            const std::vector<PBlock>* blocks[2] = {&g.a, &g.b};
+            for (int o = 0; o < 2; o++)
+            {
+                // byte offsets from the operand's lowest element
+                const std::vector<PBlock>& bl = *blocks[o];
+                Side rows, ks;
+                rows.offs = side_offsets(bl[0].rows);
+                for (size_t q = 0; q < bl.size(); q++)
+                    for (int64_t x : side_offsets(bl[q].k)) ks.offs.push_back(bl[q].base - bl[0].base + x);
+                if (unit_share(ks.offs) > unit_share(rows.offs)) kl |= 1 << o;
+                src[o] = bl[0].base;
+                for (Side* s : {&rows, &ks})
+                {
+                    const int64_t lo = *std::min_element(s->offs.begin(), s->offs.end());
+                    src[o] += lo;
+                    for (int64_t& x : s->offs) x = (x - lo) * src_elem;
+                }
+                // the kernels read offsets up to four stages past a task's end
+                ks.offs.insert(ks.offs.end(), (size_t)(4 * panel_tile_k(family, tile)), ks.offs.back());
+                rt[o] = pool.offsets(rows);
+                km[o] = pool.offsets(ks);
+            }
+            if (T.scaled)
+            {
+                std::vector<int64_t> sc;
+                for (size_t q = 0; q < g.klen.size(); q++)
+                {
+                    const double x = g.kscale.empty() ? 1.0 : g.kscale[q];
+                    int64_t bits;
+                    std::memcpy(&bits, &x, sizeof bits);
+                    sc.insert(sc.end(), (size_t)g.klen[q], bits);
+                }
+                sc.insert(sc.end(), (size_t)(4 * panel_tile_k(family, tile)), 0);
+                scales = pool.push(sc);
+            }
+        }
+        const int64_t S = std::max<int64_t>(1, ceil_div(k, kslice));
+        const int64_t crow = pool.offsets(g.c[0].rows), ccol = pool.offsets(g.c[0].cols);
+        const int64_t oc = wsc;
+        if (S > 1)
+        {
+            wsc += S * m * n;
+            UnpackJob u{};
+            u.dst = g.c[0].base;
+            u.rowmap = crow;
+            u.colmap = ccol;
+            u.panel = oc;
+            u.nr = (int32_t)m;
+            u.nc = (int32_t)n;
+            u.ld = (int32_t)n;
+            u.sstride = m * n;
+            u.nslice = (int32_t)S;
+            T.ujobs.push_back(u);
+            T.slices = std::max<int>(T.slices, (int)S);
+        }
+        const TileWalk W(MT, NT, mp, np, gemms.size());
+        for (int64_t s = 0; s < S; s++)
+        {
+            for (int64_t pid = 0; pid < MT * NT; pid++)
+            {
+                int64_t tm, tn;
+                W.at(pid, tm, tn);
+                region.push_back(nregions + W.region(tm, tn));
+                PanelTask t{};
+                t.kbeg = (int32_t)std::min(k, s * kslice);
+                t.klen = (int32_t)std::min(k, (s + 1) * kslice);
+                t.a_src = src[0];
+                t.b_src = src[1];
+                t.a_rt = rt[0] + tm * BM;
+                t.b_rt = rt[1] + tn * BN;
+                t.a_km = km[0];
+                t.b_km = km[1];
+                t.a_kt = scales;
+                t.mlen = (int32_t)std::min<int64_t>(BM, m - tm * BM);
+                t.nlen = (int32_t)std::min<int64_t>(BN, n - tn * BN);
+                if (S > 1)
+                {
+                    t.c_src = oc + s * m * n + tm * BM * n + tn * BN;
+                    t.c_ld = (int32_t)n;
+                }
+                else
+                {
+                    t.c_src = g.c[0].base;
+                    t.c_rowmap = crow + tm * BM;
+                    t.c_colmap = ccol + tn * BN;
+                }
+                all.push_back(t);
+                group.push_back(kl);
+                cost.push_back(std::max<int64_t>(t.klen - t.kbeg, 1) * t.mlen * t.nlen);
+            }
+            nregions += W.RM * W.RN;
+        }
+    }
+    if (all.empty()) return false;
+    for (size_t j = 0; j < T.ujobs.size(); j++)
+    {
+        const int64_t n = (int64_t)T.ujobs[j].nr * T.ujobs[j].nc, per = reduce_chunk_elems(T.slices);
+        if (n > INT32_MAX) fail("contraction too large for one GEMM");
+        for (int64_t e = 0; e < n; e += per) T.uchunks.push_back(UnpackChunk{(int32_t)j, (int32_t)e, 0, 0});
+    }
+    if (all.size() > (size_t)INT32_MAX || T.uchunks.size() > (size_t)INT32_MAX)
+        fail("contraction too large: panel task list exceeds 2^31 entries");
+    // one launch per combination of lanes along rows and along k
+    for (int q = 0; q < 4; q++)
+    {
+        std::vector<PanelTask> ts;
+        std::vector<int64_t> tc, tr;
+        for (size_t i = 0; i < all.size(); i++)
+            if (group[i] == q)
+            {
+                ts.push_back(all[i]);
+                tc.push_back(cost[i]);
+                tr.push_back(region[i]);
+            }
+        if (ts.empty()) continue;
+        ts = xcd_order(ts, tc, tr, nregions);
+        T.tasks.insert(T.tasks.end(), ts.begin(), ts.end());
+        T.group_n[q] = T.sched.group_n[0][q] = (int64_t)ts.size();
+    }
+    T.task_stage.assign(T.tasks.size(), 0);
+    T.direct[0] = T.direct[1] = true;
+    T.ws_c = wsc;
+    T.family = family;
+    T.tile = tile;
+    T.pool = std::move(pool.data());
+    return true;
+}
+
 bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T,
                      const bool allow_direct[2], int src_elem)
 {
     const Geom G = geom_of(family);
-    // LDS-staged tiles read both operands from the tensors (lds_applicable
-    // has checked that they can)
-    const bool lds = panel_tile_lds(family, tile);
     const bool scoped = t_direct_all && family == FAMILY_F64;
-    const bool general = direct_all(gemms) || lds || scoped;
+    const bool general = direct_all(gemms) || scoped;
     const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
 
     Pool pool;
@@ -795,7 +1150,6 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
         const int64_t rtot[2] = {m, n};
         bool dir[2] = {false, false};
         int64_t drt[2] = {0, 0}, dkt[2] = {0, 0}, dkm[2] = {0, 0}, dsrc[2] = {0, 0};
-        int32_t dkf[2] = {0, 0};
         uint32_t dbytes[2] = {0, 0};
         // split-BF16 reads FP32 operands directly (split in registers) on
         // the tiles that have such variants, for many GEMMs only
@@ -806,7 +1160,7 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
             if (o == 0 && !g.kscale.empty() && g.kscale[0] != 1.0) continue;  // scaled while packed
             const int64_t rereads = o == 0 ? ceil_div(n, BN) : ceil_div(m, BM);
             if (!general && rereads > std::max<int64_t>(direct_rows_rereads(), direct_kfast_rereads())) continue;
-            if (scoped && !lds && rereads > 64) continue;
+            if (scoped && rereads > 64) continue;
             const PBlock& blk = (*blocks[o])[0];
             if (blk.base == PANEL_MISSING) continue;
             const int64_t rm = pool.offsets(blk.rows), km = pool.offsets(blk.k);
@@ -817,16 +1171,6 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
             for (int64_t i = 0; i < k; i++) klo = std::min(klo, pd[km + i]), khi = std::max(khi, pd[km + i]);
             if (lo < 0 || klo < 0 || (hi + khi + 1) * src_elem >= ((int64_t)1 << 31)) continue;
             const int64_t kt = pool.group_table(km, 0, k, G.gk);
-            {
-                // lanes of the LDS-staged loads run along k when more k
-                // groups than row groups are unit-stride
-                const int64_t rt = pool.group_table(rm, 0, rtot[o], G.gr);
-                const int64_t* q = pool.data().data();
-                int64_t ru = 0, ku = 0;
-                for (int64_t gi = 0; gi < ceil_div(rtot[o], G.gr); gi++) ru += q[rt + 2 * gi + 1] == 1;
-                for (int64_t gi = 0; gi < ceil_div(k, G.gk); gi++) ku += q[kt + 2 * gi + 1] == 1;
-                dkf[o] = ku * ceil_div(rtot[o], G.gr) > ru * ceil_div(k, G.gk) ? 1 : 0;
-            }
             if (!general)
             {
                 const int64_t rt = pool.group_table(rm, 0, rtot[o], G.gr);
@@ -865,9 +1209,6 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
             dsrc[o] = blk.base;
             dbytes[o] = (uint32_t)((hi + khi + 1) * src_elem);
         }
-
-        if (lds && !(dir[0] && dir[1] && g.c.size() == 1))
-            fail("internal: LDS-staged tile without both operands read directly or without a single C block");
 
         // panels
         const int64_t oa = ws;
@@ -985,41 +1326,13 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
                         for (int32_t c = 0; c < u.nc; c += 64) uchunks.push_back(UnpackChunk{id, r, c, 0});
                 }
         }
-        // XCD regions: the tile grid cut into RM x RN rectangles (RM * RN <= 8),
-        // the cut that loads the fewest panel rows per region.  In plans of
-        // many GEMMs (batches) each GEMM is one region: its tiles then share
-        // one XCD's L2, where a cut GEMM has each XCD fetch its own copy of
-        // the operand panels, and the many GEMMs balance the XCDs.
-        const int64_t MT = mp / BM, NT = np / BN;
-        int64_t RM = 1, RN = 1;
-        if ((int64_t)gemms.size() < whole_gemm_regions())
+        const TileWalk W(mp / BM, np / BN, mp, np, gemms.size());
+        for (int64_t pid = 0; pid < W.MT * W.NT; pid++)
         {
-            int64_t best = -1;
-            for (int64_t rm = 1; rm <= kXcds; rm *= 2)
+            int64_t tm, tn;
+            W.at(pid, tm, tn);
             {
-                const int64_t rn = kXcds / rm;
-                if (rm > MT || rn > NT) continue;
-                const int64_t load = mp / rm + np / rn;
-                if (best < 0 || rm * rn > RM * RN || (rm * rn == RM * RN && load < best))
-                {
-                    best = load;
-                    RM = rm;
-                    RN = rn;
-                }
-            }
-        }
-        // Tiles in groups of G rows, columns walked with the rows fastest:
-        // the tiles an XCD runs at once then share G row panels of A' and
-        // a few column panels of B' in its L2, where a row-major walk would
-        // share one A' panel and stream a new B' panel per tile.
-        const int64_t GR = std::max<int64_t>(1, tile_group_rows());
-        for (int64_t pid = 0; pid < MT * NT; pid++)
-        {
-            const int64_t first = pid / (GR * NT) * GR, gm = std::min(GR, MT - first);
-            const int64_t local = pid % (GR * NT);  // < gm * NT
-            const int64_t tm = first + local % gm, tn = local / gm;
-            {
-                region.push_back(nregions + (tm * RM / MT) * RN + tn * RN / NT);
+                region.push_back(nregions + W.region(tm, tn));
                 PanelTask t{};
                 const int64_t ge = (int64_t)G.terms * G.gr * G.gk;  // values per group
                 t.a = oa + tm * (BM / G.gr) * nkg * ge;
@@ -1033,7 +1346,6 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
                 t.b_kt = dkt[1];
                 t.a_km = dkm[0];
                 t.b_km = dkm[1];
-                t.pad_ = dkf[0] | (dkf[1] << 1);  // LDS-staged loads: lanes along k
                 t.a_bytes = dbytes[0];
                 t.b_bytes = dbytes[1];
                 t.nkg = (int32_t)nkg;
@@ -1063,7 +1375,7 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
                 cost.push_back(std::max<int64_t>(nkg, 1) * t.mlen * t.nlen);
             }
         }
-        nregions += RM * RN;
+        nregions += W.RM * W.RN;
     }
     if (tasks.empty()) return false;
     const int forced = pack_chunks_forced();
@@ -1333,7 +1645,7 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
         if (real ? !tables_uniform(gemms, family, c, T1, dtype == 0 ? 8 : 4)
                  : !tables_for_tile(gemms, family, c, T1, none, dtype == 0 ? 8 : 4))
             return -1;
-        const bool reads = T1.group_n[1] + T1.group_n[2] + T1.group_n[3] > 0;
+        const bool reads = panel_tile_lds(family, c) || T1.group_n[1] + T1.group_n[2] + T1.group_n[3] > 0;
         cands.push_back(c);
         tabs.push_back(std::move(T1));
         if (real && reads && !t_direct_all && !panel_tile_lds(family, c))
@@ -1438,6 +1750,8 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
                 G.ntasks = (int)sc.group_n[st][g];
                 G.direct_a = (g & 1) != 0;
                 G.direct_b = (g & 2) != 0;
+                G.group = g;
+                G.scaled = tabs[i].scaled;
                 if (launch_panel_gemm(G) != hipSuccess) return false;
                 at += sc.group_n[st][g];
             }
@@ -1465,6 +1779,8 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
     {
         t[i] = time_of(i, 3);
         ok = t[i] >= 0;
+        // the timed launches leave the k slices' panels as they are
+        if (tabs[i].slices > 1) t[i] += (float)(1e-3 * reduce_us(8.0 * (double)tabs[i].ws_c));
     }
     int best_tile = -1;
     std::vector<size_t> fin;    // finalists
@@ -1497,6 +1813,7 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
                     ok = ok1 && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
                          hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
                     ms /= (float)n;
+                    if (tabs[fin[f]].slices > 1) ms += (float)(1e-3 * reduce_us(8.0 * (double)tabs[fin[f]].ws_c));
                     if (ok && (steady[f] < 0 || ms < steady[f])) steady[f] = ms;
                 }
             if (ok)
@@ -1596,6 +1913,8 @@ bool build_panel_plan(Plan& plan, std::vector<PanelGemm> gemms, int elem_size, i
     plan.direct[0] = T.direct[0];
     plan.direct[1] = T.direct[1];
     for (int g = 0; g < 4; g++) plan.group_n[g] = T.group_n[g];
+    plan.scaled = T.scaled;
+    plan.slices = T.slices;
     plan.sched = T.sched;
     plan.key.family = family;
     plan.key.dtype = dtype;

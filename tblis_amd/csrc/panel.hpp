@@ -81,6 +81,8 @@ struct PanelTables
     // tasks come in four consecutive groups by which operands they read from
     // the tensors (none, A, B, both); one GEMM launch per non-empty group
     int64_t group_n[4] = {0, 0, 0, 0};
+    bool scaled = false;  // gather tiles: some k block is scaled
+    int slices = 1;       // gather tiles: most k slices of one GEMM
     // chunks and tasks ordered by stage: sched.chunks[s] pack chunks and
     // sched.group_n[s][g] tasks of group g in stage s (group-major within
     // the stage); task_stage is each task's stage (host bookkeeping)
@@ -92,8 +94,9 @@ struct PanelTables
     int64_t useful_flops = 0, mfma_flops = 0;
 };
 
-// Can the LDS-staged FP64 tiles run these GEMMs (single blocks, operands in
-// reach of a buffer resource)?  src_elem: bytes per tensor element.
+// Can the gather tiles (gemm_lds.hip) run these GEMMs: direct reads enabled,
+// one row block per operand, one C block, the same rows in every k block, and
+// each operand's offsets within 4 GiB?  src_elem: bytes per tensor element.
 bool lds_applicable(const std::vector<PanelGemm>& gemms, int src_elem);
 
 // Orientation, tile, pack jobs, tasks and C unpack jobs (host only).

@@ -349,6 +349,7 @@ void launch_panel_calls(const PanelLaunch& P, const PanelSchedule& S, bool overl
             G.ntasks = (int)S.group_n[s][g];
             G.direct_a = (g & 1) != 0;
             G.direct_b = (g & 2) != 0;
+            G.group = g;
             hip_check(launch_panel_gemm(G), "kernel launch");
             at += S.group_n[s][g];
         }
@@ -386,6 +387,8 @@ void run_plan(const std::shared_ptr<Plan>& pp, const void* A, const void* B, voi
     P.family = p.key.family;
     P.direct_a = p.direct[0];
     P.direct_b = p.direct[1];
+    P.scaled = p.scaled;
+    P.slices = p.slices;
     P.alpha = alpha;
     P.beta = beta;
     P.use_k = use_k && p.reads_ab ? 1 : 0;

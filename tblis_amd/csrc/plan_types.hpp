@@ -81,6 +81,11 @@ struct PackChunk
 // group's (base + lane k * stride) or, for a group that is not affine
 // (stride SCATTERED), its own k offset; lanes past the valid rows or k read
 // offset 0xffffffff, which the buffer bounds check returns as zero.
+// The gather tiles (gemm_lds.hip) read both operands from the tensors with
+// a_src / b_src the operand's lowest element, a_rt / b_rt the tile's first
+// row offset and a_km / b_km the per-k offsets (block bases included) in
+// bytes from it, a_kt the per-k scales (as doubles) in scaled plans; k runs
+// over [kbeg, klen).
 struct PanelTask
 {
     int64_t a, b;        // workspace offsets (values) of the tile's first row block of A', B'
@@ -103,20 +108,25 @@ struct PanelTask
     int64_t a_kt, b_kt;    // pool index of k group 0's (base, stride)
     int64_t a_km, b_km;    // pool index of the per-element k offsets
     uint32_t a_bytes, b_bytes;  // extent of the block from x_src
-    int32_t klen;          // valid k
-    int32_t pad_;
+    int32_t klen;          // valid k (end of the task's k range)
+    int32_t kbeg;          // first k (gather tiles: one k slice of the tile)
 };
 
 // C panel -> C block: C[dst + rowmap[i] + colmap[j]] = alpha * P[i * ld + j] + beta * C[...]
+// With nslice > 1 the panel is the sum of nslice panels, sstride apart.
 struct UnpackJob
 {
     int64_t dst, rowmap, colmap, panel;
     int32_t nr, nc, ld, rows_fast;
+    int64_t sstride;
+    int32_t nslice, pad;
 };
 
 struct UnpackChunk
 {
-    int32_t job, r0, c0, pad;  // 64 x 64 element sub-block
+    // 64 x 64 element sub-block; in plans with k slices r0 is the first of
+    // the chunk's elements, counted row by row
+    int32_t job, r0, c0, pad;
 };
 
 // Kernel families.

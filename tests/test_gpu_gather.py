@@ -1,0 +1,116 @@
+"""The gather tiles (both operands read from the tensors through LDS) and the
+k slices of GEMMs with few C tiles, against the oracle.
+
+Sizes sit where the kernels can go wrong: one row or column, tile edges and
+one past them, k below, at and past a stage and a slice, slices that a short
+k leaves without work, rows and k in odd strides, several k blocks with
+scales (complex and indexed contractions).  FP64 bar: 1e-12 relative
+Frobenius error, the repository's bound for every FP64 path (the sums here
+have at most 1100 terms, whose rounding stays under 1e-13 of the norm)."""
+import numpy as np
+import pytest
+import torch
+
+import tblis_amd as T
+from tests.test_gpu_parity import DEV, FP64_TOL, _dense_case, rel_fro
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def plans(monkeypatch):
+    """Set knobs for plans built in the test; no plan outlives it."""
+    T.lib().tblis_hip_clear_plan_cache()
+    yield monkeypatch
+    T.lib().tblis_hip_clear_plan_cache()
+
+
+@pytest.mark.parametrize("slices", ["1", "2", "5", "40"])
+@pytest.mark.parametrize("tile", ["9", "10", "11"])
+def test_gather_tiles_in_slices(tile, slices, plans):
+    plans.setenv("TBLIS_HIP_PANEL_TILE", tile)
+    plans.setenv("TBLIS_HIP_KSPLIT", slices)
+    rng = np.random.default_rng(71000 + int(tile) * 100 + int(slices))
+    for m, n, k in [(1, 1, 1), (1, 65, 17), (64, 1, 33), (32, 32, 16), (33, 31, 15), (65, 64, 32), (129, 127, 47),
+                    (40, 24, 1100)]:
+        kinds = ["col", "row", "random"]
+        rng.shuffle(kinds)
+        _dense_case(rng, "ak", "kb", "ab", dict(a=m, b=n, k=k), kinds, alpha=1.5, beta=-0.5)
+        assert T.last_tile() == int(tile)
+    # k of several dimensions in another order than the rows', odd extents
+    _dense_case(rng, "eafb", "jefi", "iabj", dict(a=7, b=9, e=5, f=13, i=3, j=11), ["col"] * 3, beta=0.0)
+    _dense_case(rng, "aebf", "fjei", "aibj", dict(a=12, b=10, e=9, f=11, i=7, j=13), ["col"] * 3,
+                dtype=np.float32, config="fp64_mfma", tol=2e-7)
+
+
+@pytest.mark.parametrize("slices", ["1", "3"])
+@pytest.mark.parametrize("tile", ["9", "10", "11"])
+def test_gather_scaled_blocks(tile, slices, plans):
+    """Complex contractions are two k blocks per GEMM, one of them negated;
+    indexed ones a block per matching pair, scaled by the entries' factors."""
+    from tests.test_gpu_complex import _case
+    plans.setenv("TBLIS_HIP_PANEL_TILE", tile)
+    plans.setenv("TBLIS_HIP_KSPLIT", slices)
+    rng = np.random.default_rng(72000 + int(tile) * 10 + int(slices))
+    _case(rng, "aebf", "fjei", "aibj", dict(a=9, b=7, e=5, f=6, i=4, j=11), torch.complex128, 0.5 - 0.25j, 1.0,
+          conj_B=True)
+    assert T.last_tile() == int(tile)
+    d = [torch.rand(6, 35, 21, dtype=torch.float64, device=DEV) - 0.5 for _ in range(2)]
+    fa, fb = [0.5, -1.0, 2.0, 1.0, 0.25, 3.0], [1.0, 1.5, -0.5, 1.0, 2.0, -1.0]
+    A = T.Indexed([x for x in d[0]], [(i,) for i in range(6)], [8], fa)
+    B = T.Indexed([x for x in d[1]], [(i + 1,) for i in range(6)], [8], fb)
+    c = torch.zeros(35, 35, dtype=torch.float64, device=DEV)
+    T.indexed_mult(1.0, A, "aef", B, "bef", 0.0, T.Indexed([c], [()], []), "ab")
+    torch.cuda.synchronize()
+    want = sum(fa[i + 1] * fb[i] * (d[0][i + 1].cpu() @ d[1][i].cpu().T) for i in range(5))
+    assert rel_fro(c.cpu().numpy(), want.numpy()) <= FP64_TOL
+
+
+@pytest.mark.parametrize("m,n,k", [(32, 32, 8192), (1, 1, 5000), (3, 65, 4097), (64, 32768, 32),
+                                   (60, 36001, 63), (513, 600, 70)])
+def test_gather_chosen_by_shape(m, n, k, plans):
+    """Long sums into few results and short sums into many take the gather
+    tiles without a knob, and TBLIS_HIP_DIRECT=0 packs as before."""
+    g = torch.Generator(device=DEV).manual_seed(73000 + k)
+    A = torch.rand(k, m, dtype=torch.float64, device=DEV, generator=g).t() - 0.5
+    B = torch.rand(n, k, dtype=torch.float64, device=DEV, generator=g).t() - 0.5
+    C0 = torch.rand(n, m, dtype=torch.float64, device=DEV, generator=g).t()
+    want = 0.5 * (A.cpu().numpy() @ B.cpu().numpy()) + 2.0 * C0.cpu().numpy()
+    for direct, both in (("1", True), ("0", False)):
+        plans.setenv("TBLIS_HIP_DIRECT", direct)
+        T.lib().tblis_hip_clear_plan_cache()
+        C = C0.clone()
+        T.mult(0.5, A, "ak", B, "kb", 2.0, C, "ab")
+        torch.cuda.synchronize()
+        assert (T.last_tile() >= 9) == both
+        assert rel_fro(C.cpu().numpy(), want) <= FP64_TOL
+
+
+def test_sliced_call_in_a_graph(plans):
+    """A plan cut along k is two launches and a workspace: captured once, and
+    every replay agrees with the eager call while eager calls run between."""
+    g = torch.Generator(device=DEV).manual_seed(74000)
+    A = torch.rand(20000, 24, dtype=torch.float64, device=DEV, generator=g) - 0.5
+    B = torch.rand(20000, 40, dtype=torch.float64, device=DEV, generator=g) - 0.5
+    want = A.cpu().numpy().T @ B.cpu().numpy()
+    C = torch.zeros(24, 40, dtype=torch.float64, device=DEV)
+    D = torch.zeros(24, 40, dtype=torch.float64, device=DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    T.set_stream(side.cuda_stream)
+    try:
+        T.mult(1.0, A, "km", B, "kn", 0.0, C, "mn")
+        assert T.last_tile() >= 9
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            T.mult(1.0, A, "km", B, "kn", 0.0, C, "mn")
+    finally:
+        T.set_stream(0)
+    for _ in range(4):
+        C.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_fro(C.cpu().numpy(), want) <= FP64_TOL
+        T.mult(2.0, A, "km", B, "kn", 0.0, D, "mn")
+        torch.cuda.synchronize()
+        assert rel_fro(D.cpu().numpy(), 2.0 * want) <= FP64_TOL
