@@ -135,6 +135,9 @@ std::vector<int64_t> all_offsets(const Group& g, int slot)
     return out;
 }
 
+// Both tensors start on 16 bytes (plans may read them in 16-byte pieces).
+bool aligned16(const void* a, const void* b) { return (((uintptr_t)a | (uintptr_t)b) & 15) == 0; }
+
 // The GEMM of one canonical dense contraction (m = AC, n = BC, k = AB,
 // batch = ABC), with bases added for batched calls.
 int dtype_code(type_t t) { return t == TYPE_DOUBLE ? 0 : 1; }
@@ -239,6 +242,8 @@ void tensor_mult(const tblis_config* cfg, const tblis_tensor* A, const label_typ
 
     std::string key;
     put(key, (int32_t)algo);
+    const bool aligned = aligned16(A->data, B->data);
+    put(key, aligned);
     tensor_key(key, *A, idx_A);
     tensor_key(key, *B, idx_B);
     tensor_key(key, *C, idx_C);
@@ -264,6 +269,7 @@ void tensor_mult(const tblis_config* cfg, const tblis_tensor* A, const label_typ
                 check_data(B, "B");
             }
             TuneOperandsScope ops(reads ? A->data : nullptr, reads ? B->data : nullptr);
+            AlignedScope pieces(aligned);
             PlanBuilder pb(elem_size(type), dtype_code(type), family_of(algo));
             pb.add(g);
             plan = pb.build();
@@ -447,6 +453,8 @@ void tensor_mult_batch(const tblis_config* cfg, int64_t count, const tblis_tenso
 
     std::string key;
     put(key, (int32_t)algo);
+    const bool aligned = aligned16(A[0]->data, B[0]->data);
+    put(key, aligned);
     put(key, count);
     put(key, sa);
     put(key, sb);
@@ -491,6 +499,7 @@ void tensor_mult_batch(const tblis_config* cfg, int64_t count, const tblis_tenso
             }
         TuneOperandsScope ops(reads ? A[0]->data : nullptr, reads ? B[0]->data : nullptr);
         DirectAllScope direct;
+        AlignedScope pieces(aligned);
         plan = pb.build();
         if (!plan) plan = empty_plan();
         cache_put(key, plan);

@@ -55,6 +55,7 @@ struct PanelLaunch
     bool direct_a, direct_b;  // FP64: operand read from the tensor (PanelTask)
     int group;                // gather tiles: lanes along k, 1 A + 2 B
     bool scaled;              // gather tiles: per-k scales (PanelTask::a_kt)
+    bool pieces;              // gather tiles: FP64 operands in aligned pairs (gemm_lds.hip)
     int slices;               // most k slices of one GEMM (C panels to add up)
     hipStream_t stream;
 };

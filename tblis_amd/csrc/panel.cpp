@@ -27,6 +27,9 @@ namespace tblis_amd
 namespace
 {
 
+thread_local bool t_direct_all = false;  // DirectAllScope
+thread_local bool t_aligned = false;     // AlignedScope
+
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Re-read limit (tiles) of rows-fast direct operands (TBLIS_HIP_DIRECT_ROWS,
@@ -287,40 +290,137 @@ int64_t total_k(const PanelGemm& g)
 
 // Adding the k slices of a plan up: one launch, and the C panels written
 // and read once.
-double reduce_us(double panel_bytes) { return 4.0 + 2.0 * panel_bytes / 4.2e6; }
+double reduce_us(double panel_bytes) { return 4.5 + 2.0 * panel_bytes / 4.2e6; }
+
+// Share of neighbouring offsets that are one element apart.
+double unit_share(const std::vector<int64_t>& off)
+{
+    int64_t c = 0;
+    const int64_t n = (int64_t)off.size();
+    for (int64_t i = 0; i + 1 < n; i++) c += off[i + 1] - off[i] == 1;
+    return n > 1 ? (double)c / (double)(n - 1) : 0.0;
+}
+
+// Offsets of a side in odometer order.
+std::vector<int64_t> side_offsets(const Side& s)
+{
+    if (!s.offs.empty()) return s.offs;
+    Pool p;
+    const int64_t at = p.offsets(s);
+    return std::vector<int64_t>(p.data().begin() + at, p.data().begin() + at + side_len(s));
+}
+
+// Can an FP64 operand be read in 16-byte pieces (gemm_pieces_kernel)?  rows
+// and ks in bytes from its lowest element, itself at an even element.  Lanes
+// along rows: rows in aligned pairs.  Lanes along k: every stage of bk k is
+// one aligned run.  Both: the offsets within a stage, from its first k, are
+// the same in every stage, and stages start on 16 bytes.
+bool vec_layout(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks, int64_t src, bool lanes_k, int64_t bk)
+{
+    if (src % 2 || (lanes_k ? ks : rows).size() % 2) return false;
+    if (!lanes_k)
+        for (size_t i = 0; i < rows.size(); i += 2)
+            if (rows[i] % 16 || rows[i + 1] != rows[i] + 8) return false;
+    if (lanes_k)
+        for (int64_t r : rows)
+            if (r % 16) return false;
+    for (size_t i = 0; i < ks.size(); i++)
+    {
+        const int64_t at = ks[i] - ks[i - i % bk];
+        if (at != (lanes_k ? 8 * (int64_t)(i % bk) : ks[i % bk] - ks[0])) return false;
+        if ((!lanes_k || i % bk == 0) && ks[i] % 16) return false;
+    }
+    return true;
+}
+
+// One operand of a GEMM on a gather tile: byte offsets of its rows and k
+// (block bases included) from its lowest element src, and whether the lanes
+// of a load run along k (more neighbouring k than rows are one element apart).
+struct GatherOperand
+{
+    std::vector<int64_t> rows, ks;
+    int64_t src = 0;
+    bool lanes_k = false;
+};
+
+GatherOperand gather_operand(const std::vector<PBlock>& bl, int src_elem)
+{
+    GatherOperand o;
+    o.rows = side_offsets(bl[0].rows);
+    for (const PBlock& b : bl)
+        for (int64_t x : side_offsets(b.k)) o.ks.push_back(b.base - bl[0].base + x);
+    o.lanes_k = unit_share(o.ks) > unit_share(o.rows);
+    o.src = bl[0].base;
+    for (std::vector<int64_t>* v : {&o.rows, &o.ks})
+    {
+        const int64_t lo = *std::min_element(v->begin(), v->end());
+        o.src += lo;
+        for (int64_t& x : *v) x = (x - lo) * src_elem;
+    }
+    return o;
+}
+
+// Do the gather kernels with stages of bk k read every operand of these
+// GEMMs in 16-byte pieces?
+bool pieces_apply(const std::vector<PanelGemm>& gemms, int src_elem, int64_t bk)
+{
+    if (!t_aligned || src_elem != 8) return false;
+    for (const PanelGemm& g : gemms)
+    {
+        for (double x : g.kscale)
+            if (x != 1.0) return false;
+        if (total_k(g) == 0) continue;
+        for (const std::vector<PBlock>* bl : {&g.a, &g.b})
+        {
+            const GatherOperand o = gather_operand(*bl, src_elem);
+            if (!vec_layout(o.rows, o.ks, o.src, o.lanes_k, bk)) return false;
+        }
+    }
+    return true;
+}
 
 struct GatherChoice
 {
     int tile = -1;
     int slices = 1;
     double us = 0;
+    bool pieces = false;
 };
 
 // Best gather tile (gemm_lds.hip; only: that one) and number of k slices
-// for these GEMMs, from a model of a CU that holds up to occ workgroups: a stage takes the
-// MFMA and issue cycles of every resident workgroup's stage, at least the
-// memory latency of the one stage of loads in flight, and a task 1.5 stages
-// more than its k (filling, epilogue).  Cycles per stage and latency fitted
-// to (us, model / measured): 24^4 on tile 10 whole 36 / 34.1, in 3 slices
-// 19 / 20.2, on tile 11 21 / 21.9; the permuted 64/32 contraction 566 / 564,
-// the 8-irrep DPD GEMMs 58 / 59.
+// for these GEMMs, from a model of a CU that holds up to occ workgroups.  A
+// workgroup's stage takes `stage` cycles of the CU's MFMA units, a round of
+// resident workgroups at least `latency` per stage, and a task `fill` cycles
+// for its chain of table loads, first stage and epilogue.  us, model /
+// measured, in pieces: 10^4 6 / 6.1, 16^4 7.5 / 7.4, 22^4 11 / 10.4, 24^4 17
+// / 15.7, 30^4 39 / 37.6, 36^4 82 / 84.8, 42^4 202 / 202 on the 32 x 32 tile,
+// permuted 64/32 508 / 508 on the 64 x 64 one; element-wise: 17^4 10.3 /
+// 10.2, 25^4 23 / 23.5, 31^4 59 / 60.
 GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int src_elem, int cus, int only = -1)
 {
     struct Model
     {
-        int lt, occ;
-        double stage;  // cycles of one workgroup's stage on a CU
+        int lt;
+        bool pieces;
+        int occ;
+        double stage, latency, fill;
     };
-    constexpr Model models[] = {{1, 4, 1170}, {2, 3, 800}};
-    constexpr double kLatency = 2000, kGHz = 2.15;
+    constexpr Model models[] = {{1, true, 4, 1050, 1500, 5000}, {2, true, 4, 567, 1000, 5000},
+                                {0, false, 2, 2500, 2600, 6000}, {1, false, 4, 1170, 2000, 6000},
+                                {2, false, 3, 960, 1300, 6000}};
+    constexpr double kGHz = 2.15;
     GatherChoice best;
     const int first = panel_num_tiles(family) - lds_num_tiles();
+    int known = -1;
+    bool pieces = false;
     for (const Model& md : models)
     {
         const int tile = first + md.lt;
-        if (only >= 0 && tile != only) continue;
+        if (only >= 0 ? tile != only : md.lt == 0) continue;
         const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
         const int64_t bk = panel_tile_k(family, tile);
+        if (known != (int)bk) pieces = pieces_apply(gemms, src_elem, bk), known = (int)bk;
+        if (md.pieces != pieces && !(md.lt == 0)) continue;
         int64_t kmax = 1;
         double bytes = 0;
         for (const PanelGemm& g : gemms)
@@ -329,7 +429,8 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
             kmax = std::max(kmax, k);
             bytes += (double)src_elem * ((double)g.mlen[0] * k + (double)g.nlen[0] * k + (double)g.mlen[0] * g.nlen[0]);
         }
-        for (int64_t S = 1; S <= std::min<int64_t>(ceil_div(kmax, 2 * bk), 1024); S += S < 4 ? 1 : S / 4)
+        for (int64_t S = 1; S <= std::min<int64_t>(std::max<int64_t>(1, ceil_div(kmax, 2 * bk)), 1024);
+             S += S < 4 ? 1 : S / 4)
         {
             const int64_t kslice = ceil_div(ceil_div(kmax, S), bk) * bk;
             int64_t ntask = 0;
@@ -339,54 +440,62 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
                 const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g), s = std::max<int64_t>(1, ceil_div(k, kslice));
                 const int64_t nt = ceil_div(m, BM) * ceil_div(n, BN) * s;
                 ntask += nt;
-                work += (double)nt * (std::min((double)kslice, (double)k) / (double)bk + 1.5) * md.stage;
+                work += (double)nt * std::ceil(std::min((double)kslice, (double)k) / (double)bk) * md.stage;
                 if (s > 1) panels += 8.0 * (double)s * (double)m * (double)n;
             }
             if (S > 1 && (panels > (double)(64 << 20) || ntask > 8 * cus)) break;
-            const double st = (double)kslice / (double)bk + 1.5;
-            const int64_t res = std::min<int64_t>(md.occ, ceil_div(ntask, cus));
-            double cyc = st * std::max(res * md.stage, kLatency);
-            if (ntask > md.occ * cus) cyc = std::max(cyc, 1.05 * work / cus);
-            double us = std::max(cyc / (kGHz * 1e3), bytes / 4.2e6) + 3.0;
+            const double st = (double)(std::min(kslice, ceil_div(kmax, bk) * bk) / bk);
+            const int64_t per = ceil_div(ntask, cus);
+            double cyc;
+            if (per <= md.occ)
+                cyc = md.fill + st * std::max((double)per * md.stage, md.latency);
+            else if (gemms.size() == 1)
+                cyc = (double)ceil_div(per, md.occ) * md.fill + (double)per * st * md.stage;
+            else
+                cyc = (double)ceil_div(per, md.occ) * md.fill + std::max(1.05 * work / cus, st * md.stage * md.occ);
+            double us = std::max(cyc / (kGHz * 1e3), bytes / 5.5e6) + 1.5;
             if (panels > 0) us += reduce_us(panels);
-            if (best.tile < 0 || us < best.us) best = GatherChoice{tile, (int)S, us};
+            if (best.tile < 0 || us < best.us) best = GatherChoice{tile, (int)S, us, pieces};
         }
     }
     return best;
 }
 
-// Plans that take a gather tile without a measurement: GEMMs whose operands
-// have unit-stride rows or k (others are packed once instead of gathered by
-// every tile) and that the register-fed tiles serve badly (us, register tile
-// / gather tile, same box).
+// Plans that take a gather tile without a measurement (us, best register-fed
+// tile / gather tile, same box unless noted).
+//   Operands in 16-byte pieces: always.  10^4 6.7 / 6.1, 16^4 9.6 / 7.4, 24^4
+//   27.3 / 15.7, 36^4 95 / 85, permuted 64/32 575 / 508 (no pack, no panels).
+// Element by element, where the register-fed tiles do badly and operands
+// have unit-stride rows or k (others are packed once rather than gathered
+// by every tile):
+//   Batches, whose small instances leave each register tile a short loop of
+//   scattered reads: 4096-instance mix (1024 of them) 5478 / 4862, 1000 of
+//   extents 12-24 1946 / 1627, 200 of 10-40 2482 / 1922.
 //   Long k and few C tiles (under two 32 x 32 tiles per CU): without k
-//   slices the chip is idle.  32 x 32 x 131072 3125 / 22.6, 50 x 50 x 22785
-//   558 / 15.3, 16 x 16 x 2560 41 / 8.2.
-//   One to two 32 x 32 tiles per CU: the register tile runs a second,
-//   nearly empty round.  24^4 (324 tiles) 27.3 / 22.0; up to one round it
-//   is the better one at this k (22^4, 256 tiles: 13.4 / 17.4; 10^4 6.7 / 6.8).
+//   slices the chip is idle.  32 x 32 x 131072 3125 / 21, 91 x 91 x 357
+//   (odd extents) 42 / 8.1.
+//   One to two 32 x 32 tiles per CU: the register tile runs a second, nearly
+//   empty round.  23^4 20.8 / 20.4, 33/17 permuted 37 / 29; up to one round
+//   it is the better one at this k (21^4 12.1 / 12.6) as long as it reads
+//   both operands in place.
 //   Short k (up to 64): packing an operand moves as many bytes as the
-//   contraction itself.  64 x 65536 x 32 34.2 / 20.4, 70 x 112000 x 40 75 /
-//   55; not where the 64 x 64 tile is mostly padding (33 x 14553 x 21 13.3 /
-//   13.9).
-bool gather_preferred(const std::vector<PanelGemm>& gemms, int cus)
+//   contraction itself.  33 x 14553 x 21 13.1 / 7.8, 70 x 112000 x 40 75 / 59.
+bool gather_preferred(const std::vector<PanelGemm>& gemms, int cus, bool pieces)
 {
+    if (pieces) return true;
     int64_t tiles = 0, kmax = 0;
-    double area = 0, padded = 0;
     for (const PanelGemm& g : gemms)
     {
-        const int64_t m = g.mlen[0], n = g.nlen[0];
-        tiles += ceil_div(m, 32) * ceil_div(n, 32);
-        area += (double)m * (double)n;
-        padded += 4096.0 * (double)(ceil_div(m, 64) * ceil_div(n, 64));
+        tiles += ceil_div(g.mlen[0], 32) * ceil_div(g.nlen[0], 32);
         kmax = std::max(kmax, total_k(g));
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
             for (const PBlock& b : *bl)
                 if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1)
                     return false;
     }
-    if (tiles < 2 * cus) return tiles > cus || kmax >= 1024;
-    return kmax <= 64 && padded <= 1.6 * area;
+    if (t_direct_all) return true;
+    if (tiles < 2 * cus) return tiles > cus || kmax >= 1024 || kmax <= 64;
+    return kmax <= 64;
 }
 
 }  // namespace
@@ -595,12 +704,14 @@ struct TuneOperands
 };
 thread_local TuneOperands t_tune_ops;
 thread_local bool t_tune_off = false;    // AutotuneOffScope
-thread_local bool t_direct_all = false;  // DirectAllScope
 
 }  // namespace
 
 DirectAllScope::DirectAllScope() : was_(t_direct_all) { t_direct_all = true; }
 DirectAllScope::~DirectAllScope() { t_direct_all = was_; }
+
+AlignedScope::AlignedScope(bool aligned) : was_(t_aligned) { t_aligned = aligned; }
+AlignedScope::~AlignedScope() { t_aligned = was_; }
 
 AutotuneOffScope::AutotuneOffScope() : was_(t_tune_off) { t_tune_off = true; }
 AutotuneOffScope::~AutotuneOffScope() { t_tune_off = was_; }
@@ -659,10 +770,10 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         char* sbase = nullptr;
         size_t sbytes = 0;
         static_storage(sbase, sbytes);
-        if (family == FAMILY_F64 && !sbase && lds_applicable(gemms, dtype == 0 ? 8 : 4) && gather_preferred(gemms, cus))
+        if (family == FAMILY_F64 && !sbase && lds_applicable(gemms, dtype == 0 ? 8 : 4))
         {
             const GatherChoice c = gather_choice(gemms, family, dtype == 0 ? 8 : 4, cus);
-            tile = c.tile;
+            if (gather_preferred(gemms, cus, c.pieces)) tile = c.tile;
         }
     }
     bool packed = false;
@@ -838,24 +949,6 @@ struct TileWalk
     int64_t region(int64_t tm, int64_t tn) const { return (tm * RM / MT) * RN + tn * RN / NT; }
 };
 
-// Share of neighbouring offsets that are one element apart.
-double unit_share(const std::vector<int64_t>& off)
-{
-    int64_t c = 0;
-    const int64_t n = (int64_t)off.size();
-    for (int64_t i = 0; i + 1 < n; i++) c += off[i + 1] - off[i] == 1;
-    return n > 1 ? (double)c / (double)(n - 1) : 0.0;
-}
-
-// Offsets of a side in odometer order.
-std::vector<int64_t> side_offsets(const Side& s)
-{
-    if (!s.offs.empty()) return s.offs;
-    Pool p;
-    const int64_t at = p.offsets(s);
-    return std::vector<int64_t>(p.data().begin() + at, p.data().begin() + at + side_len(s));
-}
-
 // k slices per GEMM forced by TBLIS_HIP_KSPLIT (read at every plan build), or 0.
 int ksplit_forced()
 {
@@ -875,6 +968,7 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
     std::vector<int> group;
     std::vector<PanelTask> all;
     int64_t nregions = 0, wsc = 0;
+    T.pieces = src_elem == 8 && t_aligned;
     for (const PanelGemm& g : gemms)
         for (double x : g.kscale) T.scaled |= x != 1.0;
     for (const PanelGemm& g : gemms)
@@ -895,22 +989,15 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
             const std::vector<PBlock>* blocks[2] = {&g.a, &g.b};
             for (int o = 0; o < 2; o++)
             {
-                // byte offsets from the operand's lowest element
-                const std::vector<PBlock>& bl = *blocks[o];
-                Side rows, ks;
-                rows.offs = side_offsets(bl[0].rows);
-                for (size_t q = 0; q < bl.size(); q++)
-                    for (int64_t x : side_offsets(bl[q].k)) ks.offs.push_back(bl[q].base - bl[0].base + x);
-                if (unit_share(ks.offs) > unit_share(rows.offs)) kl |= 1 << o;
-                src[o] = bl[0].base;
-                for (Side* s : {&rows, &ks})
-                {
-                    const int64_t lo = *std::min_element(s->offs.begin(), s->offs.end());
-                    src[o] += lo;
-                    for (int64_t& x : s->offs) x = (x - lo) * src_elem;
-                }
+                GatherOperand x = gather_operand(*blocks[o], src_elem);
+                T.pieces = T.pieces && vec_layout(x.rows, x.ks, x.src, x.lanes_k, panel_tile_k(family, tile));
+                if (x.lanes_k) kl |= 1 << o;
                 // the kernels read offsets up to four stages past a task's end
-                ks.offs.insert(ks.offs.end(), (size_t)(4 * panel_tile_k(family, tile)), ks.offs.back());
+                x.ks.insert(x.ks.end(), (size_t)(4 * panel_tile_k(family, tile)), x.ks.back());
+                Side rows, ks;
+                rows.offs.swap(x.rows);
+                ks.offs.swap(x.ks);
+                src[o] = x.src;
                 rt[o] = pool.offsets(rows);
                 km[o] = pool.offsets(ks);
             }
@@ -1752,6 +1839,7 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
                 G.direct_b = (g & 2) != 0;
                 G.group = g;
                 G.scaled = tabs[i].scaled;
+                G.pieces = tabs[i].pieces;
                 if (launch_panel_gemm(G) != hipSuccess) return false;
                 at += sc.group_n[st][g];
             }
@@ -1914,6 +2002,7 @@ bool build_panel_plan(Plan& plan, std::vector<PanelGemm> gemms, int elem_size, i
     plan.direct[1] = T.direct[1];
     for (int g = 0; g < 4; g++) plan.group_n[g] = T.group_n[g];
     plan.scaled = T.scaled;
+    plan.pieces = T.pieces;
     plan.slices = T.slices;
     plan.sched = T.sched;
     plan.key.family = family;

@@ -82,6 +82,7 @@ struct PanelTables
     // the tensors (none, A, B, both); one GEMM launch per non-empty group
     int64_t group_n[4] = {0, 0, 0, 0};
     bool scaled = false;  // gather tiles: some k block is scaled
+    bool pieces = false;  // gather tiles: operands in 16-byte pieces (vec_layout)
     int slices = 1;       // gather tiles: most k slices of one GEMM
     // chunks and tasks ordered by stage: sched.chunks[s] pack chunks and
     // sched.group_n[s][g] tasks of group g in stage s (group-major within
@@ -140,6 +141,18 @@ struct DirectAllScope
 {
     DirectAllScope();
     ~DirectAllScope();
+
+  private:
+    bool was_;
+};
+
+// Plans built on this thread while one lives are for tensors A and B that
+// start on 16 bytes (aligned), or may not (the callers put that in the
+// plan's key).
+struct AlignedScope
+{
+    explicit AlignedScope(bool aligned);
+    ~AlignedScope();
 
   private:
     bool was_;

@@ -388,6 +388,7 @@ void run_plan(const std::shared_ptr<Plan>& pp, const void* A, const void* B, voi
     P.direct_a = p.direct[0];
     P.direct_b = p.direct[1];
     P.scaled = p.scaled;
+    P.pieces = p.pieces;
     P.slices = p.slices;
     P.alpha = alpha;
     P.beta = beta;

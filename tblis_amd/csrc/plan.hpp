@@ -54,6 +54,7 @@ struct Plan
     bool direct[2] = {false, false};  // FP64 operands read from the tensors (every task)
     int64_t group_n[4] = {0, 0, 0, 0};  // panel tasks reading none / A / B / both from the tensors
     bool scaled = false;                // gather tiles: per-k scales
+    bool pieces = false;                // gather tiles: operands in 16-byte pieces
     int slices = 1;                     // gather tiles: most k slices of one GEMM
     PanelSchedule sched;                // stages of chunks and task groups
     int p_nchunks = 0, p_nuchunks = 0;

@@ -43,6 +43,44 @@ def test_gather_tiles_in_slices(tile, slices, plans):
                 dtype=np.float32, config="fp64_mfma", tol=2e-7)
 
 
+@pytest.mark.parametrize("at", [0, 1])
+@pytest.mark.parametrize("slices", ["1", "3"])
+@pytest.mark.parametrize("tile", ["9", "10", "11"])
+def test_gather_in_pieces(tile, slices, at, plans):
+    """Operands whose rows or k come in pairs are read 16 bytes at a time when
+    the tensors start on 16 bytes (at 0), element by element when they do not
+    (at 1): lanes along rows and along k on either side, last stages of 2 to
+    BK - 2 k and of an odd number of them, an odd number of rows, k of two
+    dimensions, beta = 0 over NaN."""
+    plans.setenv("TBLIS_HIP_PANEL_TILE", tile)
+    plans.setenv("TBLIS_HIP_KSPLIT", slices)
+    g = torch.Generator(device=DEV).manual_seed(75000 + int(tile) * 10 + int(slices) + at)
+
+    def tensor(shape, row_major):
+        flat = torch.rand(at + shape[0] * shape[1], dtype=torch.float64, device=DEV, generator=g) - 0.5
+        v = flat[at:]
+        return v.view(shape) if row_major else v.view(shape[1], shape[0]).t()
+
+    for m, n, k in [(2, 2, 2), (32, 64, 16), (34, 66, 18), (130, 2, 130), (66, 34, 31), (33, 64, 98), (64, 130, 162)]:
+        for ra in (False, True):
+            for rb in (False, True):
+                A, B = tensor((m, k), ra), tensor((k, n), rb)
+                C = torch.full((m, n), float("nan"), dtype=torch.float64, device=DEV)
+                T.mult(1.5, A, "ak", B, "kb", 0.0, C, "ab")
+                torch.cuda.synchronize()
+                assert T.last_tile() == int(tile)
+                want = 1.5 * (A.cpu().numpy() @ B.cpu().numpy())
+                assert rel_fro(C.cpu().numpy(), want) <= FP64_TOL, (m, n, k, ra, rb)
+    # k = (e, f) in stages of one dimension: 32 and 64 fill the stages
+    x = torch.rand(at + 6 * 32 * 10 * 4, dtype=torch.float64, device=DEV, generator=g)[at:].view(4, 10, 32, 6) - 0.5
+    y = torch.rand(at + 32 * 8 * 4 * 5, dtype=torch.float64, device=DEV, generator=g)[at:].view(5, 4, 8, 32) - 0.5
+    C = torch.zeros(5, 8, 10, 6, dtype=torch.float64, device=DEV)
+    T.mult(1.0, x, "fbea", y, "jfie", 0.0, C, "jiba")
+    torch.cuda.synchronize()
+    want = np.einsum("fbea,jfie->jiba", x.cpu().numpy(), y.cpu().numpy())
+    assert rel_fro(C.cpu().numpy(), want) <= FP64_TOL
+
+
 @pytest.mark.parametrize("slices", ["1", "3"])
 @pytest.mark.parametrize("tile", ["9", "10", "11"])
 def test_gather_scaled_blocks(tile, slices, plans):
