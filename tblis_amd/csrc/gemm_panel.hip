@@ -534,17 +534,18 @@ __global__ __launch_bounds__(256) void unpack_panel_kernel(const UnpackJob* __re
     }
 }
 
-// C panels of k slices: adds a job's nslice panels up and applies
+// C panels of k slices (double; float from the split-BF16 gather tiles): adds
+// a job's nslice panels up in double and applies
 // alpha / beta through C's offsets.  A workgroup takes E consecutive elements
 // (row by row) of one job; its threads form SP sets that each add every
 // SP-th slice, and the sets' sums meet in LDS in slice-set order, so that the
 // result does not depend on which workgroup ran when.  Bound by the reads of
 // the panels, or, for a small C with many slices, by their latency: 16 sets
 // keep 16 x 4 loads in flight per element.
-template <typename TC, int SP>
+template <typename TC, typename TP, int SP>
 __global__ __launch_bounds__(SP == 16 ? 1024 : 256) void reduce_slices_kernel(
     const UnpackJob* __restrict__ jobs, const UnpackChunk* __restrict__ chunks, const int64_t* __restrict__ pool,
-    const double* __restrict__ ws, TC* __restrict__ C, double alpha, double beta)
+    const TP* __restrict__ ws, TC* __restrict__ C, double alpha, double beta)
 {
     constexpr int NT = SP == 16 ? 1024 : 256, E = NT / SP;
     const UnpackChunk ch = chunks[blockIdx.x];
@@ -554,7 +555,7 @@ __global__ __launch_bounds__(SP == 16 ? 1024 : 256) void reduce_slices_kernel(
     double sum = 0.0;
     if (e < n)
     {
-        const double* p = ws + j.panel + e;
+        const TP* p = ws + j.panel + e;
         int s = set;
         for (; s + 3 * SP < j.nslice; s += 4 * SP)
         {
@@ -580,19 +581,19 @@ __global__ __launch_bounds__(SP == 16 ? 1024 : 256) void reduce_slices_kernel(
     *c = (TC)v;
 }
 
-template <typename TC>
+template <typename TC, typename TP>
 void launch_reduce(const PanelLaunch& L)
 {
     auto go = [&](auto* k, int threads) {
         hipLaunchKernelGGL(k, dim3(L.nuchunks), dim3(threads), 0, L.stream, L.ujobs, L.uchunks, L.pool,
-                           (const double*)L.cws, (TC*)L.C, L.alpha, L.beta);
+                           (const TP*)L.cws, (TC*)L.C, L.alpha, L.beta);
     };
     if (L.slices >= 32)
-        go(&reduce_slices_kernel<TC, 16>, 1024);
+        go(&reduce_slices_kernel<TC, TP, 16>, 1024);
     else if (L.slices >= 8)
-        go(&reduce_slices_kernel<TC, 4>, 256);
+        go(&reduce_slices_kernel<TC, TP, 4>, 256);
     else
-        go(&reduce_slices_kernel<TC, 1>, 256);
+        go(&reduce_slices_kernel<TC, TP, 1>, 256);
 }
 
 // ------------------------------------------------------------------ fill
@@ -739,23 +740,39 @@ int persistent_grid(const void* kernel, int block, int ntasks)
 // The Ozaki family has one tile: 64 x 64 per workgroup, 2 x 2 waves.  The
 // FP64 family's tiles are the register-fed ones, then the LDS-staged ones
 // (gemm_lds.hip, four waves each).
+namespace
+{
+// first gather tile of a family (its panel tiles come before)
+int first_gather(int family) { return family == FAMILY_F64 ? kNumTiles : panel_bf16_num_tiles(); }
+}  // namespace
+
 int panel_num_tiles(int family)
 {
     if (family == FAMILY_OZAKI) return 1;
-    return family == FAMILY_F64 ? kNumTiles + lds_num_tiles() : panel_bf16_num_tiles();
+    if (family == FAMILY_BF16X3_FAST) return panel_bf16_num_tiles();
+    return first_gather(family) + (family == FAMILY_F64 ? lds_num_tiles() : gather_bf16_num_tiles());
 }
-bool panel_tile_lds(int family, int t) { return family == FAMILY_F64 && t >= kNumTiles; }
-int panel_tile_k(int family, int t) { return panel_tile_lds(family, t) ? lds_tile_k(t - kNumTiles) : 0; }
+bool panel_tile_lds(int family, int t)
+{
+    return (family == FAMILY_F64 || family == FAMILY_BF16X3) && t >= first_gather(family);
+}
+int panel_tile_k(int family, int t)
+{
+    if (!panel_tile_lds(family, t)) return 0;
+    return family == FAMILY_F64 ? lds_tile_k(t - kNumTiles) : gather_bf16_tile_k(t - first_gather(family));
+}
 int panel_tile_m(int family, int t)
 {
     if (family == FAMILY_OZAKI) return 64;
-    if (panel_tile_lds(family, t)) return lds_tile_m(t - kNumTiles);
+    if (panel_tile_lds(family, t))
+        return family == FAMILY_F64 ? lds_tile_m(t - kNumTiles) : gather_bf16_tile_m(t - first_gather(family));
     return family == FAMILY_F64 ? kTiles[t].bm : panel_bf16_tile_m(t);
 }
 int panel_tile_n(int family, int t)
 {
     if (family == FAMILY_OZAKI) return 64;
-    if (panel_tile_lds(family, t)) return lds_tile_n(t - kNumTiles);
+    if (panel_tile_lds(family, t))
+        return family == FAMILY_F64 ? lds_tile_n(t - kNumTiles) : gather_bf16_tile_n(t - first_gather(family));
     return family == FAMILY_F64 ? kTiles[t].bn : panel_bf16_tile_n(t);
 }
 int panel_tile_waves(int family, int t)
@@ -781,6 +798,8 @@ hipError_t launch_panel_pack(const PanelLaunch& L)
 hipError_t launch_panel_gemm(const PanelLaunch& L)
 {
     if (L.ntasks == 0) return hipSuccess;
+    if (panel_tile_lds(L.family, L.tile) && L.family != FAMILY_F64)
+        return launch_gemm_gather_bf16(L, L.tile - first_gather(L.family));
     if (L.family != FAMILY_F64) return launch_panel_gemm_bf16(L);
     if (L.tile >= kNumTiles) return launch_gemm_lds(L, L.tile - kNumTiles);
     if (L.tile < 0) return hipErrorInvalidValue;
@@ -803,9 +822,11 @@ hipError_t launch_panel_unpack(const PanelLaunch& L)
     if (L.slices > 1)
     {
         if (L.dtype == 0)
-            launch_reduce<double>(L);
+            launch_reduce<double, double>(L);
+        else if (L.family == FAMILY_F64)
+            launch_reduce<float, double>(L);
         else
-            launch_reduce<float>(L);
+            launch_reduce<float, float>(L);
         return hipGetLastError();
     }
     if (L.dtype == 0)

@@ -53,7 +53,7 @@ struct PanelLaunch
     int family;  // FAMILY_F64 or a split-BF16 family
     int tile;
     bool direct_a, direct_b;  // FP64: operand read from the tensor (PanelTask)
-    int group;                // gather tiles: lanes along k, 1 A + 2 B
+    int group;                // gather tiles: how the operands' loads run (kTaskGroups)
     bool scaled;              // gather tiles: per-k scales (PanelTask::a_kt)
     bool pieces;              // gather tiles: FP64 operands in aligned pairs (gemm_lds.hip)
     int slices;               // most k slices of one GEMM (C panels to add up)
@@ -76,6 +76,13 @@ bool panel_bf16_tile_direct(int tile);  // has variants reading FP32 operands di
 // FP64 GEMM gathering both operands from the tensors through LDS
 // (gemm_lds.hip); its tiles follow the register-fed FP64 tiles.
 int lds_num_tiles();
+// split-BF16 GEMM gathering both FP32 operands (gemm_gather_bf16.hip); its
+// tiles follow the panel tiles of FAMILY_BF16X3
+int gather_bf16_num_tiles();
+int gather_bf16_tile_m(int t);
+int gather_bf16_tile_n(int t);
+int gather_bf16_tile_k(int t);
+hipError_t launch_gemm_gather_bf16(const PanelLaunch& L, int t);
 int lds_tile_k(int lt);  // k per stage
 int lds_tile_m(int lt);
 int lds_tile_n(int lt);

@@ -118,6 +118,16 @@ class Pool
         }
         return at;
     }
+    // explicit values at an even index, deduplicated
+    int64_t aligned(const std::vector<int64_t>& v)
+    {
+        std::vector<int64_t> key(v);
+        key.push_back(-2);
+        auto it = index_.find(key);
+        if (it != index_.end()) return it->second;
+        if (data_.size() % 2) data_.push_back(0);
+        return index_[key] = push(v);
+    }
     // append raw values; returns their pool index
     int64_t push(const std::vector<int64_t>& v)
     {
@@ -247,8 +257,8 @@ struct TileModel
 const TileModel kModelsF64[] = {{0, 0.85, 2}, {2, 0.70, 2}, {3, 0.82, 2}, {4, 0.80, 2},
                                 {1, 0.62, 6}, {5, 0.72, 6}, {6, 0.62, 4}, {7, 0.62, 4},
                                 {8, 0.50, 4}, {9, 0.88, 1}, {10, 0.55, 2}, {11, 0.80, 1}};
-const TileModel kModelsBf16[] = {{0, 0.55, 1}, {1, 0.55, 1}, {2, 0.45, 2},
-                                 {3, 0.35, 4}, {4, 0.30, 4}, {5, 0.25, 4}};
+const TileModel kModelsBf16[] = {{0, 0.55, 1}, {1, 0.55, 1}, {2, 0.45, 2}, {3, 0.35, 4},
+                                 {4, 0.30, 4}, {5, 0.25, 4}, {6, 0, 2},    {7, 0, 3}};
 const TileModel kModelsOzaki[] = {{0, 0.30, 1}};
 
 // Estimated run time of the GEMM tasks for a tile.
@@ -333,6 +343,18 @@ bool vec_layout(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks
     return true;
 }
 
+// Can split-BF16 load an FP32 operand's aligned runs of 8 k 16 bytes at a
+// time (lanes along k; rows and ks in bytes)?
+bool octet_layout(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks, int64_t src)
+{
+    if (src % 4 || ks.size() % 8) return false;
+    for (int64_t r : rows)
+        if (r % 16) return false;
+    for (size_t i = 0; i < ks.size(); i++)
+        if (i % 8 ? ks[i] != ks[i - 1] + 4 : ks[i] % 16 != 0) return false;
+    return true;
+}
+
 // One operand of a GEMM on a gather tile: byte offsets of its rows and k
 // (block bases included) from its lowest element src, and whether the lanes
 // of a load run along k (more neighbouring k than rows are one element apart).
@@ -379,6 +401,72 @@ bool pieces_apply(const std::vector<PanelGemm>& gemms, int src_elem, int64_t bk)
     return true;
 }
 
+// 128-byte lines that an operand's loads touch, over those its elements
+// would fill: 1 for long runs, about 2 for runs of 29 floats.
+double line_share(const GatherOperand& o, int src_elem)
+{
+    const std::vector<int64_t>& v = o.lanes_k ? o.ks : o.rows;
+    int64_t lines = 1;
+    for (size_t i = 1; i < v.size(); i++) lines += v[i] / 128 != v[i - 1] / 128;
+    return std::max(1.0, (double)lines * 128.0 / ((double)v.size() * src_elem));
+}
+
+// Index in a side's dimensions of its unit stride one, or -1.
+int unit_dim(const Side& s)
+{
+    for (size_t i = 0; s.offs.empty() && i < s.len.size() && i < s.stride.size(); i++)
+        if (s.stride[i] == 1 && s.len[i] > 1) return (int)i;
+    return -1;
+}
+
+void move_first(Side& s, int d)
+{
+    std::rotate(s.len.begin(), s.len.begin() + d, s.len.begin() + d + 1);
+    std::rotate(s.stride.begin(), s.stride.begin() + d, s.stride.begin() + d + 1);
+}
+
+// The order in which the gather kernels walk the dimensions of m, n and k.
+// The planner's order follows C, and may leave an operand read with a stride
+// along its rows and along k, a line per element, on each of its re-reads.
+// Moving its unit stride dimension first costs scattered writes of C, once;
+// it is done from k = 256, where the operand has more elements than that.
+// 1517 x 713 x 1247 floats in runs of 41 and 23, one operand read across its
+// runs: 53.4 -> 42.1 us; another order of six odd extents 79 -> 50 us.
+std::vector<PanelGemm> coalesced(std::vector<PanelGemm> gemms)
+{
+    const auto strided = [](const PBlock& b) {
+        return first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1;
+    };
+    for (PanelGemm& g : gemms)
+    {
+        if (g.c.size() != 1 || g.a.empty() || g.b.empty() || total_k(g) < 256) continue;
+        for (int op = 0; op < 2; op++)
+        {
+            std::vector<PBlock>&own = op ? g.b : g.a, &other = op ? g.a : g.b;
+            if (!strided(own[0])) continue;
+            Side& c = op ? g.c[0].cols : g.c[0].rows;
+            const int d = unit_dim(own[0].rows);
+            bool match = d >= 0 && c.offs.empty() && c.len == own[0].rows.len;
+            for (const PBlock& b : own) match = match && b.rows.offs.empty() && b.rows.len == c.len;
+            if (match)
+            {
+                move_first(c, d);
+                for (PBlock& b : own) move_first(b.rows, d);
+                continue;
+            }
+            for (size_t q = 0; q < own.size() && q < other.size(); q++)
+            {
+                const int dk = unit_dim(own[q].k);
+                if (dk < 0 || !other[q].k.offs.empty() || other[q].k.len != own[q].k.len) break;
+                if (first_step(other[q].k) == 1 && first_step(other[q].rows) != 1) break;
+                move_first(own[q].k, dk);
+                move_first(other[q].k, dk);
+            }
+        }
+    }
+    return gemms;
+}
+
 struct GatherChoice
 {
     int tile = -1;
@@ -387,40 +475,61 @@ struct GatherChoice
     bool pieces = false;
 };
 
-// Best gather tile (gemm_lds.hip; only: that one) and number of k slices
-// for these GEMMs, from a model of a CU that holds up to occ workgroups.  A
-// workgroup's stage takes `stage` cycles of the CU's MFMA units, a round of
-// resident workgroups at least `latency` per stage, and a task `fill` cycles
-// for its chain of table loads, first stage and epilogue.  us, model /
-// measured, in pieces: 10^4 6 / 6.1, 16^4 7.5 / 7.4, 22^4 11 / 10.4, 24^4 17
-// / 15.7, 30^4 39 / 37.6, 36^4 82 / 84.8, 42^4 202 / 202 on the 32 x 32 tile,
-// permuted 64/32 508 / 508 on the 64 x 64 one; element-wise: 17^4 10.3 /
-// 10.2, 25^4 23 / 23.5, 31^4 59 / 60.
+// Best gather tile (gemm_lds.hip, gemm_gather_bf16.hip; only: that one) and
+// number of k slices for these GEMMs, from a model of a CU that holds up to
+// occ workgroups.  A workgroup's stage takes `stage` cycles of the CU, a
+// round of resident workgroups at least `latency` per stage, and a task
+// `fill` cycles for its chain of table loads, first stage and epilogue.  us,
+// model / measured.  FP64 in pieces: 10^4 6 / 6.1, 16^4 7.5 / 7.4, 22^4 11 /
+// 10.4, 24^4 17 / 15.7, 30^4 39 / 37.6, 36^4 82 / 84.8, 42^4 202 / 202 on the
+// 32 x 32 tile, permuted 64/32 508 / 508 on the 64 x 64 one; element-wise:
+// 17^4 10.3 / 10.2, 25^4 23 / 23.5, 31^4 59 / 60.  Split-BF16: 24^4 17 / 17.7
+// and 36^4 44 / 44.3 on the 64 x 64 tile, permuted 64/32 233 / 237 whole and
+// 214 / 210 in two slices on the 128 x 128 one; its stages are bound by L2
+// where short runs make it fetch lines that it uses a part of (line_share:
+// runs of 29 and 31 floats took 1.7-2.1 times the cycles).
 GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int src_elem, int cus, int only = -1)
 {
     struct Model
     {
-        int lt;
+        int family, lt;
         bool pieces;
         int occ;
         double stage, latency, fill;
     };
-    constexpr Model models[] = {{1, true, 4, 1050, 1500, 5000}, {2, true, 4, 567, 1000, 5000},
-                                {0, false, 2, 2500, 2600, 6000}, {1, false, 4, 1170, 2000, 6000},
-                                {2, false, 3, 960, 1300, 6000}};
+    constexpr Model models[] = {{FAMILY_F64, 1, true, 4, 1050, 1500, 5000},
+                                {FAMILY_F64, 2, true, 4, 567, 1000, 5000},
+                                {FAMILY_F64, 0, false, 2, 2500, 2600, 6000},
+                                {FAMILY_F64, 1, false, 4, 1170, 2000, 6000},
+                                {FAMILY_F64, 2, false, 3, 960, 1300, 6000},
+                                {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000},
+                                {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000}};
+    const bool f64 = family == FAMILY_F64;
+    double lines = 1.0;  // the worse operand of the largest GEMM
+    if (!f64)
+    {
+        const PanelGemm* big = &gemms[0];
+        for (const PanelGemm& g : gemms)
+            if (g.mlen[0] * g.nlen[0] > big->mlen[0] * big->nlen[0] && total_k(g) > 0) big = &g;
+        if (total_k(*big) > 0)
+            for (const std::vector<PBlock>* bl : {&big->a, &big->b})
+                lines = std::max(lines, std::min(2.0, line_share(gather_operand(*bl, src_elem), src_elem)));
+        lines = 1.0 + 0.8 * (lines - 1.0);
+    }
     constexpr double kGHz = 2.15;
     GatherChoice best;
-    const int first = panel_num_tiles(family) - lds_num_tiles();
+    const int first = panel_num_tiles(family) - (f64 ? lds_num_tiles() : gather_bf16_num_tiles());
     int known = -1;
     bool pieces = false;
     for (const Model& md : models)
     {
+        if (md.family != family) continue;
         const int tile = first + md.lt;
-        if (only >= 0 ? tile != only : md.lt == 0) continue;
+        if (only >= 0 ? tile != only : f64 && md.lt == 0) continue;
         const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
         const int64_t bk = panel_tile_k(family, tile);
         if (known != (int)bk) pieces = pieces_apply(gemms, src_elem, bk), known = (int)bk;
-        if (md.pieces != pieces && !(md.lt == 0)) continue;
+        if (f64 && md.pieces != pieces && md.lt != 0) continue;
         int64_t kmax = 1;
         double bytes = 0;
         for (const PanelGemm& g : gemms)
@@ -440,19 +549,19 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
                 const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g), s = std::max<int64_t>(1, ceil_div(k, kslice));
                 const int64_t nt = ceil_div(m, BM) * ceil_div(n, BN) * s;
                 ntask += nt;
-                work += (double)nt * std::ceil(std::min((double)kslice, (double)k) / (double)bk) * md.stage;
-                if (s > 1) panels += 8.0 * (double)s * (double)m * (double)n;
+                work += (double)nt * std::ceil(std::min((double)kslice, (double)k) / (double)bk) * md.stage * lines;
+                if (s > 1) panels += (f64 ? 8.0 : 4.0) * (double)s * (double)m * (double)n;
             }
             if (S > 1 && (panels > (double)(64 << 20) || ntask > 8 * cus)) break;
             const double st = (double)(std::min(kslice, ceil_div(kmax, bk) * bk) / bk);
             const int64_t per = ceil_div(ntask, cus);
             double cyc;
             if (per <= md.occ)
-                cyc = md.fill + st * std::max((double)per * md.stage, md.latency);
+                cyc = md.fill + st * lines * std::max((double)per * md.stage, md.latency);
             else if (gemms.size() == 1)
-                cyc = (double)ceil_div(per, md.occ) * md.fill + (double)per * st * md.stage;
+                cyc = (double)ceil_div(per, md.occ) * md.fill + (double)per * st * md.stage * lines;
             else
-                cyc = (double)ceil_div(per, md.occ) * md.fill + std::max(1.05 * work / cus, st * md.stage * md.occ);
+                cyc = (double)ceil_div(per, md.occ) * md.fill + std::max(1.05 * work / cus, st * md.stage * lines * md.occ);
             double us = std::max(cyc / (kGHz * 1e3), bytes / 5.5e6) + 1.5;
             if (panels > 0) us += reduce_us(panels);
             if (best.tile < 0 || us < best.us) best = GatherChoice{tile, (int)S, us, pieces};
@@ -480,9 +589,31 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
 //   both operands in place.
 //   Short k (up to 64): packing an operand moves as many bytes as the
 //   contraction itself.  33 x 14553 x 21 13.1 / 7.8, 70 x 112000 x 40 75 / 59.
-bool gather_preferred(const std::vector<PanelGemm>& gemms, int cus, bool pieces)
+// Split-BF16: all but GEMMs that fill the chip with 256 x 128 panel tiles
+// and use each packed element in 16 of them and more.  8^4 12.5 / 6.8, 24^4
+// 22.4 / 15.7, 36^4 81 / 44, 8-irrep DPD 48.7 / 29.7, 1024-instance batch
+// 3494 / 2246, 48^4 281 / 171, permuted 67/35 608 / 383; at 56^4 (325 tiles)
+// 468 / 463, at 61^4 (450) 657 / 718, at 80^4 2562 / 2856.
+bool gather_preferred(const std::vector<PanelGemm>& gemms, int family, int cus, bool pieces)
 {
     if (pieces) return true;
+    if (family != FAMILY_F64)
+    {
+        double large = 0, all = 0;
+        for (const PanelGemm& g : gemms)
+        {
+            const double f = (double)g.mlen[0] * (double)g.nlen[0] * (double)total_k(g);
+            const int64_t m = g.mlen[0], n = g.nlen[0];
+            all += f;
+            if (std::min(m, n) >= 2048 && ceil_div(m, 256) * ceil_div(n, 128) >= 400) large += f;
+            for (const std::vector<PBlock>* bl : {&g.a, &g.b})
+                for (const PBlock& b : *bl)
+                    if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 &&
+                        side_count(b.k) > 1)
+                        return false;
+        }
+        return large <= 0.5 * all;
+    }
     int64_t tiles = 0, kmax = 0;
     for (const PanelGemm& g : gemms)
     {
@@ -752,8 +883,9 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     for (int mi = 0; mi < nmodels; mi++)
     {
         const TileModel& tm = models[mi];
-        if (family == FAMILY_BF16X3 && panel_bf16_tile_fast_only(tm.tile)) continue;
-        if (panel_tile_lds(family, tm.tile) && !lds_applicable(gemms, dtype == 0 ? 8 : 4)) continue;
+        if (tm.tile >= panel_num_tiles(family)) continue;
+        if (family == FAMILY_BF16X3 && !panel_tile_lds(family, tm.tile) && panel_bf16_tile_fast_only(tm.tile)) continue;
+        if (panel_tile_lds(family, tm.tile) && !lds_applicable(gemms, family, dtype == 0 ? 8 : 4)) continue;
         cands.push_back(tm.tile);
         if (panel_tile_lds(family, tm.tile)) continue;  // gather tiles have a model of their own
         double c = tile_cost(gemms, tm, cus, family);
@@ -770,10 +902,11 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         char* sbase = nullptr;
         size_t sbytes = 0;
         static_storage(sbase, sbytes);
-        if (family == FAMILY_F64 && !sbase && lds_applicable(gemms, dtype == 0 ? 8 : 4))
+        if ((family == FAMILY_F64 || family == FAMILY_BF16X3) && !sbase && lds_applicable(gemms, family, dtype == 0 ? 8 : 4))
         {
-            const GatherChoice c = gather_choice(gemms, family, dtype == 0 ? 8 : 4, cus);
-            if (gather_preferred(gemms, cus, c.pieces)) tile = c.tile;
+            const std::vector<PanelGemm> walk = coalesced(gemms);
+            const GatherChoice c = gather_choice(walk, family, dtype == 0 ? 8 : 4, cus);
+            if (gather_preferred(walk, family, cus, c.pieces)) tile = c.tile;
         }
     }
     bool packed = false;
@@ -787,8 +920,8 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     {
         int t = std::atoi(e);
         if (e[0] >= '0' && e[0] <= '9' && t < panel_num_tiles(family) &&
-            !(family == FAMILY_BF16X3 && panel_bf16_tile_fast_only(t)) &&
-            !(panel_tile_lds(family, t) && !lds_applicable(gemms, dtype == 0 ? 8 : 4)))
+            !(family == FAMILY_BF16X3 && !panel_tile_lds(family, t) && panel_bf16_tile_fast_only(t)) &&
+            !(panel_tile_lds(family, t) && !lds_applicable(gemms, family, dtype == 0 ? 8 : 4)))
         {
             tile = t;
             packed = false;
@@ -812,12 +945,13 @@ bool tables_uniform(const std::vector<PanelGemm>& gemms, int family, int tile, P
     T = PanelTables();
     if (panel_tile_lds(family, tile))
     {
+        const std::vector<PanelGemm> walk = coalesced(gemms);
         int64_t kmax = 1;
-        for (const PanelGemm& g : gemms) kmax = std::max(kmax, total_k(g));
+        for (const PanelGemm& g : walk) kmax = std::max(kmax, total_k(g));
         const int64_t bk = panel_tile_k(family, tile);
         int64_t S = ksplit_forced();
-        if (!S) S = gather_choice(gemms, family, src_elem, device_cu_count(), tile).slices;
-        return gather_tables(gemms, family, tile, T, src_elem, ceil_div(ceil_div(kmax, S), bk) * bk);
+        if (!S) S = gather_choice(walk, family, src_elem, device_cu_count(), tile).slices;
+        return gather_tables(walk, family, tile, T, src_elem, ceil_div(ceil_div(kmax, S), bk) * bk);
     }
     if (!tables_for_tile(gemms, family, tile, T, allow, src_elem)) return false;
     auto group = [](const PanelTask& t) {
@@ -866,11 +1000,14 @@ bool same_side(const Side& a, const Side& b) { return a.len == b.len && a.stride
 
 }  // namespace
 
-bool lds_applicable(const std::vector<PanelGemm>& gemms, int src_elem)
+bool lds_applicable(const std::vector<PanelGemm>& gemms, int family, int src_elem)
 {
     if (!direct_enabled()) return false;
     for (const PanelGemm& g : gemms)
     {
+        if (family != FAMILY_F64)
+            for (double x : g.kscale)
+                if (x != 1.0) return false;
         if (g.mlen.size() != 1 || g.nlen.size() != 1 || g.c.size() != 1) return false;
         if (g.a.size() != g.klen.size() || g.b.size() != g.klen.size()) return false;
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
@@ -991,15 +1128,27 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
             {
                 GatherOperand x = gather_operand(*blocks[o], src_elem);
                 T.pieces = T.pieces && vec_layout(x.rows, x.ks, x.src, x.lanes_k, panel_tile_k(family, tile));
-                if (x.lanes_k) kl |= 1 << o;
-                // the kernels read offsets up to four stages past a task's end
-                x.ks.insert(x.ks.end(), (size_t)(4 * panel_tile_k(family, tile)), x.ks.back());
+                const bool f64 = family == FAMILY_F64;
+                const int mode = !x.lanes_k ? 0 : !f64 && t_aligned && octet_layout(x.rows, x.ks, x.src) ? 2 : 1;
+                kl += mode * (o == 0 ? 1 : f64 ? 2 : 3);
+                // the kernels read offsets up to four stages past a task's
+                // end (whole octets of split-BF16's 16-byte loads)
+                const int64_t rep = std::min<int64_t>(k, 8);
+                for (int64_t i = 0; i < 4 * panel_tile_k(family, tile); i++)
+                    x.ks.push_back(x.ks[k - rep + (k + i) % rep]);
+                if (!f64)
+                {
+                    // 32-bit words, two to a pool entry, on 16 bytes
+                    std::vector<int64_t> w((x.ks.size() + 1) / 2, 0);
+                    for (size_t i = 0; i < x.ks.size(); i++) w[i / 2] |= (int64_t)((uint64_t)x.ks[i] << (32 * (i % 2)));
+                    x.ks.swap(w);
+                }
                 Side rows, ks;
                 rows.offs.swap(x.rows);
                 ks.offs.swap(x.ks);
                 src[o] = x.src;
+                km[o] = f64 ? pool.offsets(ks) : pool.aligned(ks.offs);
                 rt[o] = pool.offsets(rows);
-                km[o] = pool.offsets(ks);
             }
             if (T.scaled)
             {
@@ -1082,7 +1231,7 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
     if (all.size() > (size_t)INT32_MAX || T.uchunks.size() > (size_t)INT32_MAX)
         fail("contraction too large: panel task list exceeds 2^31 entries");
     // one launch per combination of lanes along rows and along k
-    for (int q = 0; q < 4; q++)
+    for (int q = 0; q < kTaskGroups; q++)
     {
         std::vector<PanelTask> ts;
         std::vector<int64_t> tc, tr;
@@ -1100,7 +1249,7 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
     }
     T.task_stage.assign(T.tasks.size(), 0);
     T.direct[0] = T.direct[1] = true;
-    T.ws_c = wsc;
+    T.ws_c = family == FAMILY_F64 ? wsc : (wsc + 1) / 2;  // split-BF16 slices store floats
     T.family = family;
     T.tile = tile;
     T.pool = std::move(pool.data());
@@ -1829,7 +1978,7 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
         int64_t at = 0;
         const PanelSchedule& sc = tabs[i].sched;
         for (int st = 0; st < sc.nstages; st++)
-            for (int g = 0; g < 4; g++)
+            for (int g = 0; g < kTaskGroups; g++)
             {
                 if (sc.group_n[st][g] == 0) continue;
                 PanelLaunch G = L;
@@ -2000,7 +2149,7 @@ bool build_panel_plan(Plan& plan, std::vector<PanelGemm> gemms, int elem_size, i
     plan.panel_tile = T.tile;
     plan.direct[0] = T.direct[0];
     plan.direct[1] = T.direct[1];
-    for (int g = 0; g < 4; g++) plan.group_n[g] = T.group_n[g];
+    for (int g = 0; g < kTaskGroups; g++) plan.group_n[g] = T.group_n[g];
     plan.scaled = T.scaled;
     plan.pieces = T.pieces;
     plan.slices = T.slices;

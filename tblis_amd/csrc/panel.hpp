@@ -78,9 +78,9 @@ struct PanelTables
     bool swap = false;  // GEMMs were transposed: operand 0 is the B tensor
     bool reads_ab = false;
     bool direct[2] = {false, false};  // operand read from the tensor by every task
-    // tasks come in four consecutive groups by which operands they read from
-    // the tensors (none, A, B, both); one GEMM launch per non-empty group
-    int64_t group_n[4] = {0, 0, 0, 0};
+    // tasks come in consecutive groups (kTaskGroups); one GEMM launch per
+    // non-empty group
+    int64_t group_n[kTaskGroups] = {};
     bool scaled = false;  // gather tiles: some k block is scaled
     bool pieces = false;  // gather tiles: operands in 16-byte pieces (vec_layout)
     int slices = 1;       // gather tiles: most k slices of one GEMM
@@ -97,8 +97,9 @@ struct PanelTables
 
 // Can the gather tiles (gemm_lds.hip) run these GEMMs: direct reads enabled,
 // one row block per operand, one C block, the same rows in every k block, and
-// each operand's offsets within 4 GiB?  src_elem: bytes per tensor element.
-bool lds_applicable(const std::vector<PanelGemm>& gemms, int src_elem);
+// each operand's offsets within 4 GiB?  Split-BF16 (gemm_gather_bf16.hip):
+// also no scaled k block.  src_elem: bytes per tensor element.
+bool lds_applicable(const std::vector<PanelGemm>& gemms, int family, int src_elem);
 
 // Orientation, tile, pack jobs, tasks and C unpack jobs (host only).
 // Returns false when there is nothing to launch.  dtype: 0 double, 1 float.

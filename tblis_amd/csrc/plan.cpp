@@ -341,7 +341,7 @@ void launch_panel_calls(const PanelLaunch& P, const PanelSchedule& S, bool overl
     for (int s = 0; s < S.nstages; s++)
     {
         if (staged) hip_check(hipStreamWaitEvent(P.stream, ts.stage_ev[s + 1], 0), "hipStreamWaitEvent");
-        for (int g = 0; g < 4; g++)
+        for (int g = 0; g < kTaskGroups; g++)
         {
             if (S.group_n[s][g] == 0) continue;
             PanelLaunch G = P;

@@ -52,7 +52,7 @@ struct Plan
     size_t ws_rmax_offset = 0;  // Ozaki: byte offset of the row-maximum array
     int64_t oz_rows = 0;        // Ozaki: its entries
     bool direct[2] = {false, false};  // FP64 operands read from the tensors (every task)
-    int64_t group_n[4] = {0, 0, 0, 0};  // panel tasks reading none / A / B / both from the tensors
+    int64_t group_n[kTaskGroups] = {};  // panel tasks by group
     bool scaled = false;                // gather tiles: per-k scales
     bool pieces = false;                // gather tiles: operands in 16-byte pieces
     int slices = 1;                     // gather tiles: most k slices of one GEMM

@@ -84,7 +84,7 @@ struct PackChunk
 // The gather tiles (gemm_lds.hip) read both operands from the tensors with
 // a_src / b_src the operand's lowest element, a_rt / b_rt the tile's first
 // row offset and a_km / b_km the per-k offsets (block bases included) in
-// bytes from it, a_kt the per-k scales (as doubles) in scaled plans; k runs
+// bytes from it (split-BF16: the per-k ones as 32-bit words), a_kt the per-k scales (as doubles) in scaled plans; k runs
 // over [kbeg, klen).
 struct PanelTask
 {
@@ -139,11 +139,15 @@ constexpr int FAMILY_OZAKI = 3;        // FP64-accurate: int8 digit planes (gemm
 // stage s has chunks[s] pack chunks and group_n[s][g] GEMM tasks reading
 // operands directly by group g (0 none, 1 A, 2 B, 3 both), in that order.
 constexpr int kMaxStages = 8;
+// Task groups, one launch each: which operands a task reads from the tensors
+// (0 none, 1 A, 2 B, 3 both), or on the gather tiles how its operands' loads
+// run (FP64: lanes along k, A + 2 B; split-BF16: modes, A + 3 B).
+constexpr int kTaskGroups = 9;
 struct PanelSchedule
 {
     int nstages = 1;
     int64_t chunks[kMaxStages] = {};
-    int64_t group_n[kMaxStages][4] = {};
+    int64_t group_n[kMaxStages][kTaskGroups] = {};
 };
 
 // Kernel variant selector.

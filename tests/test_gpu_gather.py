@@ -152,3 +152,89 @@ def test_sliced_call_in_a_graph(plans):
         T.mult(2.0, A, "km", B, "kn", 0.0, D, "mn")
         torch.cuda.synchronize()
         assert rel_fro(D.cpu().numpy(), 2.0 * want) <= FP64_TOL
+
+
+def _f32_case(m, n, k, ra, rb, at, g, alpha=1.25, beta=-0.5):
+    """C = alpha A B + beta C on tensors `at` floats past a 16-byte boundary.
+    Returns the error's norm over the result's; over |alpha| |A| |B| + |beta|
+    |C| where the result is a single entry, whose two terms may cancel."""
+
+    def tensor(shape, row_major):
+        v = (torch.rand(at + shape[0] * shape[1], device=DEV, generator=g) - 0.5)[at:]
+        return v.view(shape) if row_major else v.view(shape[1], shape[0]).t()
+
+    A, B, C = tensor((m, k), ra), tensor((k, n), rb), tensor((m, n), True)
+    a, b, c = (x.double().cpu() for x in (A, B, C))
+    want, size = alpha * (a @ b) + beta * c, abs(alpha) * (a.abs() @ b.abs()) + abs(beta) * c.abs()
+    if m * n > 1:
+        size = want
+    T.mult(alpha, A, "ak", B, "kb", beta, C, "ab")
+    torch.cuda.synchronize()
+    return ((C.double().cpu() - want).norm() / size.norm()).item()
+
+
+@pytest.mark.parametrize("at", [0, 1])
+@pytest.mark.parametrize("slices", ["1", "3"])
+@pytest.mark.parametrize("tile", ["6", "7"])
+def test_gather_split_bf16(tile, slices, at, plans):
+    """The split-BF16 gather tiles: lanes along rows or along k on either
+    side, rows in aligned eights or not, k below, at and past a stage, one row
+    or column, edges of tiles.  Bar: 1e-6, the bound of every split-BF16 path
+    (three BF16 terms hold a float; what the sums of at most 1100 products in
+    float lose stays under 16 units of 2^-24)."""
+    plans.setenv("TBLIS_HIP_PANEL_TILE", tile)
+    plans.setenv("TBLIS_HIP_KSPLIT", slices)
+    g = torch.Generator(device=DEV).manual_seed(76000 + int(tile) * 10 + int(slices) + at)
+    for m, n, k in [(1, 1, 1), (1, 65, 17), (64, 64, 32), (128, 136, 16), (129, 127, 47), (65, 63, 33), (200, 8, 80),
+                    (8, 264, 1100), (130, 62, 31)]:
+        for ra in (False, True):
+            for rb in (False, True):
+                assert _f32_case(m, n, k, ra, rb, at, g) <= 1e-6, (m, n, k, ra, rb)
+                assert T.last_tile() == int(tile)
+    # k of two dimensions, odd extents, an operand with no unit stride along
+    # its rows or k in the order of C; beta = 0 over NaN
+    for A, B, C in [("eafb", "jefi", "iabj"), ("aebf", "fjei", "aibj"), ("feba", "ijfe", "baji")]:
+        ext = dict(a=7, b=9, e=5, f=13, i=3, j=11)
+        x, y = (torch.rand([ext[d] for d in s], device=DEV, generator=g) - 0.5 for s in (A, B))
+        c = torch.full([ext[d] for d in C], float("nan"), device=DEV)
+        T.mult(1.0, x, A, y, B, 0.0, c, C)
+        torch.cuda.synchronize()
+        want = np.einsum(f"{A},{B}->{C}", x.double().cpu().numpy(), y.double().cpu().numpy())
+        assert rel_fro(c.double().cpu().numpy(), want) <= 1e-6, (A, B, C)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_orders_of_the_general_path(dtype, plans):
+    """Every order of the labels in both operands gives what packing gives,
+    whichever way the gather tiles walk them (the sums over e, f are long
+    enough for them to reorder rows and k)."""
+    import itertools
+    ext = dict(a=18, b=7, e=21, f=14, i=5, j=19)
+    g = torch.Generator(device=DEV).manual_seed(77000)
+    tol = 1e-12 if dtype == torch.float64 else 1e-6
+    for n, (A, B) in enumerate(itertools.product(list(itertools.permutations("abef"))[::3],
+                                                 list(itertools.permutations("efij"))[::5])):
+        C = ["abij", "jiba", "iabj", "bjai"][n % 4]
+        x, y = (torch.rand([ext[d] for d in s], dtype=dtype, device=DEV, generator=g) - 0.5 for s in (A, B))
+        out = []
+        for direct in ("1", "0"):
+            plans.setenv("TBLIS_HIP_DIRECT", direct)
+            T.lib().tblis_hip_clear_plan_cache()
+            c = torch.ones([ext[d] for d in C], dtype=dtype, device=DEV)
+            T.mult(1.0, x, "".join(A), y, "".join(B), 0.5, c, C)
+            torch.cuda.synchronize()
+            out.append(c.double().cpu().numpy())
+        assert rel_fro(out[0], out[1]) <= tol, (A, B, C)
+
+
+@pytest.mark.parametrize("m,n,k,gather", [(64, 64, 64, True), (1296, 1296, 1296, True), (32, 32, 8192, True),
+                                          (4096, 3712, 96, False)])
+def test_split_bf16_chosen_by_shape(m, n, k, gather, plans):
+    """Up to a few hundred 256 x 128 tiles the split-BF16 gather tiles run
+    without a knob; above, and with TBLIS_HIP_DIRECT=0, the panel tiles."""
+    g = torch.Generator(device=DEV).manual_seed(78000 + k)
+    for direct in ("1", "0"):
+        plans.setenv("TBLIS_HIP_DIRECT", direct)
+        T.lib().tblis_hip_clear_plan_cache()
+        assert _f32_case(m, n, k, False, False, 0, g) <= 1e-6
+        assert (T.last_tile() >= 6) == (gather and direct == "1")
