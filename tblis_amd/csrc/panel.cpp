@@ -248,9 +248,10 @@ struct TileModel
     int occ;     // waves per SIMD (register limited)
 };
 
-// Per-wave efficiency by wave tile.  FP64: 64x64 waves are 4x4 MFMA
-// blocks, 32x32 waves 2x2; set so that without the autotuner the model
-// picks what the tuner measured fastest on the permuted 64/32 GEMM (tile 5),
+// Per-wave efficiency by wave tile.  FP64 (plans in caller storage; others
+// count rounds, packed_us): 64x64 waves are 4x4 MFMA blocks, 32x32 waves
+// 2x2; set so that without the autotuner the model picks what the tuner
+// measured fastest on the permuted 64/32 GEMM (tile 5),
 // the 8-irrep DPD GEMMs (5), the 4096-instance batch (3; 128x64 over its
 // mirror 64x128, which tied in the model and ran 30 against 23 ms) and the
 // dense 24^4 GEMM (8).  Split-BF16: per tile of the BF16 table.
@@ -260,6 +261,13 @@ const TileModel kModelsF64[] = {{0, 0.85, 2}, {2, 0.70, 2}, {3, 0.82, 2}, {4, 0.
 const TileModel kModelsBf16[] = {{0, 0.55, 1}, {1, 0.55, 1}, {2, 0.45, 2}, {3, 0.35, 4},
                                  {4, 0.30, 4}, {5, 0.25, 4}, {6, 0, 2},    {7, 0, 3}};
 const TileModel kModelsOzaki[] = {{0, 0.30, 1}};
+
+int64_t total_k(const PanelGemm& g)
+{
+    int64_t k = 0;
+    for (auto x : g.klen) k += x;
+    return k;
+}
 
 // Estimated run time of the GEMM tasks for a tile.
 double tile_cost(const std::vector<PanelGemm>& gemms, const TileModel& tm, int cus, int family)
@@ -291,11 +299,59 @@ double tile_cost(const std::vector<PanelGemm>& gemms, const TileModel& tm, int c
     return std::max(total / (busy * per_simd), maxtask / (W * simd * tm.eff));
 }
 
-int64_t total_k(const PanelGemm& g)
+struct RegisterTile
 {
-    int64_t k = 0;
-    for (auto x : g.klen) k += x;
-    return k;
+    int tile;
+    double eff;    // share of the MFMA rate (16 multiply-adds a cycle), several waves to a SIMD
+    double alone;  // the same, one wave to a SIMD
+};
+
+// The FP64 register-fed tiles.  128 x 64 tiles (two waves) alone on a CU
+// share a SIMD.
+constexpr RegisterTile kRegisterTiles[] = {{0, 1.0, 0.77},  {1, 0.95, 0.60},  {2, 0.95, 0.94}, {3, 0.97, 0.50},
+                                           {4, 0.95, 0.82}, {5, 0.965, 0.90}, {7, 0.92, 0.75}, {8, 0.97, 0.85}};
+
+// us of FP64 GEMMs packed and multiplied on a register-fed tile: whole
+// rounds of waves over the SIMDs, whose last may be nearly empty (GEMMs of
+// several lengths fill one another's: half the longest wave).  Model /
+// measured: 1225^3 tile 5 93 / 92, 8 78 / 75; 1521^3 5 165 / 158, 8 132 /
+// 127; 1849^3 1 263 / 244, 2 264 / 250, 8 233 / 222; 4489 x 1225 x 4489
+// 0 1160 / 1186, 8 862 / 873; 8-irrep DPD 8 55 / 56.  Against a choice by
+// each tile's rate alone (us, rate / rounds): 2304^2 x 942 (48^4 with a
+// sparse index) 219 / 156, 1521^3 158 / 127, 4489 x 1225 x 4489 1176 / 872,
+// 41^4 complex 880 / 674.
+double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, int cus)
+{
+    const int64_t BM = panel_tile_m(FAMILY_F64, rt.tile), BN = panel_tile_n(FAMILY_F64, rt.tile);
+    const int64_t W = panel_tile_waves(FAMILY_F64, rt.tile), simds = 4LL * cus;
+    int64_t waves = 0, ngemm = 0;
+    double work = 0, longest = 0, shortest = 0, packed = 0, results = 0;
+    for (const PanelGemm& g : gemms)
+    {
+        const int64_t k = total_k(g);
+        int64_t m = 0, n = 0;
+        for (auto x : g.mlen) m += x;
+        for (auto x : g.nlen) n += x;
+        if (!m || !n) continue;
+        const int64_t nt = ceil_div(m, BM) * ceil_div(n, BN);
+        const double wave = (double)(BM * BN * std::max<int64_t>(ceil_div(k, 16) * 16, 16)) / (double)(16 * W);
+        waves += nt * W;
+        work += (double)(nt * W) * wave;
+        longest = std::max(longest, wave);
+        shortest = ngemm ? std::min(shortest, wave) : wave;
+        packed += 16.0 * (double)(m + n) * (double)k;
+        results += 8.0 * (double)m * (double)n;
+        ngemm++;
+    }
+    constexpr double kTask = 1500;  // a wave's first loads and its results
+    double cyc;
+    if (waves <= simds)
+        cyc = longest / rt.alone + kTask;
+    else if (shortest == longest)
+        cyc = (double)ceil_div(waves, simds) * (longest / rt.eff + kTask);
+    else
+        cyc = (work / (double)simds + 0.5 * longest) / rt.eff + (double)waves / (double)simds * kTask;
+    return std::max(cyc / 2150.0, results / 5.0e6) + packed / 5.0e6 + 6.3 + 0.08 * (double)(ngemm - 1);
 }
 
 // Adding the k slices of a plan up: one launch, and the C panels written
@@ -500,7 +556,7 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
     constexpr Model models[] = {{FAMILY_F64, 1, true, 4, 1050, 1500, 5000},
                                 {FAMILY_F64, 2, true, 4, 567, 1000, 5000},
                                 {FAMILY_F64, 0, false, 2, 2500, 2600, 6000},
-                                {FAMILY_F64, 1, false, 4, 1170, 2000, 6000},
+                                {FAMILY_F64, 1, false, 4, 1260, 2000, 6000},
                                 {FAMILY_F64, 2, false, 3, 960, 1300, 6000},
                                 {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000},
                                 {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000}};
@@ -570,63 +626,43 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
     return best;
 }
 
-// Plans that take a gather tile without a measurement (us, best register-fed
-// tile / gather tile, same box unless noted).
-//   Operands in 16-byte pieces: always.  10^4 6.7 / 6.1, 16^4 9.6 / 7.4, 24^4
-//   27.3 / 15.7, 36^4 95 / 85, permuted 64/32 575 / 508 (no pack, no panels).
-// Element by element, where the register-fed tiles do badly and operands
-// have unit-stride rows or k (others are packed once rather than gathered
-// by every tile):
-//   Batches, whose small instances leave each register tile a short loop of
-//   scattered reads: 4096-instance mix (1024 of them) 5478 / 4862, 1000 of
-//   extents 12-24 1946 / 1627, 200 of 10-40 2482 / 1922.
-//   Long k and few C tiles (under two 32 x 32 tiles per CU): without k
-//   slices the chip is idle.  32 x 32 x 131072 3125 / 21, 91 x 91 x 357
-//   (odd extents) 42 / 8.1.
-//   One to two 32 x 32 tiles per CU: the register tile runs a second, nearly
-//   empty round.  23^4 20.8 / 20.4, 33/17 permuted 37 / 29; up to one round
-//   it is the better one at this k (21^4 12.1 / 12.6) as long as it reads
-//   both operands in place.
-//   Short k (up to 64): packing an operand moves as many bytes as the
-//   contraction itself.  33 x 14553 x 21 13.1 / 7.8, 70 x 112000 x 40 75 / 59.
+// Does a plan take its best gather tile (us by the model) without a
+// measurement?  packed: the best register-fed tile's us (FP64).
+// FP64:
+//   Operands in 16-byte pieces: always (no pack, no panels).  10^4 6.7 / 6.1,
+//   16^4 9.6 / 7.4, 24^4 27.3 / 15.7, 36^4 95 / 85, permuted 64/32 575 / 508
+//   (us, packed / gathered).
+//   Batches: packing leaves each register tile a short loop of scattered
+//   reads.  4096-instance mix (1024 of them) 5478 / 4862, 1000 of extents
+//   12-24 1495 / 1224, 200 of 12-40 2949 / 2427.
+//   Otherwise element by element, where that costs less and operands have
+//   unit-stride rows or k (others are packed once rather than gathered by
+//   every tile): long k and few C tiles, cut along k (32 x 32 x 131072 3125 /
+//   21, 91 x 91 x 357 42 / 8.1), short k (33 x 14553 x 21 13.1 / 7.8, 70 x
+//   112000 x 40 75 / 59), small DPD blocks (27.5 / 17.9), 4489 x 225 x 4489
+//   254 / 203.
 // Split-BF16: all but GEMMs that fill the chip with 256 x 128 panel tiles
 // and use each packed element in 16 of them and more.  8^4 12.5 / 6.8, 24^4
 // 22.4 / 15.7, 36^4 81 / 44, 8-irrep DPD 48.7 / 29.7, 1024-instance batch
 // 3494 / 2246, 48^4 281 / 171, permuted 67/35 608 / 383; at 56^4 (325 tiles)
 // 468 / 463, at 61^4 (450) 657 / 718, at 80^4 2562 / 2856.
-bool gather_preferred(const std::vector<PanelGemm>& gemms, int family, int cus, bool pieces)
+bool gather_preferred(const std::vector<PanelGemm>& gemms, int family, int cus, const GatherChoice& c, double packed)
 {
-    if (pieces) return true;
-    if (family != FAMILY_F64)
-    {
-        double large = 0, all = 0;
-        for (const PanelGemm& g : gemms)
-        {
-            const double f = (double)g.mlen[0] * (double)g.nlen[0] * (double)total_k(g);
-            const int64_t m = g.mlen[0], n = g.nlen[0];
-            all += f;
-            if (std::min(m, n) >= 2048 && ceil_div(m, 256) * ceil_div(n, 128) >= 400) large += f;
-            for (const std::vector<PBlock>* bl : {&g.a, &g.b})
-                for (const PBlock& b : *bl)
-                    if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 &&
-                        side_count(b.k) > 1)
-                        return false;
-        }
-        return large <= 0.5 * all;
-    }
-    int64_t tiles = 0, kmax = 0;
+    if (c.pieces) return true;
+    double large = 0, all = 0;
     for (const PanelGemm& g : gemms)
     {
-        tiles += ceil_div(g.mlen[0], 32) * ceil_div(g.nlen[0], 32);
-        kmax = std::max(kmax, total_k(g));
+        const double f = (double)g.mlen[0] * (double)g.nlen[0] * (double)total_k(g);
+        const int64_t m = g.mlen[0], n = g.nlen[0];
+        all += f;
+        if (std::min(m, n) >= 2048 && ceil_div(m, 256) * ceil_div(n, 128) >= 400) large += f;
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
             for (const PBlock& b : *bl)
                 if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1)
                     return false;
     }
-    if (t_direct_all) return true;
-    if (tiles < 2 * cus) return tiles > cus || kmax >= 1024 || kmax <= 64;
-    return kmax <= 64;
+    if (family != FAMILY_F64) return large <= 0.5 * all;
+    return t_direct_all || c.us < packed;
 }
 
 }  // namespace
@@ -879,6 +915,12 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     const int nmodels = family == FAMILY_F64     ? (int)(sizeof(kModelsF64) / sizeof(kModelsF64[0]))
                         : family == FAMILY_OZAKI ? 1
                                                  : (int)(sizeof(kModelsBf16) / sizeof(kModelsBf16[0]));
+    // Plans in caller storage keep the tiles, and so the panel sizes, that
+    // their size limit was met with.
+    char* sbase = nullptr;
+    size_t sbytes = 0;
+    static_storage(sbase, sbytes);
+    const bool rounds = family == FAMILY_F64 && !sbase;
     std::vector<int> cands;
     for (int mi = 0; mi < nmodels; mi++)
     {
@@ -888,6 +930,7 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         if (panel_tile_lds(family, tm.tile) && !lds_applicable(gemms, family, dtype == 0 ? 8 : 4)) continue;
         cands.push_back(tm.tile);
         if (panel_tile_lds(family, tm.tile)) continue;  // gather tiles have a model of their own
+        if (rounds) continue;
         double c = tile_cost(gemms, tm, cus, family);
         if (best < 0 || c < best)
         {
@@ -895,19 +938,22 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
             tile = tm.tile;
         }
     }
-    // Gather tiles: chosen by their model where the register-fed tiles do
-    // badly; not for plans in caller storage, whose size limit a plan's
-    // panels are held against.
+    for (const RegisterTile& rt : kRegisterTiles)
     {
-        char* sbase = nullptr;
-        size_t sbytes = 0;
-        static_storage(sbase, sbytes);
-        if ((family == FAMILY_F64 || family == FAMILY_BF16X3) && !sbase && lds_applicable(gemms, family, dtype == 0 ? 8 : 4))
+        if (!rounds) break;
+        const double us = packed_us(gemms, rt, cus);
+        if (best < 0 || us < best)
         {
-            const std::vector<PanelGemm> walk = coalesced(gemms);
-            const GatherChoice c = gather_choice(walk, family, dtype == 0 ? 8 : 4, cus);
-            if (gather_preferred(walk, family, cus, c.pieces)) tile = c.tile;
+            best = us;
+            tile = rt.tile;
         }
+    }
+    // Gather tiles: by their own model, against the best register-fed tile.
+    if ((family == FAMILY_F64 || family == FAMILY_BF16X3) && !sbase && lds_applicable(gemms, family, dtype == 0 ? 8 : 4))
+    {
+        const std::vector<PanelGemm> walk = coalesced(gemms);
+        const GatherChoice c = gather_choice(walk, family, dtype == 0 ? 8 : 4, cus);
+        if (gather_preferred(walk, family, cus, c, best)) tile = c.tile;
     }
     bool packed = false;
     const int tuned = autotune_tile(gemms, family, dtype, swap, cands, tile);

@@ -238,3 +238,12 @@ def test_split_bf16_chosen_by_shape(m, n, k, gather, plans):
         T.lib().tblis_hip_clear_plan_cache()
         assert _f32_case(m, n, k, False, False, 0, g) <= 1e-6
         assert (T.last_tile() >= 6) == (gather and direct == "1")
+
+
+@pytest.mark.parametrize("m,n,k", [(1225, 1225, 120), (33, 4489, 225), (1025, 1023, 31), (2500, 31, 2499), (71, 5041, 35)])
+def test_tiles_by_rounds(m, n, k, plans):
+    """Odd extents, where whole rounds of waves choose among register-fed and
+    gather tiles, on every side of the rule's line."""
+    rng = np.random.default_rng(79000 + m)
+    _dense_case(rng, "ak", "kb", "ab", dict(a=m, b=n, k=k), ["col"] * 3, alpha=0.5, beta=2.0)
+    _dense_case(rng, "ak", "kb", "ab", dict(a=m, b=n, k=k), ["row", "col", "row"], alpha=1.0, beta=0.0)
