@@ -269,6 +269,64 @@ int64_t total_k(const PanelGemm& g)
     return k;
 }
 
+// Best split-BF16 panel tile of GEMMs that are packed, and its us.  A 16-k
+// step of the 256 x 128 tile (one workgroup to a CU) takes 0.95 us a round
+// and more the more CUs draw power, of the 128 x 128 tile 0.86 us a round; the
+// 64 x 64 ones, cut along k over two or four waves, fill the chip evenly.
+// Model / measured: 2401^3 (190 tiles) 0 215 / 205, 2809^3 (242) 0 268 / 272,
+// 3025^3 (288) 0 484 / 458, 3969^3 (512) 0 732 / 748, 2304^3 2 280 / 281;
+// complex 30^4 4 104 / 98, 40^4 0 264 / 269.  Against the rates of kModelsBf16
+// (us, rate / this): complex 30^4 126 / 98, 40^4 397 / 269, permuted 45/21
+// 268 / 215; 2601^3 350 / 240.
+struct SplitTile
+{
+    int tile;
+    double us;
+};
+SplitTile split_tile(const std::vector<PanelGemm>& gemms, int cus)
+{
+    struct Step
+    {
+        int tile;
+        int64_t bm, bn;
+        double round, share;  // us of 16 k: per round of tiles, and per CU's share of the tiles
+        double base;
+    };
+    constexpr Step steps[] = {{0, 256, 128, 0.95, 0.33, 0.0}, {2, 128, 128, 0.86, 0.0, 0.0},
+                              {4, 64, 64, 0.0, 0.26, 0.30},   {5, 64, 64, 0.0, 0.28, 0.27}};
+    double packed = 9.0;
+    int64_t klo = -1, khi = 0;
+    for (const PanelGemm& g : gemms)
+    {
+        int64_t m = 0, n = 0;
+        for (auto x : g.mlen) m += x;
+        for (auto x : g.nlen) n += x;
+        const int64_t k = ceil_div(total_k(g), 16);
+        packed += 10.0 * (double)(m + n) * (double)total_k(g) / 3.83e6;
+        klo = klo < 0 ? k : std::min(klo, k);
+        khi = std::max(khi, k);
+    }
+    SplitTile best{-1, 0};
+    for (const Step& st : steps)
+    {
+        double share = 0;  // 16-k steps of a CU's share of the tiles
+        for (const PanelGemm& g : gemms)
+        {
+            int64_t m = 0, n = 0;
+            for (auto x : g.mlen) m += x;
+            for (auto x : g.nlen) n += x;
+            share += (double)(ceil_div(m, st.bm) * ceil_div(n, st.bn) * ceil_div(total_k(g), 16)) / (double)cus;
+        }
+        // rounds: whole ones of equal tiles; those of several lengths fill
+        // one another's
+        const double rounds = klo == khi && khi > 0 ? std::ceil(share / (double)khi - 1e-9) * (double)khi
+                                                    : std::max((double)khi, share + 0.5 * (double)khi);
+        const double us = packed + st.round * rounds + st.share * share + st.base * (double)khi;
+        if (best.tile < 0 || us < best.us) best = SplitTile{st.tile, us};
+    }
+    return best;
+}
+
 // Estimated run time of the GEMM tasks for a tile.
 double tile_cost(const std::vector<PanelGemm>& gemms, const TileModel& tm, int cus, int family)
 {
@@ -542,8 +600,9 @@ struct GatherChoice
 // 17^4 10.3 / 10.2, 25^4 23 / 23.5, 31^4 59 / 60.  Split-BF16: 24^4 17 / 17.7
 // and 36^4 44 / 44.3 on the 64 x 64 tile, permuted 64/32 233 / 237 whole and
 // 214 / 210 in two slices on the 128 x 128 one; its stages are bound by L2
-// where short runs make it fetch lines that it uses a part of (line_share:
-// runs of 29 and 31 floats took 1.7-2.1 times the cycles).
+// where short runs make it fetch lines that it uses a part of (line_share: runs
+// of 29 and 31 floats, 2.0, took the 64 x 64 tile 1.7-2.1 times the cycles and
+// the 128 x 128 one 1.5-1.8; runs of 49 and 51, 1.6, the latter 1.07-1.17).
 GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int src_elem, int cus, int only = -1)
 {
     struct Model
@@ -561,7 +620,7 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
                                 {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000},
                                 {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000}};
     const bool f64 = family == FAMILY_F64;
-    double lines = 1.0;  // the worse operand of the largest GEMM
+    double share = 1.0;  // of the worse operand of the largest GEMM
     if (!f64)
     {
         const PanelGemm* big = &gemms[0];
@@ -569,8 +628,7 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
             if (g.mlen[0] * g.nlen[0] > big->mlen[0] * big->nlen[0] && total_k(g) > 0) big = &g;
         if (total_k(*big) > 0)
             for (const std::vector<PBlock>* bl : {&big->a, &big->b})
-                lines = std::max(lines, std::min(2.0, line_share(gather_operand(*bl, src_elem), src_elem)));
-        lines = 1.0 + 0.8 * (lines - 1.0);
+                share = std::max(share, std::min(2.0, line_share(gather_operand(*bl, src_elem), src_elem)));
     }
     constexpr double kGHz = 2.15;
     GatherChoice best;
@@ -586,6 +644,8 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
         const int64_t bk = panel_tile_k(family, tile);
         if (known != (int)bk) pieces = pieces_apply(gemms, src_elem, bk), known = (int)bk;
         if (f64 && md.pieces != pieces && md.lt != 0) continue;
+        const double over = std::max(0.0, share - 1.3);
+        const double lines = f64 ? 1.0 : md.lt == 0 ? 1.0 + 1.6 * over * over : std::max(1.0, 0.9 * share);
         int64_t kmax = 1;
         double bytes = 0;
         for (const PanelGemm& g : gemms)
@@ -608,14 +668,15 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
                 work += (double)nt * std::ceil(std::min((double)kslice, (double)k) / (double)bk) * md.stage * lines;
                 if (s > 1) panels += (f64 ? 8.0 : 4.0) * (double)s * (double)m * (double)n;
             }
-            if (S > 1 && (panels > (double)(64 << 20) || ntask > 8 * cus)) break;
+            if (S > 1 && (panels > (double)(128 << 20) || ntask > 8 * cus)) break;
             const double st = (double)(std::min(kslice, ceil_div(kmax, bk) * bk) / bk);
             const int64_t per = ceil_div(ntask, cus);
             double cyc;
             if (per <= md.occ)
                 cyc = md.fill + st * lines * std::max((double)per * md.stage, md.latency);
-            else if (gemms.size() == 1)
-                cyc = (double)ceil_div(per, md.occ) * md.fill + (double)per * st * md.stage * lines;
+            else if (gemms.size() == 1)  // 64 x 64 split-BF16 tiles in several rounds: bound by L2
+                cyc = (double)ceil_div(per, md.occ) * md.fill +
+                      (double)per * st * md.stage * lines * (!f64 && md.lt == 1 ? 1.16 : 1.0);
             else
                 cyc = (double)ceil_div(per, md.occ) * md.fill + std::max(1.05 * work / cus, st * md.stage * lines * md.occ);
             double us = std::max(cyc / (kGHz * 1e3), bytes / 5.5e6) + 1.5;
@@ -641,27 +702,27 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
 //   21, 91 x 91 x 357 42 / 8.1), short k (33 x 14553 x 21 13.1 / 7.8, 70 x
 //   112000 x 40 75 / 59), small DPD blocks (27.5 / 17.9), 4489 x 225 x 4489
 //   254 / 203.
-// Split-BF16: all but GEMMs that fill the chip with 256 x 128 panel tiles
-// and use each packed element in 16 of them and more.  8^4 12.5 / 6.8, 24^4
-// 22.4 / 15.7, 36^4 81 / 44, 8-irrep DPD 48.7 / 29.7, 1024-instance batch
-// 3494 / 2246, 48^4 281 / 171, permuted 67/35 608 / 383; at 56^4 (325 tiles)
-// 468 / 463, at 61^4 (450) 657 / 718, at 80^4 2562 / 2856.
-bool gather_preferred(const std::vector<PanelGemm>& gemms, int family, int cus, const GatherChoice& c, double packed)
+// Split-BF16: always, but for GEMMs with both sides from 2048 on, where the
+// 256 x 128 panel tiles (packed: their us) may fill their rounds better.
+// 8^4 12.5 / 6.8, 24^4 22.4 / 15.7, 36^4 81 / 44, 8-irrep DPD 48.7 / 29.7,
+// 1024-instance batch 3494 / 2246, 48^4 281 / 171, permuted 67/35 608 / 383;
+// 53^4 (242 tiles) 272 / 284, 55^4 (288) 458 / 419, 59^4 (392) 569 / 638,
+// 61^4 657 / 718, 80^4 2562 / 2856.
+bool gather_preferred(const std::vector<PanelGemm>& gemms, int family, const GatherChoice& c, double packed)
 {
     if (c.pieces) return true;
     double large = 0, all = 0;
     for (const PanelGemm& g : gemms)
     {
         const double f = (double)g.mlen[0] * (double)g.nlen[0] * (double)total_k(g);
-        const int64_t m = g.mlen[0], n = g.nlen[0];
         all += f;
-        if (std::min(m, n) >= 2048 && ceil_div(m, 256) * ceil_div(n, 128) >= 400) large += f;
+        if (std::min(g.mlen[0], g.nlen[0]) >= 2048) large += f;
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
             for (const PBlock& b : *bl)
                 if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1)
                     return false;
     }
-    if (family != FAMILY_F64) return large <= 0.5 * all;
+    if (family != FAMILY_F64) return large <= 0.5 * all || 1.06 * c.us < packed;
     return t_direct_all || c.us < packed;
 }
 
@@ -920,7 +981,7 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     char* sbase = nullptr;
     size_t sbytes = 0;
     static_storage(sbase, sbytes);
-    const bool rounds = family == FAMILY_F64 && !sbase;
+    const bool rounds = (family == FAMILY_F64 || family == FAMILY_BF16X3) && !sbase;
     std::vector<int> cands;
     for (int mi = 0; mi < nmodels; mi++)
     {
@@ -938,9 +999,15 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
             tile = tm.tile;
         }
     }
+    if (rounds && family == FAMILY_BF16X3)
+    {
+        const SplitTile st = split_tile(gemms, cus);
+        best = st.us;
+        tile = st.tile;
+    }
     for (const RegisterTile& rt : kRegisterTiles)
     {
-        if (!rounds) break;
+        if (!rounds || family != FAMILY_F64) break;
         const double us = packed_us(gemms, rt, cus);
         if (best < 0 || us < best)
         {
@@ -949,11 +1016,11 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         }
     }
     // Gather tiles: by their own model, against the best register-fed tile.
-    if ((family == FAMILY_F64 || family == FAMILY_BF16X3) && !sbase && lds_applicable(gemms, family, dtype == 0 ? 8 : 4))
+    if (rounds && lds_applicable(gemms, family, dtype == 0 ? 8 : 4))
     {
         const std::vector<PanelGemm> walk = coalesced(gemms);
         const GatherChoice c = gather_choice(walk, family, dtype == 0 ? 8 : 4, cus);
-        if (gather_preferred(walk, family, cus, c, best)) tile = c.tile;
+        if (gather_preferred(walk, family, c, best)) tile = c.tile;
     }
     bool packed = false;
     const int tuned = autotune_tile(gemms, family, dtype, swap, cands, tile);

@@ -228,10 +228,10 @@ def test_orders_of_the_general_path(dtype, plans):
 
 
 @pytest.mark.parametrize("m,n,k,gather", [(64, 64, 64, True), (1296, 1296, 1296, True), (32, 32, 8192, True),
-                                          (4096, 3712, 96, False)])
+                                          (4096, 4096, 2048, False)])
 def test_split_bf16_chosen_by_shape(m, n, k, gather, plans):
-    """Up to a few hundred 256 x 128 tiles the split-BF16 gather tiles run
-    without a knob; above, and with TBLIS_HIP_DIRECT=0, the panel tiles."""
+    """The split-BF16 gather tiles run without a knob; large operands in even
+    rounds of 256 x 128 tiles, and TBLIS_HIP_DIRECT=0, take the panel tiles."""
     g = torch.Generator(device=DEV).manual_seed(78000 + k)
     for direct in ("1", "0"):
         plans.setenv("TBLIS_HIP_DIRECT", direct)
@@ -247,3 +247,18 @@ def test_tiles_by_rounds(m, n, k, plans):
     rng = np.random.default_rng(79000 + m)
     _dense_case(rng, "ak", "kb", "ab", dict(a=m, b=n, k=k), ["col"] * 3, alpha=0.5, beta=2.0)
     _dense_case(rng, "ak", "kb", "ab", dict(a=m, b=n, k=k), ["row", "col", "row"], alpha=1.0, beta=0.0)
+
+
+@pytest.mark.parametrize("m,n,k", [(2304, 2304, 40), (2401, 2401, 96), (2049, 2047, 33), (2561, 2049, 1700)])
+def test_split_bf16_tiles_by_rounds(m, n, k, plans):
+    """Around the line between gathering and packing large operands."""
+    g = torch.Generator(device=DEV).manual_seed(80000 + m)
+    assert _f32_case(m, n, k, False, False, 0, g) <= 1e-6
+
+
+@pytest.mark.parametrize("v", [9, 17, 30, 33])
+def test_complex_split_bf16_tiles(v, plans):
+    """complex64 GEMMs over the sizes where the panel tile changes."""
+    from tests.test_gpu_complex import _case
+    rng = np.random.default_rng(81000 + v)
+    _case(rng, "abef", "efij", "abij", dict(a=v, b=v, e=3, f=7, i=v, j=v), torch.complex64, 0.5 - 0.25j, 1.0)
