@@ -750,6 +750,7 @@ PanelGemm transpose_gemm(const PanelGemm& g)
     t.b = g.a;
     t.kscale = g.kscale;
     t.kscale_im = g.kscale_im;
+    t.share = g.share ? 3 - g.share : 0;
     const size_t nm = g.mlen.size(), nn = g.nlen.size();
     t.c.resize(g.c.size());
     for (size_t p = 0; p < nm; p++)
@@ -1369,6 +1370,20 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
     return true;
 }
 
+// The operand (0 a, 1 b) that kscale is applied to.
+int scaled_operand(const PanelGemm& g) { return g.share == 1 ? 1 : 0; }
+
+// Do two GEMMs read one list of blocks as operand o (0 a, 1 b)?
+bool same_operand(const PanelGemm& x, const PanelGemm& y, int o)
+{
+    if (x.share != o + 1 || y.share != o + 1 || x.klen != y.klen) return false;
+    if ((o == 0 ? x.mlen : x.nlen) != (o == 0 ? y.mlen : y.nlen)) return false;
+    const std::vector<PBlock>&p = o == 0 ? x.a : x.b, &q = o == 0 ? y.a : y.b;
+    for (size_t i = 0; i < p.size() && p.size() == q.size(); i++)
+        if (p[i].base != q[i].base || !same_side(p[i].rows, q[i].rows) || !same_side(p[i].k, q[i].k)) return false;
+    return p.size() == q.size();
+}
+
 bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T,
                      const bool allow_direct[2], int src_elem)
 {
@@ -1463,6 +1478,11 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
         chunk_job(id, false, narrow_pack_groups(family));
     };
 
+    // plans in caller storage keep the panels that their size limit was met with
+    char* sbase = nullptr;
+    size_t sbytes = 0;
+    static_storage(sbase, sbytes);
+    int64_t prev_out[2] = {-1, -1};  // the previous GEMM's panels
     for (size_t gidx = 0; gidx < gemms.size(); gidx++)
     {
         const PanelGemm& g = gemms[gidx];
@@ -1473,7 +1493,11 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
         for (size_t i = 0; i < NN; i++) n0[i + 1] = n0[i] + g.nlen[i];
         for (size_t i = 0; i < NK; i++) k0[i + 1] = k0[i] + g.klen[i];
         const int64_t m = m0[NM], n = n0[NN], k = k0[NK];
-        if (m == 0 || n == 0) continue;
+        if (m == 0 || n == 0)
+        {
+            prev_out[0] = prev_out[1] = -1;
+            continue;
+        }
         const int64_t mp = ceil_div(m, BM) * BM, np = ceil_div(n, BN) * BN;
         const int64_t kp = ceil_div(k, G.kpad) * G.kpad;
         const int64_t nkg = kp / G.gk;
@@ -1506,7 +1530,7 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
         for (int o = 0; o < 2 && can_direct && direct_enabled() && kp > 0; o++)
         {
             if (!allow_direct[o] || nrp[o] != 1 || NK != 1) continue;
-            if (o == 0 && !g.kscale.empty() && g.kscale[0] != 1.0) continue;  // scaled while packed
+            if (o == scaled_operand(g) && !g.kscale.empty() && g.kscale[0] != 1.0) continue;  // scaled while packed
             const int64_t rereads = o == 0 ? ceil_div(n, BN) : ceil_div(m, BM);
             if (!general && rereads > std::max<int64_t>(direct_rows_rereads(), direct_kfast_rereads())) continue;
             if (scoped && rereads > 64) continue;
@@ -1560,17 +1584,22 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
         }
 
         // panels
-        const int64_t oa = ws;
-        if (!dir[0]) ws += G.terms * mp * kp;
-        const int64_t ob = ws;
-        if (!dir[1]) ws += G.terms * np * kp;
+        const PanelGemm* prev = gidx > 0 && !ozaki && !sbase ? &gemms[gidx - 1] : nullptr;
+        bool shared[2] = {false, false};
+        for (int o = 0; o < 2 && prev; o++) shared[o] = !dir[o] && prev_out[o] >= 0 && same_operand(*prev, g, o);
+        const int64_t oa = shared[0] ? prev_out[0] : ws;
+        if (!dir[0] && !shared[0]) ws += G.terms * mp * kp;
+        const int64_t ob = shared[1] ? prev_out[1] : ws;
+        if (!dir[1] && !shared[1]) ws += G.terms * np * kp;
+        prev_out[0] = dir[0] ? -1 : oa;
+        prev_out[1] = dir[1] ? -1 : ob;
         const int64_t ea = rows, eb = rows + mp;
         if (ozaki) rows += mp + np;
         const std::vector<int64_t>* rpre[2] = {&m0, &n0};
         const int64_t rpad[2] = {mp, np}, outs[2] = {oa, ob};
         for (int o = 0; o < 2 && kp > 0; o++)
         {
-            if (dir[o]) continue;
+            if (dir[o] || shared[o]) continue;
             const size_t NR = (o == 0 ? NM : NN);
             for (size_t p = 0; p < NR; p++)
                 for (size_t q = 0; q < NK; q++)
@@ -1586,7 +1615,7 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
                     j.pnkg = (int32_t)nkg;
                     j.operand = o;
                     j.eoff = o == 0 ? ea : eb;
-                    if (o == 0 && !g.kscale.empty()) j.scale = g.kscale[q];
+                    if (o == scaled_operand(g) && !g.kscale.empty()) j.scale = g.kscale[q];
                     if (j.nr == 0 || j.nk == 0) continue;
                     if (blk.base != PANEL_MISSING)
                     {

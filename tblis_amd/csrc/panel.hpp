@@ -31,10 +31,14 @@ struct PanelGemm
     std::vector<int64_t> mlen, nlen, klen;
     std::vector<PBlock> a, b;
     std::vector<CBlock> c;
-    std::vector<double> kscale;  // per k block, applied to A while packing (empty: all 1)
+    std::vector<double> kscale;  // per k block, applied to A (share 1: B) while packing (empty: all 1)
     // imaginary parts of the k-block scales of a complex GEMM (empty: all
     // 0); complex_split_gemms turns them into real term scales
     std::vector<double> kscale_im;
+    // An operand whose blocks (all of them, in order) the next GEMM may read
+    // as well, so that it is packed once: 1 a, 2 b; kscale is then applied to
+    // the other one.  0: neither.
+    int share = 0;
 };
 
 // C^T = B^T A^T.

@@ -189,3 +189,19 @@ def test_complex_batch(dtype, scalars):
         got = c.cpu().to(torch.complex128).numpy()
         err = np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-300)
         assert err <= TOL[dtype], (lA, lB, alpha, beta, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("a,i", [(37, 5), (5, 37), (16, 16)])
+@pytest.mark.parametrize("conj_A,conj_B", [(False, False), (True, False), (False, True), (True, True)])
+def test_packed_operand_read_by_both_parts(a, i, conj_A, conj_B, dtype, monkeypatch):
+    """The packed panels of the larger operand serve Re C and Im C: either
+    operand, either orientation of C, packed and not."""
+    rng = np.random.default_rng(82000 + a)
+    for direct in ("0", "1"):
+        monkeypatch.setenv("TBLIS_HIP_DIRECT", direct)
+        T.lib().tblis_hip_clear_plan_cache()
+        for C in ("abij", "ijba"):
+            _case(rng, "aebf", "fjei", C, dict(a=a, b=6, e=9, f=7, i=i, j=4), dtype, 0.5 - 0.25j, 1.0 + 0.5j,
+                  conj_A=conj_A, conj_B=conj_B)
+    T.lib().tblis_hip_clear_plan_cache()
