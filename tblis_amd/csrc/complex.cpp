@@ -92,7 +92,7 @@ struct Term
 // terms whose scale is zero are left out.  With s real, both read the larger
 // operand's parts in the same order (Ar, Ai or Br, Bi), which is packed once
 // for the two, and the signs go to the other operand: 4096 x 1024 x 4096
-// 2338 -> 2236 us in complex128, 987 -> 836 in complex64.
+// 2338 -> 2236 us in complex128 (pack 381 -> 276), 987 -> 836 in complex64.
 void split_gemm(const PanelGemm& g, double sa, double sb, std::vector<PanelGemm>& out)
 {
     const size_t NM = g.mlen.size(), NN = g.nlen.size(), NK = g.klen.size();
