@@ -483,6 +483,30 @@ void tblis_hip_debug_fill_block_scatter(int ndim, const len_type* len, const str
 int64_t tblis_hip_debug_panel_side(int ndim, const len_type* len, const stride_type* stride, len_type G,
                                    len_type r0, stride_type* offs, stride_type* tab, int64_t max_out);
 
+/* The plan of a dense contraction, from the planner's host tables alone.
+ * aligned: whether A and B are taken to start on 16 bytes.  out receives
+ * TBLIS_HIP_PLAN_HEADER int64:
+ *   [tile, gather tile, 16-byte pieces, most k slices of a GEMM, A and B
+ *    exchanged, k per stage, tile rows, tile columns, bytes per element of
+ *    the real tensors, kernel family, tasks, slice sums, table entries,
+ *    scaled k blocks, tasks of groups 0..8]
+ * and, for a gather tile, 16 int64 per task in launch order
+ *   [group, first k, k end, A start, B start, A row table, B row table,
+ *    A k table, B k table, k scales, rows, columns, C start, C row table,
+ *    C column table, leading dimension (0: C itself, else a slice's sums)],
+ * 8 per slice sum
+ *   [C start, C row table, C column table, sums start, rows, columns,
+ *    slices, distance between slices],
+ * and the tables.  Starts are in elements of the real type, A and B row and
+ * k tables in bytes from the start (split-BF16 k tables: 32-bit words).
+ * Returns the number of int64, 0 when there is nothing to launch, -2 if
+ * max_out is too small, -1 on error. */
+#define TBLIS_HIP_PLAN_HEADER 24
+int64_t tblis_hip_debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_type* idx_A,
+                             const tblis_tensor* B, const label_type* idx_B,
+                             const tblis_tensor* C, const label_type* idx_C, int aligned,
+                             int64_t* out, int64_t max_out);
+
 /* DPD block address (offset from the data pointer, lengths, strides) of the
  * block with the given irreps, from this library's DPD layout code. */
 void tblis_hip_debug_dpd_block(const tblis_dpd_tensor* t, const unsigned* irreps,

@@ -96,7 +96,7 @@ EXPORTED = [
     "tblis_hip_set_autotune", "tblis_hip_autotune_runs", "tblis_hip_last_tile", "tblis_hip_last_direct",
     "tblis_hip_tensor_mult_noalloc", "tblis_hip_device_alloc_count",
     "tblis_hip_debug_canonical", "tblis_hip_debug_fill_block_scatter", "tblis_hip_debug_panel_side",
-    "tblis_hip_debug_dpd_block",
+    "tblis_hip_debug_plan", "tblis_hip_debug_dpd_block",
     "tblis_hip_debug_dpd_patches", "tblis_hip_debug_mfma_probe", "tblis_hip_debug_mfma_probe_bf16",
 ]
 
@@ -133,6 +133,9 @@ def lib():
         L.tblis_hip_debug_panel_side.restype = C.c_int64
         L.tblis_hip_debug_panel_side.argtypes = [C.c_int, P(C.c_ssize_t), P(C.c_ssize_t), C.c_ssize_t,
                                                  C.c_ssize_t, P(C.c_ssize_t), P(C.c_ssize_t), C.c_int64]
+        L.tblis_hip_debug_plan.restype = C.c_int64
+        L.tblis_hip_debug_plan.argtypes = [C.c_void_p, T, C.c_char_p, T, C.c_char_p, T, C.c_char_p, C.c_int,
+                                           P(C.c_int64), C.c_int64]
         L.tblis_get_config.restype = C.c_void_p
         L.tblis_get_config.argtypes = [C.c_char_p]
         L.tblis_hip_get_last_error.restype = C.c_char_p

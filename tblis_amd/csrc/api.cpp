@@ -493,6 +493,15 @@ int64_t tblis_hip_debug_panel_side(int ndim, const len_type* len, const stride_t
         (int64_t)-1);
 }
 
+int64_t tblis_hip_debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_type* idx_A,
+                             const tblis_tensor* B, const label_type* idx_B,
+                             const tblis_tensor* C, const label_type* idx_C, int aligned,
+                             int64_t* out, int64_t max_out)
+{
+    return guarded(
+        [&] { return debug_plan(cfg, A, idx_A, B, idx_B, C, idx_C, aligned != 0, out, max_out); }, (int64_t)-1);
+}
+
 void tblis_hip_debug_dpd_block(const tblis_dpd_tensor* t, const unsigned* irreps, len_type* len,
                                stride_type* offset, stride_type* stride)
 {

@@ -3,6 +3,7 @@
 
 #include <cstring>
 
+#include "kernels.hpp"
 #include "panel.hpp"
 #include "plan.hpp"
 
@@ -298,6 +299,72 @@ void tensor_mult(const tblis_config* cfg, const tblis_tensor* A, const label_typ
         }
     }
     reset_scalar(C);
+}
+
+int64_t debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_type* idx_A,
+                   const tblis_tensor* B, const label_type* idx_B, const tblis_tensor* C,
+                   const label_type* idx_C, bool aligned, int64_t* out, int64_t max_out)
+{
+    check_tensor(A, idx_A, "A");
+    check_tensor(B, idx_B, "B");
+    check_tensor(C, idx_C, "C");
+    if (A->type != B->type || A->type != C->type) fail("A, B and C must have the same type");
+    const bool cplx = A->type == TYPE_SCOMPLEX || A->type == TYPE_DCOMPLEX;
+    const type_t rtype = A->type == TYPE_DOUBLE || A->type == TYPE_DCOMPLEX ? TYPE_DOUBLE : TYPE_SINGLE;
+    const int family = family_of(resolve_algo(cfg, rtype));
+    Canonical c;
+    std::string why;
+    if (!canonicalize(*A, idx_A, *B, idx_B, *C, idx_C, c, why)) fail("invalid contraction: " + why);
+    GemmDesc g;
+    if (!dense_gemm(c, g, 0, 0, 0)) return 0;
+    std::vector<PanelGemm> gemms;
+    panel_from_desc(g, gemms);
+    if (cplx)
+    {
+        std::vector<PanelGemm> parts;
+        complex_split_gemms(gemms, A->conj ? -1.0 : 1.0, B->conj ? -1.0 : 1.0, parts);
+        gemms.swap(parts);
+    }
+    PanelTables T;
+    {
+        AlignedScope pieces(aligned && !cplx);
+        if (!plan_panel_tables(std::move(gemms), T, family, dtype_code(rtype))) return 0;
+    }
+    const bool gather = panel_tile_lds(family, T.tile);
+    std::vector<int64_t> v = {T.tile,
+                              gather,
+                              T.pieces,
+                              T.slices,
+                              T.swap,
+                              panel_tile_k(family, T.tile),
+                              panel_tile_m(family, T.tile),
+                              panel_tile_n(family, T.tile),
+                              elem_size(rtype),
+                              family,
+                              (int64_t)T.tasks.size(),
+                              (int64_t)T.ujobs.size(),
+                              (int64_t)T.pool.size(),
+                              T.scaled};
+    v.insert(v.end(), T.group_n, T.group_n + kTaskGroups);
+    v.resize(TBLIS_HIP_PLAN_HEADER, 0);
+    if (gather)
+    {
+        int group = 0;
+        int64_t left = T.group_n[0];
+        for (const PanelTask& t : T.tasks)
+        {
+            while (left == 0) left = T.group_n[++group];
+            left--;
+            v.insert(v.end(), {group, t.kbeg, t.klen, t.a_src, t.b_src, t.a_rt, t.b_rt, t.a_km, t.b_km, t.a_kt,
+                               t.mlen, t.nlen, t.c_src, t.c_rowmap, t.c_colmap, t.c_ld});
+        }
+        for (const UnpackJob& u : T.ujobs)
+            v.insert(v.end(), {u.dst, u.rowmap, u.colmap, u.panel, u.nr, u.nc, u.nslice, u.sstride});
+        v.insert(v.end(), T.pool.begin(), T.pool.end());
+    }
+    if ((int64_t)v.size() > max_out) return -2;
+    std::copy(v.begin(), v.end(), out);
+    return (int64_t)v.size();
 }
 
 // The same contraction with its plan tables and workspace in the device

@@ -74,6 +74,11 @@ void complex_tensor_mult(const tblis_config* cfg, const tblis_tensor* A, const l
                          const tblis_tensor* B, const label_type* idx_B, tblis_tensor* C,
                          const label_type* idx_C);
 
+// tblis_hip_debug_plan.
+int64_t debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_type* idx_A,
+                   const tblis_tensor* B, const label_type* idx_B, const tblis_tensor* C,
+                   const label_type* idx_C, bool aligned, int64_t* out, int64_t max_out);
+
 // The batched GEMM of a canonical contraction (m = AC, n = BC, k = AB,
 // batch = ABC) at the given element bases; false when C is empty.
 bool dense_gemm(const Canonical& c, GemmDesc& g, int64_t base_a, int64_t base_b, int64_t base_c);

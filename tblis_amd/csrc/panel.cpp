@@ -438,7 +438,8 @@ std::vector<int64_t> side_offsets(const Side& s)
 // and ks in bytes from its lowest element, itself at an even element.  Lanes
 // along rows: rows in aligned pairs.  Lanes along k: every stage of bk k is
 // one aligned run.  Both: the offsets within a stage, from its first k, are
-// the same in every stage, and stages start on 16 bytes.
+// the same in every stage and not negative (the kernel adds them as unsigned
+// words to the stage's first), and stages start on 16 bytes.
 bool vec_layout(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks, int64_t src, bool lanes_k, int64_t bk)
 {
     if (src % 2 || (lanes_k ? ks : rows).size() % 2) return false;
@@ -451,7 +452,7 @@ bool vec_layout(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks
     for (size_t i = 0; i < ks.size(); i++)
     {
         const int64_t at = ks[i] - ks[i - i % bk];
-        if (at != (lanes_k ? 8 * (int64_t)(i % bk) : ks[i % bk] - ks[0])) return false;
+        if (at < 0 || at != (lanes_k ? 8 * (int64_t)(i % bk) : ks[i % bk] - ks[0])) return false;
         if ((!lanes_k || i % bk == 0) && ks[i] % 16) return false;
     }
     return true;

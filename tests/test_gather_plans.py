@@ -1,0 +1,189 @@
+"""The tables of the gather tiles (tblis_hip_debug_plan) on the host: every
+address that the kernels form from them, in their own 32- and 64-bit
+arithmetic, lies inside its operand and on the boundary its load needs, and
+the products at these addresses are the contraction.  Inputs are small whole
+numbers, so the comparison is exact."""
+import ctypes as C
+import itertools
+
+import numpy as np
+import pytest
+
+import tblis_amd as T
+from tests.test_boundary import _HostDesc
+
+HEADER = 24  # TBLIS_HIP_PLAN_HEADER
+F64, F32, C64, C128 = T.TYPE_DOUBLE, T.TYPE_SINGLE, T.TYPE_SCOMPLEX, T.TYPE_DCOMPLEX
+
+
+class Plan:
+    """A plan of C = A B over tensors given as (lengths, strides, labels)."""
+
+    def __init__(self, A, B, C_, dtype=F64, aligned=True, config=None):
+        d = [_HostDesc(x[0], x[1], dtype) for x in (A, B, C_)]
+        args = [y for t, x in zip(d, (A, B, C_)) for y in (C.byref(t.d), x[2].encode("latin1"))]
+        cap = 1 << 22
+        out = np.zeros(cap, dtype=np.int64)
+        n = T.lib().tblis_hip_debug_plan(T.get_config(config) if config else None, *args, int(aligned),
+                                         out.ctypes.data_as(C.POINTER(C.c_int64)), cap)
+        assert n >= HEADER, (n, T.last_error())
+        (self.tile, self.gather, self.pieces, self.slices, self.swap, self.bk, self.bm, self.bn, self.elem,
+         self.family, nt, nu, npool, self.scaled) = (int(x) for x in out[:14])
+        self.groups = {g: int(x) for g, x in enumerate(out[14:23]) if x}
+        if self.gather:
+            at = HEADER
+            self.tasks = out[at:at + 16 * nt].reshape(nt, 16)
+            at += 16 * nt
+            self.sums = out[at:at + 8 * nu].reshape(nu, 8)
+            self.pool = out[at + 8 * nu:n].copy()
+            assert len(self.pool) == npool
+
+    def loads(self, o, t, data, lo):
+        """Operand o's tile of task t as the kernel reads it from data, whose
+        first element is element lo of the tensor."""
+        group, kbeg, kend = (int(x) for x in t[:3])
+        src, rt, km = (int(t[3 + o + 2 * i]) for i in range(3))
+        valid = int(t[10 + o])
+        f64 = self.family == 0
+        mode = (group >> o) & 1 if f64 else group // 3 ** o % 3
+        size = self.bm if o == 0 else self.bn
+        nk = kend - kbeg
+        stages = -(-nk // self.bk)
+        # the kernels load up to a stage past the end
+        k = np.arange((stages + (0 if self.pieces else 1)) * self.bk)
+        r = np.arange(size)
+        wrap = (1 << 32) - 1
+        ks = self.pool[km:] if f64 else self.pool[km:].view(np.uint32).astype(np.int64)
+        ks = ks[kbeg:]
+        row = lambda r: self.pool[rt + np.where(r < valid, r, 0)]
+        if self.pieces:
+            first = ks[k - k % self.bk]
+            lead = k % self.bk if not mode else k % self.bk - k % self.bk % 2
+            delta = (ks[np.where(lead < nk, lead, 0)] - ks[0]) & wrap
+            rows = row(r - r % 2 if not mode else r)
+            at = first + (((rows & wrap)[:, None] + delta) & wrap)
+            keep = k < nk
+            assert (at[:, keep] + src * 8 >= lo * 8).all() and ((at[:, keep] + src * 8) % 16 == 0).all()
+            at += 8 * ((r % 2)[:, None] if not mode else k % 2)
+            at, k = at[:, keep], k[keep]
+        else:
+            assert (ks[:len(k)] >= 0).all() and (ks[:len(k)] <= wrap).all()
+            at = row(r)[:, None] + (ks[k] if mode < 2 else ks[k - k % 8])
+            assert (at >= 0).all() and (at <= wrap).all()
+            if mode == 2:
+                assert ((at + src * 4) % 16 == 0).all()
+                at = at + 4 * (k % 8)
+        at = at + src * self.elem
+        assert (at % self.elem == 0).all()
+        at = at // self.elem - lo
+        assert (at >= 0).all() and (at < len(data)).all(), (at.min(), at.max(), len(data))
+        return data[at][:valid, :nk]
+
+    def run(self, a, b, c):
+        """C += A B on host arrays (each: data, lo) through the plan's tables."""
+        ops = (b, a) if self.swap else (a, b)
+        slices = np.zeros(sum(int(u[4] * u[5] * u[6]) for u in self.sums))
+        for t in self.tasks:
+            x, y = (self.loads(o, t, *ops[o]) for o in range(2))
+            if self.scaled:
+                x = x * self.pool[int(t[9]) + int(t[1]):][:x.shape[1]].view(np.float64)
+            p = x @ y.T
+            i, j = (np.arange(int(t[10 + o])) for o in range(2))
+            if t[15]:
+                slices[int(t[12]) + i[:, None] * int(t[15]) + j] = p
+            else:
+                self.store(c, t[12:15], p)
+        for u in self.sums:
+            m, n = int(u[4]), int(u[5])
+            p = sum(slices[int(u[3]) + s * int(u[7]):][:m * n] for s in range(int(u[6])))
+            self.store(c, u[:3], p.reshape(m, n))
+
+    def store(self, c, at, p):
+        data, lo = c
+        i, j = (np.arange(x) for x in p.shape)
+        at = int(at[0]) + self.pool[int(at[1]) + i][:, None] + self.pool[int(at[2]) + j] - lo
+        assert (at >= 0).all() and (at < len(data)).all()
+        data[at] += p
+
+
+def _span(lens, strides):
+    reach = [(n - 1) * s for n, s in zip(lens, strides)]
+    return sum(min(x, 0) for x in reach), sum(max(x, 0) for x in reach)
+
+
+def _check(A, B, C_, dtype=F64, **kw):
+    """The plan's products against numpy's; returns the plan."""
+    plan = Plan(A, B, C_, dtype, **kw)
+    if not plan.gather:
+        return plan
+    parts = 2 if dtype in (C64, C128) else 1
+    rng = np.random.default_rng(1)
+    flat, view = [], []
+    for lens, strides, _ in (A, B, C_):
+        lo, hi = _span(lens, strides)
+        x = rng.integers(-4, 5, size=parts * (hi - lo + 1)).astype(np.float64)
+        flat.append((x, parts * lo))
+        x = x.view(np.complex128) if parts == 2 else x
+        view.append(np.lib.stride_tricks.as_strided(x[-lo:], lens, [s * x.itemsize for s in strides]))
+    want = np.array(view[2]) + np.einsum(f"{A[2]},{B[2]}->{C_[2]}", view[0], view[1])
+    plan.run(*flat)
+    assert (np.array(view[2]) == want).all()
+    return plan
+
+
+def _packed(lens):
+    return [int(np.prod(lens[:i])) for i in range(len(lens))]
+
+
+def _tensor(ext, labels, negative="", gap=1):
+    """Packed in the order of the labels (gap: of the first stride), the
+    strides of `negative` turned round."""
+    lens = [ext[x] for x in labels]
+    return lens, [(-s if x in negative else s) * gap for s, x in zip(_packed(lens), labels)], labels
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+@pytest.mark.parametrize("negA,negB", [("k", ""), ("", "k"), ("k", "k"), ("a", ""), ("ak", "b"), ("ak", "bk")])
+@pytest.mark.parametrize("A,B", [("ak", "kb"), ("ka", "kb"), ("ak", "bk"), ("ka", "bk")])
+def test_negative_strides(A, B, negA, negB, dtype):
+    """Rows, k or both of an operand in descending order, on extents that
+    allow 16-byte pieces when they ascend."""
+    for ext in (dict(a=64, b=64, k=64), dict(a=34, b=66, k=80), dict(a=8, b=8, k=4096)):
+        plan = _check(_tensor(ext, A, negA), _tensor(ext, B, negB), _tensor(ext, "ab"), dtype)
+        if dtype == F64 and not negA + negB:
+            assert plan.pieces
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+def test_negative_strides_in_two_dimensions_of_k(dtype):
+    """k = (e, f): either of them descending, in both operands or in one."""
+    ext = dict(a=32, e=16, f=6, b=34)
+    for negA, negB in itertools.product(["", "e", "f", "ef"], repeat=2):
+        for A, B in (("aef", "efb"), ("efa", "bfe"), ("eaf", "ebf")):
+            plan = _check(_tensor(ext, A, negA), _tensor(ext, B, negB), _tensor(ext, "ab"), dtype)
+            assert plan.gather or (negA + negB)
+
+
+@pytest.mark.parametrize("seed", range(60))
+def test_forms_of_the_general_path(seed, monkeypatch):
+    """Orders of the labels, gaps, negative and zero strides, odd extents,
+    every gather tile and number of slices, aligned tensors or not."""
+    rng = np.random.default_rng(8000 + seed)
+    ran = 0
+    for dtype, tiles in ((F64, "9 10 11"), (F32, "6 7"), (C128, "9 10 11")):
+        for tile in tiles.split():
+            monkeypatch.setenv("TBLIS_HIP_PANEL_TILE", tile)
+            monkeypatch.setenv("TBLIS_HIP_KSPLIT", str(rng.choice([1, 1, 2, 3])))
+            ext = {x: int(rng.choice([1, 2, 3, 4, 5, 8, 16, 17])) for x in "abij"}
+            ext.update({x: int(rng.choice([1, 2, 3, 7, 8, 16, 32])) for x in "ef"})
+            form = []
+            for labels in ("abef", "efij", "abij"):
+                s = "".join(rng.permutation(list(labels)))
+                neg = "".join(x for x in s if rng.random() < 0.15)
+                lens, strides, s = _tensor(ext, s, neg, int(rng.choice([1, 1, 1, 2])))
+                if labels != "abij" and rng.random() < 0.15:
+                    strides[int(rng.integers(4))] = 0
+                form.append((lens, strides, s))
+            plan = _check(*form, dtype, aligned=bool(rng.integers(2)))
+            ran += plan.gather and plan.tile == int(tile)
+    assert ran == 8

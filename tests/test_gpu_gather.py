@@ -262,3 +262,44 @@ def test_complex_split_bf16_tiles(v, plans):
     from tests.test_gpu_complex import _case
     rng = np.random.default_rng(81000 + v)
     _case(rng, "abef", "efij", "abij", dict(a=v, b=v, e=3, f=7, i=v, j=v), torch.complex64, 0.5 - 0.25j, 1.0)
+
+
+def _mult_turned(A, la, negA, B, lb, negB, C_, lc, negC, alpha, beta):
+    """T.mult on descriptors whose dimensions in neg* run backwards (data at
+    their last element, negative stride); returns the tensors as seen."""
+    import ctypes
+    from tblis_amd import _Desc
+    descs, seen = [], []
+    for x, labels, neg, s in ((A, la, negA, alpha), (B, lb, negB, 1.0), (C_, lc, negC, beta)):
+        d = _Desc(x, s)
+        at = x.data_ptr()
+        for i, label in enumerate(labels):
+            if label in neg:
+                at += (x.shape[i] - 1) * x.stride(i) * x.element_size()
+                d.stride[i] = -x.stride(i)
+        d.d.data = ctypes.c_void_p(at)
+        descs.append(d)
+        seen.append(lambda x=x, labels=labels, neg=neg:
+                    x.double().cpu().flip([i for i, label in enumerate(labels) if label in neg]).numpy())
+    before = [s() for s in seen]
+    T.lib().tblis_tensor_mult(None, None, *[y for d, labels in zip(descs, (la, lb, lc))
+                                            for y in (ctypes.byref(d.d), labels.encode())])
+    torch.cuda.synchronize()
+    return before, seen[2]()
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, FP64_TOL), (torch.float32, 1e-6)])
+def test_negative_strides(dtype, tol, plans):
+    """Descending rows, k, both, and results, on even extents (where ascending
+    operands are read in 16-byte pieces) and odd ones, against the general
+    path's bar for each type."""
+    g = torch.Generator(device=DEV).manual_seed(83000)
+    for ext in (dict(a=64, b=66, e=8, f=16), dict(a=33, b=7, e=5, f=13), dict(a=16, b=16, e=64, f=80)):
+        for la, lb in (("aef", "efb"), ("fea", "bef"), ("eaf", "ebf")):
+            for negA, negB, negC in (("e", "", ""), ("ef", "", ""), ("a", "b", "a"), ("aef", "bef", ""),
+                                     ("", "f", "b"), ("ef", "ef", "ab")):
+                A, B, C = (torch.rand([ext[x] for x in reversed(s)], dtype=dtype, device=DEV, generator=g)
+                           .permute(*reversed(range(len(s)))) - 0.5 for s in (la, lb, "ab"))
+                (a, b, c), got = _mult_turned(A, la, negA, B, lb, negB, C, "ab", negC, 1.5, -0.5)
+                want = 1.5 * np.einsum(f"{la},{lb}->ab", a, b) - 0.5 * c
+                assert rel_fro(got, want) <= tol, (ext, la, lb, negA, negB, negC)
