@@ -484,12 +484,14 @@ int64_t tblis_hip_debug_panel_side(int ndim, const len_type* len, const stride_t
                                    len_type r0, stride_type* offs, stride_type* tab, int64_t max_out);
 
 /* The plan of a dense contraction, from the planner's host tables alone.
- * aligned: whether A and B are taken to start on 16 bytes.  out receives
+ * aligned: whether A and B are taken to start on 16 bytes.  The data are
+ * not read; with the autotuner on, results that it has already apply, as
+ * they do to calls on these tensors.  out receives
  * TBLIS_HIP_PLAN_HEADER int64:
  *   [tile, gather tile, 16-byte pieces, most k slices of a GEMM, A and B
  *    exchanged, k per stage, tile rows, tile columns, bytes per element of
  *    the real tensors, kernel family, tasks, slice sums, table entries,
- *    scaled k blocks, tasks of groups 0..8]
+ *    scaled k blocks, tasks of groups 0..8, key of the tuning file's line]
  * and, for a gather tile, 16 int64 per task in launch order
  *   [group, first k, k end, A start, B start, A row table, B row table,
  *    A k table, B k table, k scales, rows, columns, C start, C row table,

@@ -328,6 +328,8 @@ int64_t debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_t
     PanelTables T;
     {
         AlignedScope pieces(aligned && !cplx);
+        TuneOperandsScope ops(A->data, B->data);
+        AutotuneRecallScope recall;
         if (!plan_panel_tables(std::move(gemms), T, family, dtype_code(rtype))) return 0;
     }
     const bool gather = panel_tile_lds(family, T.tile);
@@ -346,7 +348,7 @@ int64_t debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_t
                               (int64_t)T.pool.size(),
                               T.scaled};
     v.insert(v.end(), T.group_n, T.group_n + kTaskGroups);
-    v.resize(TBLIS_HIP_PLAN_HEADER, 0);
+    v.push_back((int64_t)T.tune_key);
     if (gather)
     {
         int group = 0;

@@ -926,6 +926,9 @@ constexpr int kPackedBit = 256;
 // packed variant) or -1.
 int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bool swap,
                   const std::vector<int>& cands, int model_tile);
+uint64_t tune_key(const std::vector<PanelGemm>& gemms, int family, bool real);
+// Do the tuner's candidates run on the tensors?
+bool tune_real(int family);
 
 struct TuneOperands
 {
@@ -933,7 +936,8 @@ struct TuneOperands
     const void* B = nullptr;
 };
 thread_local TuneOperands t_tune_ops;
-thread_local bool t_tune_off = false;    // AutotuneOffScope
+thread_local bool t_tune_off = false;     // AutotuneOffScope
+thread_local bool t_tune_recall = false;  // AutotuneRecallScope
 
 }  // namespace
 
@@ -945,6 +949,9 @@ AlignedScope::~AlignedScope() { t_aligned = was_; }
 
 AutotuneOffScope::AutotuneOffScope() : was_(t_tune_off) { t_tune_off = true; }
 AutotuneOffScope::~AutotuneOffScope() { t_tune_off = was_; }
+
+AutotuneRecallScope::AutotuneRecallScope() : was_(t_tune_recall) { t_tune_recall = true; }
+AutotuneRecallScope::~AutotuneRecallScope() { t_tune_recall = was_; }
 
 TuneOperandsScope::TuneOperandsScope(const void* A, const void* B) { t_tune_ops = TuneOperands{A, B}; }
 TuneOperandsScope::~TuneOperandsScope() { t_tune_ops = TuneOperands{}; }
@@ -1044,6 +1051,7 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     }
     if (!tables_uniform(gemms, family, tile, T, dtype == 0 ? 8 : 4, packed)) return false;
     T.swap = swap;
+    if (t_tune_recall) T.tune_key = tune_key(gemms, family, tune_real(family));
     return true;
 }
 
@@ -1946,29 +1954,48 @@ void save_tune(int family, uint64_t h, int code)
     std::fclose(f);
 }
 
-// Stride signature of the single-block operands: with tensors to read, the
-// groups of directly read operands (and so the timing) depend on it.
-std::string layout_sig(const std::vector<PanelGemm>& gemms)
+// Hash of what, with tensors to read, decides how a tile loads them and
+// whether a gather tile can: every block's place (from the operand's first),
+// lengths, strides and offsets, scaled and shared blocks, alignment.
+uint64_t layout_hash(const std::vector<PanelGemm>& gemms)
 {
-    std::string sig;
+    uint64_t h = 1469598103934665603ULL;
+    auto put = [&](int64_t x) { h = (h ^ (uint64_t)x) * 1099511628211ULL; };
+    auto list = [&](const std::vector<int64_t>& v) {
+        put((int64_t)v.size());
+        for (int64_t x : v) put(x);
+    };
+    put(t_aligned);
     for (const PanelGemm& g : gemms)
+    {
+        put(g.share);
+        bool scaled = false;
+        for (double x : g.kscale) scaled = scaled || x != 1.0;
+        put(scaled);
+        list(g.mlen);
+        list(g.nlen);
+        list(g.klen);
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
         {
-            sig += bl->size() == 1 ? "|" : "|m";
-            if (bl->size() != 1) continue;
-            for (const Side* sd : {&(*bl)[0].rows, &(*bl)[0].k})
+            put((int64_t)bl->size());
+            for (const PBlock& b : *bl)
             {
-                for (int64_t x : sd->stride) sig += std::to_string(x) + ",";
-                if (!sd->offs.empty())
-                {
-                    uint64_t h = 1469598103934665603ULL;
-                    for (int64_t x : sd->offs) h = (h ^ (uint64_t)x) * 1099511628211ULL;
-                    sig += "x" + std::to_string(h);
-                }
-                sig += "/";
+                put(b.base == PANEL_MISSING ? b.base : b.base - (*bl)[0].base);
+                for (const Side* sd : {&b.rows, &b.k}) list(sd->len), list(sd->stride), list(sd->offs);
             }
         }
-    return sig;
+    }
+    return h;
+}
+
+bool tune_real(int family) { return family != FAMILY_OZAKI && t_tune_ops.A && t_tune_ops.B && direct_enabled(); }
+
+// Key of the measurement for these GEMMs; real: candidates run on the tensors.
+uint64_t tune_key(const std::vector<PanelGemm>& gemms, int family, bool real)
+{
+    uint64_t h = shape_hash(gemms, family);
+    if (real) h = fnv1a(std::to_string(h) + "r" + std::to_string(layout_hash(gemms)));
+    return h;
 }
 
 int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bool swap,
@@ -1976,6 +2003,21 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
 {
     const std::vector<int>& cands0 = cands_in;
     if (t_tune_off || !autotune_on() || cands0.size() < 2) return -1;
+    // time candidates as they will run when the tensors can be read
+    const TuneOperands ops = t_tune_ops;
+    const bool real = tune_real(family);
+    const void* opA = swap ? ops.B : ops.A;
+    const void* opB = swap ? ops.A : ops.B;
+    const uint64_t h = tune_key(gemms, family, real);
+    TuneDb& db = tune_db();
+    std::lock_guard<std::mutex> lock(db.mu);
+    if (!db.loaded) load_tune_file(db);
+    auto it = db.best.find(h ^ (uint64_t)family);
+    // (a tuning file may name a tile that these GEMMs cannot run on)
+    if (it != db.best.end() &&
+        std::find(cands0.begin(), cands0.end(), it->second % kPackedBit) != cands0.end())
+        return it->second;
+    if (t_tune_recall) return -1;
     hipStream_t s = thread_state().stream;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
@@ -1983,18 +2025,6 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
         (void)hipGetLastError();
         return -1;  // no allocation or timing inside a graph capture
     }
-    // time candidates as they will run when the tensors can be read (FP64)
-    const TuneOperands ops = t_tune_ops;
-    const bool real = family != FAMILY_OZAKI && ops.A && ops.B && direct_enabled();
-    const void* opA = swap ? ops.B : ops.A;
-    const void* opB = swap ? ops.A : ops.B;
-    uint64_t h = shape_hash(gemms, family);
-    if (real) h = fnv1a(std::to_string(h) + "r" + layout_sig(gemms));
-    TuneDb& db = tune_db();
-    std::lock_guard<std::mutex> lock(db.mu);
-    if (!db.loaded) load_tune_file(db);
-    auto it = db.best.find(h ^ (uint64_t)family);
-    if (it != db.best.end()) return it->second;
 
     // Without the tensors (or with direct reads off) the candidates run
     // from packed panels, which the LDS-staged tiles never read.

@@ -97,6 +97,7 @@ struct PanelTables
     int64_t ws_rows = 0;   // Ozaki: row-maximum entries (one per panel row)
     int64_t ws_c = 0;      // C panel doubles
     int64_t useful_flops = 0, mfma_flops = 0;
+    uint64_t tune_key = 0;  // AutotuneRecallScope
 };
 
 // Can the gather tiles (gemm_lds.hip) run these GEMMs: direct reads enabled,
@@ -131,6 +132,18 @@ struct AutotuneOffScope
 {
     AutotuneOffScope();
     ~AutotuneOffScope();
+
+  private:
+    bool was_;
+};
+
+// While one of these lives on a thread, the autotuner measures nothing for
+// plans built there; results that it has already apply, and their key is
+// left in PanelTables::tune_key.
+struct AutotuneRecallScope
+{
+    AutotuneRecallScope();
+    ~AutotuneRecallScope();
 
   private:
     bool was_;

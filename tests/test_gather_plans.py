@@ -5,6 +5,9 @@ the products at these addresses are the contraction.  Inputs are small whole
 numbers, so the comparison is exact."""
 import ctypes as C
 import itertools
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -21,6 +24,8 @@ class Plan:
 
     def __init__(self, A, B, C_, dtype=F64, aligned=True, config=None):
         d = [_HostDesc(x[0], x[1], dtype) for x in (A, B, C_)]
+        for t in d:
+            t.d.data = C.c_void_p(16)  # (never read)
         args = [y for t, x in zip(d, (A, B, C_)) for y in (C.byref(t.d), x[2].encode("latin1"))]
         cap = 1 << 22
         out = np.zeros(cap, dtype=np.int64)
@@ -29,6 +34,7 @@ class Plan:
         assert n >= HEADER, (n, T.last_error())
         (self.tile, self.gather, self.pieces, self.slices, self.swap, self.bk, self.bm, self.bn, self.elem,
          self.family, nt, nu, npool, self.scaled) = (int(x) for x in out[:14])
+        self.key = int(out[23]) & ((1 << 64) - 1)
         self.groups = {g: int(x) for g, x in enumerate(out[14:23]) if x}
         if self.gather:
             at = HEADER
@@ -187,3 +193,41 @@ def test_forms_of_the_general_path(seed, monkeypatch):
             plan = _check(*form, dtype, aligned=bool(rng.integers(2)))
             ran += plan.gather and plan.tile == int(tile)
     assert ran == 8
+
+
+# Calls of one m, n, k whose operands have several k blocks (complex parts):
+# packed tensors, and views that reach past 4 GiB, which no gather tile can
+# address.
+_TUNED = """
+import sys
+sys.path.insert(0, {root!r})
+from tests.test_gather_plans import C128, F64, Plan
+small = [([32, 32], [1, 32], s) for s in ("ak", "kb", "ab")]
+far = [([32, 32], [1, 1 << 25], "ak"), *small[1:]]
+turned = [([32, 32], [32, 1], "ak"), *small[1:]]
+for x in (small, far, turned):
+    p = Plan(*x, dtype=C128)
+    print(p.tile, p.gather, p.key)
+"""
+
+
+def test_remembered_tile_only_where_it_applies(tmp_path):
+    """A gather tile from the tuning file is used where it can run, and not
+    for operands beyond its reach; operands of several blocks that differ in
+    their strides have lines of their own."""
+
+    def plans(lines):
+        path = tmp_path / "tune.txt"
+        path.write_text("".join(
+            '{"format": "tblis-tune-v3", "family": 0, "shapes": "%016x", "tile": %d, "packed": 0}\n' % x for x in lines))
+        root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+        out = subprocess.run([sys.executable, "-c", _TUNED.format(root=root)], capture_output=True, text=True,
+                             env=dict(os.environ, TBLIS_HIP_AUTOTUNE="1", TBLIS_HIP_TUNE_FILE=str(path)))
+        assert out.returncode == 0, out.stderr
+        return [[int(x) for x in line.split()] for line in out.stdout.splitlines()]
+
+    keys = [key for _, _, key in plans([])]
+    assert len(set(keys)) == 3
+    small, far, turned = plans([(keys[0], 9), (keys[1], 9), (keys[2], 3)])
+    assert small[:2] == [9, 1] and turned[:2] == [3, 0]
+    assert not far[1]
