@@ -2006,6 +2006,8 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
     // time candidates as they will run when the tensors can be read
     const TuneOperands ops = t_tune_ops;
     const bool real = tune_real(family);
+    // without the tensors a gather tile cannot be timed: the model's stays
+    if (!real && panel_tile_lds(family, model_tile)) return -1;
     const void* opA = swap ? ops.B : ops.A;
     const void* opB = swap ? ops.A : ops.B;
     const uint64_t h = tune_key(gemms, family, real);

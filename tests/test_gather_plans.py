@@ -22,12 +22,14 @@ F64, F32, C64, C128 = T.TYPE_DOUBLE, T.TYPE_SINGLE, T.TYPE_SCOMPLEX, T.TYPE_DCOM
 class Plan:
     """A plan of C = A B over tensors given as (lengths, strides, labels)."""
 
-    def __init__(self, A, B, C_, dtype=F64, aligned=True, config=None):
+    CAP = 1 << 22
+
+    def __init__(self, A, B, C_, dtype=F64, aligned=True, config=None, data=16):
         d = [_HostDesc(x[0], x[1], dtype) for x in (A, B, C_)]
         for t in d:
-            t.d.data = C.c_void_p(16)  # (never read)
+            t.d.data = C.c_void_p(data)  # (never read)
         args = [y for t, x in zip(d, (A, B, C_)) for y in (C.byref(t.d), x[2].encode("latin1"))]
-        cap = 1 << 22
+        cap = self.CAP
         out = np.zeros(cap, dtype=np.int64)
         n = T.lib().tblis_hip_debug_plan(T.get_config(config) if config else None, *args, int(aligned),
                                          out.ctypes.data_as(C.POINTER(C.c_int64)), cap)
@@ -195,13 +197,24 @@ def test_forms_of_the_general_path(seed, monkeypatch):
     assert ran == 8
 
 
+def _plans_with(path, lines, program):
+    """What `program` prints, in a process whose tuning file has these
+    (key, family, tile) lines."""
+    path.write_text("".join('{"format": "tblis-tune-v3", "family": %d, "shapes": "%016x", "tile": %d, "packed": 0}\n'
+                            % (family, key, tile) for key, family, tile in lines))
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", "import sys; sys.path.insert(0, %r)\n" % root + program],
+                         capture_output=True, text=True,
+                         env=dict(os.environ, TBLIS_HIP_AUTOTUNE="1", TBLIS_HIP_TUNE_FILE=str(path)))
+    assert out.returncode == 0, out.stderr
+    return [[int(x) for x in line.split()] for line in out.stdout.splitlines()]
+
+
 # Calls of one m, n, k whose operands have several k blocks (complex parts):
 # packed tensors, and views that reach past 4 GiB, which no gather tile can
 # address.
 _TUNED = """
-import sys
-sys.path.insert(0, {root!r})
-from tests.test_gather_plans import C128, F64, Plan
+from tests.test_gather_plans import C128, Plan
 small = [([32, 32], [1, 32], s) for s in ("ak", "kb", "ab")]
 far = [([32, 32], [1, 1 << 25], "ak"), *small[1:]]
 turned = [([32, 32], [32, 1], "ak"), *small[1:]]
@@ -216,18 +229,28 @@ def test_remembered_tile_only_where_it_applies(tmp_path):
     for operands beyond its reach; operands of several blocks that differ in
     their strides have lines of their own."""
 
-    def plans(lines):
-        path = tmp_path / "tune.txt"
-        path.write_text("".join(
-            '{"format": "tblis-tune-v3", "family": 0, "shapes": "%016x", "tile": %d, "packed": 0}\n' % x for x in lines))
-        root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-        out = subprocess.run([sys.executable, "-c", _TUNED.format(root=root)], capture_output=True, text=True,
-                             env=dict(os.environ, TBLIS_HIP_AUTOTUNE="1", TBLIS_HIP_TUNE_FILE=str(path)))
-        assert out.returncode == 0, out.stderr
-        return [[int(x) for x in line.split()] for line in out.stdout.splitlines()]
-
-    keys = [key for _, _, key in plans([])]
+    path = tmp_path / "tune.txt"
+    keys = [key for _, _, key in _plans_with(path, [], _TUNED)]
     assert len(set(keys)) == 3
-    small, far, turned = plans([(keys[0], 9), (keys[1], 9), (keys[2], 3)])
+    small, far, turned = _plans_with(path, [(k, 0, tile) for k, tile in zip(keys, (9, 9, 3))], _TUNED)
     assert small[:2] == [9, 1] and turned[:2] == [3, 0]
     assert not far[1]
+
+
+_WITHOUT_TENSORS = """
+from tests.test_gather_plans import F32, Plan
+p = Plan(*[([200, 200], [1, 200], s) for s in ("ak", "kb", "ab")], dtype=F32, data={data})
+print(p.tile, p.gather, p.key)
+"""
+
+
+@pytest.mark.parametrize("data", [16, None])
+def test_remembered_panel_tile_against_a_gather_tile(data, tmp_path):
+    """Plans made without the tensors (indexed contractions) time panel tiles
+    only, whose best one does not replace the model's gather tile; with the
+    tensors it was timed against it and does."""
+    path = tmp_path / "tune.txt"
+    program = _WITHOUT_TENSORS.format(data=data)
+    [[tile, gather, key]] = _plans_with(path, [], program)
+    assert gather
+    assert _plans_with(path, [(key, 1, 3)], program) == [[3, 0, key] if data else [tile, gather, key]]

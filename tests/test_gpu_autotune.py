@@ -104,3 +104,25 @@ def test_last_direct_names_the_callers_operands():
         torch.cuda.synchronize()
         assert torch.allclose(C.cpu(), want, rtol=1e-13, atol=1e-13)
         assert T.last_direct() == 2, (C.stride(), T.last_direct())
+
+
+def test_gather_tile_kept_without_tensors():
+    """Indexed plans are tuned without their tensors, on panel tiles only: a
+    gather tile that the model picks stays, and the result is the same."""
+    g = torch.Generator(device="cuda").manual_seed(34000)
+    d = [torch.rand(5, 200, 40, device="cuda", generator=g) - 0.5 for _ in range(2)]
+    A, B = (T.Indexed([y for y in x], [(i,) for i in range(5)], [5]) for x in d)
+    got = []
+    for on in (False, True):
+        T.lib().tblis_hip_clear_plan_cache()
+        T.set_autotune(on)
+        try:
+            c = torch.zeros(200, 200, device="cuda")
+            T.indexed_mult(1.0, A, "aef", B, "bef", 0.0, T.Indexed([c], [()], []), "ab")
+            torch.cuda.synchronize()
+        finally:
+            T.set_autotune(False)
+            T.lib().tblis_hip_clear_plan_cache()
+        assert T.last_tile() in (6, 7)  # the split-BF16 gather tiles
+        got.append(c)
+    assert torch.equal(*got)
