@@ -333,6 +333,9 @@ int64_t debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_t
         if (!plan_panel_tables(std::move(gemms), T, family, dtype_code(rtype))) return 0;
     }
     const bool gather = panel_tile_lds(family, T.tile);
+    const int64_t size =
+        TBLIS_HIP_PLAN_HEADER + (gather ? (int64_t)(16 * T.tasks.size() + 8 * T.ujobs.size() + T.pool.size()) : 0);
+    if (size > max_out) return -2;
     std::vector<int64_t> v = {T.tile,
                               gather,
                               T.pieces,
@@ -364,9 +367,8 @@ int64_t debug_plan(const tblis_config* cfg, const tblis_tensor* A, const label_t
             v.insert(v.end(), {u.dst, u.rowmap, u.colmap, u.panel, u.nr, u.nc, u.nslice, u.sstride});
         v.insert(v.end(), T.pool.begin(), T.pool.end());
     }
-    if ((int64_t)v.size() > max_out) return -2;
     std::copy(v.begin(), v.end(), out);
-    return (int64_t)v.size();
+    return size;
 }
 
 // The same contraction with its plan tables and workspace in the device

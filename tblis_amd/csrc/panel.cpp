@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -54,44 +55,65 @@ bool unit_first(const Side& s) { return first_step(s) == 1; }
 
 int64_t side_len(const Side& s) { return side_count(s); }
 
+// Lowest and highest element offset of a side.
+void side_range(const Side& s, int64_t& lo, int64_t& hi)
+{
+    lo = hi = 0;
+    if (!s.offs.empty())
+    {
+        lo = *std::min_element(s.offs.begin(), s.offs.end());
+        hi = *std::max_element(s.offs.begin(), s.offs.end());
+        return;
+    }
+    for (size_t d = 0; d < s.len.size(); d++)
+    {
+        if (s.len[d] == 0) return;
+        const int64_t span = (s.len[d] - 1) * s.stride[d];
+        (span < 0 ? lo : hi) += span;
+    }
+}
+
+// Offsets of a side in odometer order (first dimension fastest), from base
+// on, times unit.
+void append_offsets(const Side& s, int64_t base, int64_t unit, std::vector<int64_t>& out)
+{
+    const size_t at = out.size();
+    if (!s.offs.empty())
+    {
+        out.resize(at + s.offs.size());
+        for (size_t i = 0; i < s.offs.size(); i++) out[at + i] = (base + s.offs[i]) * unit;
+        return;
+    }
+    const int64_t n = side_len(s);
+    if (n <= 0) return;
+    out.resize(at + (size_t)n);
+    int64_t* o = out.data() + at;
+    o[0] = base * unit;
+    int64_t done = 1;
+    for (size_t d = 0; d < s.len.size(); d++)
+    {
+        const int64_t step = s.stride[d] * unit;
+        for (int64_t i = 1; i < s.len[d]; i++)
+            for (int64_t j = 0; j < done; j++) o[i * done + j] = o[j] + i * step;
+        done *= s.len[d];
+    }
+}
+
 // Offset vectors, deduplicated by (lengths, strides).
 class Pool
 {
   public:
     int64_t offsets(const Side& s)
     {
-        if (!s.offs.empty())
-        {
-            std::vector<int64_t> key(s.offs);
-            key.push_back(-1);  // explicit lists never collide with (len, stride) keys
-            auto it = index_.find(key);
-            if (it != index_.end()) return it->second;
-            const int64_t at = push(s.offs);
-            index_[key] = at;
-            return at;
-        }
+        if (!s.offs.empty()) return list(s.offs);
         std::vector<int64_t> key(s.len);
         key.insert(key.end(), s.stride.begin(), s.stride.end());
         key.push_back((int64_t)s.len.size());
         auto it = index_.find(key);
         if (it != index_.end()) return it->second;
         const int64_t at = (int64_t)data_.size();
-        const int64_t n = side_len(s);
-        data_.resize(data_.size() + std::max<int64_t>(n, 1));
-        // odometer, first dimension fastest
-        std::vector<int64_t> idx(s.len.size(), 0);
-        int64_t off = 0;
-        for (int64_t i = 0; i < n; i++)
-        {
-            data_[at + i] = off;
-            for (size_t d = 0; d < s.len.size(); d++)
-            {
-                off += s.stride[d];
-                if (++idx[d] < s.len[d]) break;
-                off -= s.stride[d] * s.len[d];
-                idx[d] = 0;
-            }
-        }
+        append_offsets(s, 0, 1, data_);
+        if ((int64_t)data_.size() == at) data_.push_back(0);
         index_[key] = at;
         return at;
     }
@@ -118,15 +140,21 @@ class Pool
         }
         return at;
     }
-    // explicit values at an even index, deduplicated
-    int64_t aligned(const std::vector<int64_t>& v)
+    // explicit values, deduplicated; even: at an even index
+    int64_t list(const std::vector<int64_t>& v, bool even = false)
     {
-        std::vector<int64_t> key(v);
-        key.push_back(-2);
-        auto it = index_.find(key);
-        if (it != index_.end()) return it->second;
-        if (data_.size() % 2) data_.push_back(0);
-        return index_[key] = push(v);
+        uint64_t h = 1469598103934665603ULL;
+        for (int64_t x : v) h = (h ^ (uint64_t)x) * 1099511628211ULL;
+        const auto same = lists_.equal_range(h);
+        for (auto it = same.first; it != same.second; ++it)
+        {
+            const auto [at, n] = it->second;
+            if (n == v.size() && !(even && at % 2) && std::equal(v.begin(), v.end(), data_.begin() + at)) return at;
+        }
+        if (even && data_.size() % 2) data_.push_back(0);
+        const int64_t at = push(v);
+        lists_.emplace(h, std::make_pair(at, v.size()));
+        return at;
     }
     // append raw values; returns their pool index
     int64_t push(const std::vector<int64_t>& v)
@@ -136,11 +164,13 @@ class Pool
         if (v.empty()) data_.push_back(0);
         return at;
     }
+    void reserve(size_t n) { data_.reserve(n); }
     std::vector<int64_t>& data() { return data_; }
 
   private:
     std::vector<int64_t> data_;
-    std::map<std::vector<int64_t>, int64_t> index_;
+    std::map<std::vector<int64_t>, int64_t> index_;  // (lengths, strides) sides
+    std::unordered_multimap<uint64_t, std::pair<int64_t, size_t>> lists_;  // by hash: index, length
 };
 
 // Fragment-group geometry of a family's panels.
@@ -416,22 +446,13 @@ double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, in
 // and read once.
 double reduce_us(double panel_bytes) { return 4.5 + 2.0 * panel_bytes / 4.2e6; }
 
-// Share of neighbouring offsets that are one element apart.
-double unit_share(const std::vector<int64_t>& off)
+// Share of neighbouring offsets that are one element (step) apart.
+double unit_share(const std::vector<int64_t>& off, int64_t step)
 {
     int64_t c = 0;
     const int64_t n = (int64_t)off.size();
-    for (int64_t i = 0; i + 1 < n; i++) c += off[i + 1] - off[i] == 1;
+    for (int64_t i = 0; i + 1 < n; i++) c += off[i + 1] - off[i] == step;
     return n > 1 ? (double)c / (double)(n - 1) : 0.0;
-}
-
-// Offsets of a side in odometer order.
-std::vector<int64_t> side_offsets(const Side& s)
-{
-    if (!s.offs.empty()) return s.offs;
-    Pool p;
-    const int64_t at = p.offsets(s);
-    return std::vector<int64_t>(p.data().begin() + at, p.data().begin() + at + side_len(s));
 }
 
 // Can an FP64 operand be read in 16-byte pieces (gemm_pieces_kernel)?  rows
@@ -449,11 +470,16 @@ bool vec_layout(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks
     if (lanes_k)
         for (int64_t r : rows)
             if (r % 16) return false;
-    for (size_t i = 0; i < ks.size(); i++)
+    for (size_t first = 0; first < ks.size(); first += (size_t)bk)
     {
-        const int64_t at = ks[i] - ks[i - i % bk];
-        if (at < 0 || at != (lanes_k ? 8 * (int64_t)(i % bk) : ks[i % bk] - ks[0])) return false;
-        if ((!lanes_k || i % bk == 0) && ks[i] % 16) return false;
+        if (ks[first] % 16) return false;
+        const size_t n = std::min<size_t>((size_t)bk, ks.size() - first);
+        for (size_t j = 1; j < n; j++)
+        {
+            const int64_t at = ks[first + j] - ks[first];
+            if (at < 0 || at != (lanes_k ? 8 * (int64_t)j : ks[j] - ks[0])) return false;
+            if (!lanes_k && at % 16) return false;
+        }
     }
     return true;
 }
@@ -483,37 +509,19 @@ struct GatherOperand
 GatherOperand gather_operand(const std::vector<PBlock>& bl, int src_elem)
 {
     GatherOperand o;
-    o.rows = side_offsets(bl[0].rows);
+    int64_t lo, hi, klo = INT64_MAX;
     for (const PBlock& b : bl)
-        for (int64_t x : side_offsets(b.k)) o.ks.push_back(b.base - bl[0].base + x);
-    o.lanes_k = unit_share(o.ks) > unit_share(o.rows);
-    o.src = bl[0].base;
-    for (std::vector<int64_t>* v : {&o.rows, &o.ks})
     {
-        const int64_t lo = *std::min_element(v->begin(), v->end());
-        o.src += lo;
-        for (int64_t& x : *v) x = (x - lo) * src_elem;
+        if (side_len(b.k) == 0) continue;
+        side_range(b.k, lo, hi);
+        klo = std::min(klo, b.base - bl[0].base + lo);
     }
+    side_range(bl[0].rows, lo, hi);
+    append_offsets(bl[0].rows, -lo, src_elem, o.rows);
+    for (const PBlock& b : bl) append_offsets(b.k, b.base - bl[0].base - klo, src_elem, o.ks);
+    o.lanes_k = unit_share(o.ks, src_elem) > unit_share(o.rows, src_elem);
+    o.src = bl[0].base + lo + klo;
     return o;
-}
-
-// Do the gather kernels with stages of bk k read every operand of these
-// GEMMs in 16-byte pieces?
-bool pieces_apply(const std::vector<PanelGemm>& gemms, int src_elem, int64_t bk)
-{
-    if (!t_aligned || src_elem != 8) return false;
-    for (const PanelGemm& g : gemms)
-    {
-        for (double x : g.kscale)
-            if (x != 1.0) return false;
-        if (total_k(g) == 0) continue;
-        for (const std::vector<PBlock>* bl : {&g.a, &g.b})
-        {
-            const GatherOperand o = gather_operand(*bl, src_elem);
-            if (!vec_layout(o.rows, o.ks, o.src, o.lanes_k, bk)) return false;
-        }
-    }
-    return true;
 }
 
 // 128-byte lines that an operand's loads touch, over those its elements
@@ -590,6 +598,51 @@ struct GatherChoice
     bool pieces = false;
 };
 
+// What the gather tiles' plan and its models read of a plan's GEMMs, made
+// once: the GEMMs in the order in which the kernels walk them and, for those
+// with k, both operands' offsets.
+struct GatherWork
+{
+    GatherWork(const std::vector<PanelGemm>& planned, int family, int src_elem)
+        : gemms(coalesced(planned)), family(family), src_elem(src_elem), ops(2 * gemms.size())
+    {
+        const PanelGemm* big = &gemms[0];
+        for (const PanelGemm& g : gemms)
+            if (g.mlen[0] * g.nlen[0] > big->mlen[0] * big->nlen[0] && total_k(g) > 0) big = &g;
+        for (size_t i = 0; i < gemms.size(); i++)
+        {
+            const PanelGemm& g = gemms[i];
+            for (double x : g.kscale) scaled = scaled || x != 1.0;
+            if (total_k(g) == 0) continue;
+            ops[2 * i] = gather_operand(g.a, src_elem);
+            ops[2 * i + 1] = gather_operand(g.b, src_elem);
+            if (family == FAMILY_F64 || &g != big) continue;
+            for (int o = 0; o < 2; o++) share = std::max(share, std::min(2.0, line_share(ops[2 * i + o], src_elem)));
+        }
+    }
+    // Do kernels with stages of bk k read every operand in 16-byte pieces?
+    bool pieces(int64_t bk)
+    {
+        for (const auto& x : pieces_)
+            if (x.first == bk) return x.second;
+        bool ok = t_aligned && src_elem == 8 && !scaled;
+        for (size_t i = 0; i < ops.size() && ok; i++)
+            ok = ops[i].ks.empty() || vec_layout(ops[i].rows, ops[i].ks, ops[i].src, ops[i].lanes_k, bk);
+        pieces_.push_back({bk, ok});
+        return ok;
+    }
+
+    std::vector<PanelGemm> gemms;
+    int family, src_elem;
+    std::vector<GatherOperand> ops;  // A and B of each GEMM
+    bool scaled = false;             // some k block is scaled
+    double share = 1.0;              // split-BF16: line_share of the largest GEMM's worse operand
+    GatherChoice best;               // of all tiles (plan_panel_tables)
+
+  private:
+    std::vector<std::pair<int64_t, bool>> pieces_;  // by stage length
+};
+
 // Best gather tile (gemm_lds.hip, gemm_gather_bf16.hip; only: that one) and
 // number of k slices for these GEMMs, from a model of a CU that holds up to
 // occ workgroups.  A workgroup's stage takes `stage` cycles of the CU, a
@@ -604,8 +657,10 @@ struct GatherChoice
 // where short runs make it fetch lines that it uses a part of (line_share: runs
 // of 29 and 31 floats, 2.0, took the 64 x 64 tile 1.7-2.1 times the cycles and
 // the 128 x 128 one 1.5-1.8; runs of 49 and 51, 1.6, the latter 1.07-1.17).
-GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int src_elem, int cus, int only = -1)
+GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
 {
+    const std::vector<PanelGemm>& gemms = w.gemms;
+    const int family = w.family, src_elem = w.src_elem;
     struct Model
     {
         int family, lt;
@@ -621,21 +676,10 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
                                 {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000},
                                 {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000}};
     const bool f64 = family == FAMILY_F64;
-    double share = 1.0;  // of the worse operand of the largest GEMM
-    if (!f64)
-    {
-        const PanelGemm* big = &gemms[0];
-        for (const PanelGemm& g : gemms)
-            if (g.mlen[0] * g.nlen[0] > big->mlen[0] * big->nlen[0] && total_k(g) > 0) big = &g;
-        if (total_k(*big) > 0)
-            for (const std::vector<PBlock>* bl : {&big->a, &big->b})
-                share = std::max(share, std::min(2.0, line_share(gather_operand(*bl, src_elem), src_elem)));
-    }
+    const double share = w.share;
     constexpr double kGHz = 2.15;
     GatherChoice best;
     const int first = panel_num_tiles(family) - (f64 ? lds_num_tiles() : gather_bf16_num_tiles());
-    int known = -1;
-    bool pieces = false;
     for (const Model& md : models)
     {
         if (md.family != family) continue;
@@ -643,7 +687,7 @@ GatherChoice gather_choice(const std::vector<PanelGemm>& gemms, int family, int 
         if (only >= 0 ? tile != only : f64 && md.lt == 0) continue;
         const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
         const int64_t bk = panel_tile_k(family, tile);
-        if (known != (int)bk) pieces = pieces_apply(gemms, src_elem, bk), known = (int)bk;
+        const bool pieces = f64 && w.pieces(bk);
         if (f64 && md.pieces != pieces && md.lt != 0) continue;
         const double over = std::max(0.0, share - 1.3);
         const double lines = f64 ? 1.0 : md.lt == 0 ? 1.0 + 1.6 * over * over : std::max(1.0, 0.9 * share);
@@ -912,19 +956,19 @@ namespace
 bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T,
                      const bool allow_direct[2], int src_elem);
 int ksplit_forced();
-bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
-                   int64_t kslice);
+bool gather_tables(GatherWork& w, int tile, PanelTables& T, int64_t kslice);
 // tables_for_tile with the tasks grouped by which operands they read
 // directly (one kernel variant per launch); packed: every operand packed
-bool tables_uniform(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
-                    bool packed = false);
+// (gather tiles: from work)
+bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int tile, PanelTables& T,
+                    int src_elem, bool packed = false);
 // Autotuner candidates: a tile, or with kPackedBit the same tile with every
 // operand packed (timed next to the planner's direct reads)
 constexpr int kPackedBit = 256;
 // model_tile: the cost model's pick, preferred among finalists that tie.
 // Returns the measured choice (a tile, + kPackedBit for its every-operand-
 // packed variant) or -1.
-int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bool swap,
+int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int dtype, bool swap,
                   const std::vector<int>& cands, int model_tile);
 uint64_t tune_key(const std::vector<PanelGemm>& gemms, int family, bool real);
 // Do the tuner's candidates run on the tensors?
@@ -991,13 +1035,15 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     size_t sbytes = 0;
     static_storage(sbase, sbytes);
     const bool rounds = (family == FAMILY_F64 || family == FAMILY_BF16X3) && !sbase;
+    const int src_elem = dtype == 0 ? 8 : 4;
+    const bool gathers = (family == FAMILY_F64 || family == FAMILY_BF16X3) && lds_applicable(gemms, family, src_elem);
     std::vector<int> cands;
     for (int mi = 0; mi < nmodels; mi++)
     {
         const TileModel& tm = models[mi];
         if (tm.tile >= panel_num_tiles(family)) continue;
         if (family == FAMILY_BF16X3 && !panel_tile_lds(family, tm.tile) && panel_bf16_tile_fast_only(tm.tile)) continue;
-        if (panel_tile_lds(family, tm.tile) && !lds_applicable(gemms, family, dtype == 0 ? 8 : 4)) continue;
+        if (panel_tile_lds(family, tm.tile) && !gathers) continue;
         cands.push_back(tm.tile);
         if (panel_tile_lds(family, tm.tile)) continue;  // gather tiles have a model of their own
         if (rounds) continue;
@@ -1025,14 +1071,15 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         }
     }
     // Gather tiles: by their own model, against the best register-fed tile.
-    if (rounds && lds_applicable(gemms, family, dtype == 0 ? 8 : 4))
+    std::unique_ptr<GatherWork> work;
+    if (rounds && gathers)
     {
-        const std::vector<PanelGemm> walk = coalesced(gemms);
-        const GatherChoice c = gather_choice(walk, family, dtype == 0 ? 8 : 4, cus);
-        if (gather_preferred(walk, family, c, best)) tile = c.tile;
+        work.reset(new GatherWork(gemms, family, src_elem));
+        work->best = gather_choice(*work, cus);
+        if (gather_preferred(work->gemms, family, work->best, best)) tile = work->best.tile;
     }
     bool packed = false;
-    const int tuned = autotune_tile(gemms, family, dtype, swap, cands, tile);
+    const int tuned = autotune_tile(gemms, work.get(), family, dtype, swap, cands, tile);
     if (tuned >= 0)
     {
         tile = tuned % kPackedBit;
@@ -1043,13 +1090,14 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         int t = std::atoi(e);
         if (e[0] >= '0' && e[0] <= '9' && t < panel_num_tiles(family) &&
             !(family == FAMILY_BF16X3 && !panel_tile_lds(family, t) && panel_bf16_tile_fast_only(t)) &&
-            !(panel_tile_lds(family, t) && !lds_applicable(gemms, family, dtype == 0 ? 8 : 4)))
+            !(panel_tile_lds(family, t) && !gathers))
         {
             tile = t;
             packed = false;
         }
     }
-    if (!tables_uniform(gemms, family, tile, T, dtype == 0 ? 8 : 4, packed)) return false;
+    if (panel_tile_lds(family, tile) && !work) work.reset(new GatherWork(gemms, family, src_elem));
+    if (!tables_uniform(gemms, work.get(), family, tile, T, src_elem, packed)) return false;
     T.swap = swap;
     if (t_tune_recall) T.tune_key = tune_key(gemms, family, tune_real(family));
     return true;
@@ -1061,20 +1109,19 @@ namespace
 // Tasks grouped by which operands they read straight from the tensors
 // (GEMMs of one batch may differ): the groups become separate launches of
 // the matching kernel variant.
-bool tables_uniform(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
-                    bool packed)
+bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int tile, PanelTables& T,
+                    int src_elem, bool packed)
 {
     const bool allow[2] = {!packed, !packed};
     T = PanelTables();
     if (panel_tile_lds(family, tile))
     {
-        const std::vector<PanelGemm> walk = coalesced(gemms);
         int64_t kmax = 1;
-        for (const PanelGemm& g : walk) kmax = std::max(kmax, total_k(g));
+        for (const PanelGemm& g : gemms) kmax = std::max(kmax, total_k(g));
         const int64_t bk = panel_tile_k(family, tile);
         int64_t S = ksplit_forced();
-        if (!S) S = gather_choice(walk, family, src_elem, device_cu_count(), tile).slices;
-        return gather_tables(walk, family, tile, T, src_elem, ceil_div(ceil_div(kmax, S), bk) * bk);
+        if (!S) S = (work->best.tile == tile ? work->best : gather_choice(*work, device_cu_count(), tile)).slices;
+        return gather_tables(*work, tile, T, ceil_div(ceil_div(kmax, S), bk) * bk);
     }
     if (!tables_for_tile(gemms, family, tile, T, allow, src_elem)) return false;
     auto group = [](const PanelTask& t) {
@@ -1099,24 +1146,6 @@ bool tables_uniform(const std::vector<PanelGemm>& gemms, int family, int tile, P
     for (int o = 0; o < 2; o++)
         T.direct[o] = T.group_n[o == 0 ? 1 : 2] + T.group_n[3] == (int64_t)T.tasks.size() && !T.tasks.empty();
     return true;
-}
-
-// Lowest and highest element offset of a side.
-void side_range(const Side& s, int64_t& lo, int64_t& hi)
-{
-    lo = hi = 0;
-    if (!s.offs.empty())
-    {
-        lo = *std::min_element(s.offs.begin(), s.offs.end());
-        hi = *std::max_element(s.offs.begin(), s.offs.end());
-        return;
-    }
-    for (size_t d = 0; d < s.len.size(); d++)
-    {
-        if (s.len[d] == 0) return;
-        const int64_t span = (s.len[d] - 1) * s.stride[d];
-        (span < 0 ? lo : hi) += span;
-    }
 }
 
 bool same_side(const Side& a, const Side& b) { return a.len == b.len && a.stride == b.stride && a.offs == b.offs; }
@@ -1219,24 +1248,35 @@ int ksplit_forced()
 
 // Tables of a plan on a gather tile (gemm_lds.hip): tasks and, for GEMMs cut
 // along k, the jobs that add their C panels up.  kslice: k per task.
-bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T, int src_elem,
-                   int64_t kslice)
+bool gather_tables(GatherWork& w, int tile, PanelTables& T, int64_t kslice)
 {
-    const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile);
+    const int family = w.family;
+    const bool f64 = family == FAMILY_F64;
+    const int64_t BM = panel_tile_m(family, tile), BN = panel_tile_n(family, tile), bk = panel_tile_k(family, tile);
     Pool pool;
     std::vector<int64_t> cost, region;
     std::vector<int> group;
     std::vector<PanelTask> all;
     int64_t nregions = 0, wsc = 0;
-    T.pieces = src_elem == 8 && t_aligned;
-    for (const PanelGemm& g : gemms)
-        for (double x : g.kscale) T.scaled |= x != 1.0;
-    for (const PanelGemm& g : gemms)
+    T.pieces = f64 && w.pieces(bk);
+    T.scaled = w.scaled;
+    size_t npool = 0, ntask = 0;
+    for (const PanelGemm& g : w.gemms)
     {
-        const int64_t m = g.mlen[0], n = g.nlen[0];
-        int64_t k = 0;
-        for (auto x : g.klen) k += x;
-        if (m == 0 || n == 0) continue;
+        const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g);
+        npool += (size_t)(2 * (m + n) + (f64 ? 2 : 1) * (k + 4 * bk) + (w.scaled ? k + 4 * bk : 0) + 4);
+        ntask += (size_t)(ceil_div(m, BM) * ceil_div(n, BN) * std::max<int64_t>(1, ceil_div(k, kslice)));
+    }
+    pool.reserve(npool);
+    all.reserve(ntask);
+    cost.reserve(ntask);
+    region.reserve(ntask);
+    group.reserve(ntask);
+    std::vector<int64_t> ks;
+    for (size_t gi = 0; gi < w.gemms.size(); gi++)
+    {
+        const PanelGemm& g = w.gemms[gi];
+        const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g);
         const int64_t MT = ceil_div(m, BM), NT = ceil_div(n, BN), mp = MT * BM, np = NT * BN;
         if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX / 2) fail("contraction too large for one GEMM");
         T.useful_flops += 2 * m * n * k;
@@ -1246,32 +1286,30 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
         int kl = 0;
         if (k > 0)
         {
-            const std::vector<PBlock>* blocks[2] = {&g.a, &g.b};
             for (int o = 0; o < 2; o++)
             {
-                GatherOperand x = gather_operand(*blocks[o], src_elem);
-                T.pieces = T.pieces && vec_layout(x.rows, x.ks, x.src, x.lanes_k, panel_tile_k(family, tile));
-                const bool f64 = family == FAMILY_F64;
+                const GatherOperand& x = w.ops[2 * gi + o];
                 const int mode = !x.lanes_k ? 0 : !f64 && t_aligned && octet_layout(x.rows, x.ks, x.src) ? 2 : 1;
                 kl += mode * (o == 0 ? 1 : f64 ? 2 : 3);
                 // the kernels read offsets up to four stages past a task's
                 // end (whole octets of split-BF16's 16-byte loads)
                 const int64_t rep = std::min<int64_t>(k, 8);
-                for (int64_t i = 0; i < 4 * panel_tile_k(family, tile); i++)
-                    x.ks.push_back(x.ks[k - rep + (k + i) % rep]);
+                ks = x.ks;
+                for (int64_t i = 0; i < 4 * bk; i++) ks.push_back(x.ks[k - rep + (k + i) % rep]);
                 if (!f64)
                 {
                     // 32-bit words, two to a pool entry, on 16 bytes
-                    std::vector<int64_t> w((x.ks.size() + 1) / 2, 0);
-                    for (size_t i = 0; i < x.ks.size(); i++) w[i / 2] |= (int64_t)((uint64_t)x.ks[i] << (32 * (i % 2)));
-                    x.ks.swap(w);
+                    const size_t nk = ks.size();
+                    for (size_t i = 0; i < nk; i++)
+                    {
+                        const int64_t word = (int64_t)((uint64_t)ks[i] << (32 * (i % 2)));
+                        ks[i / 2] = i % 2 ? ks[i / 2] | word : word;
+                    }
+                    ks.resize((nk + 1) / 2);
                 }
-                Side rows, ks;
-                rows.offs.swap(x.rows);
-                ks.offs.swap(x.ks);
                 src[o] = x.src;
-                km[o] = f64 ? pool.offsets(ks) : pool.aligned(ks.offs);
-                rt[o] = pool.offsets(rows);
+                km[o] = pool.list(ks, !f64);
+                rt[o] = pool.list(x.rows);
             }
             if (T.scaled)
             {
@@ -1283,7 +1321,7 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
                     std::memcpy(&bits, &x, sizeof bits);
                     sc.insert(sc.end(), (size_t)g.klen[q], bits);
                 }
-                sc.insert(sc.end(), (size_t)(4 * panel_tile_k(family, tile)), 0);
+                sc.insert(sc.end(), (size_t)(4 * bk), 0);
                 scales = pool.push(sc);
             }
         }
@@ -1306,7 +1344,7 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
             T.ujobs.push_back(u);
             T.slices = std::max<int>(T.slices, (int)S);
         }
-        const TileWalk W(MT, NT, mp, np, gemms.size());
+        const TileWalk W(MT, NT, mp, np, w.gemms.size());
         for (int64_t s = 0; s < S; s++)
         {
             for (int64_t pid = 0; pid < MT * NT; pid++)
@@ -1354,10 +1392,13 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
     if (all.size() > (size_t)INT32_MAX || T.uchunks.size() > (size_t)INT32_MAX)
         fail("contraction too large: panel task list exceeds 2^31 entries");
     // one launch per combination of lanes along rows and along k
+    const bool one = std::count(group.begin(), group.end(), group[0]) == (int64_t)group.size();
     for (int q = 0; q < kTaskGroups; q++)
     {
+        if (one && q != group[0]) continue;
         std::vector<PanelTask> ts;
         std::vector<int64_t> tc, tr;
+        if (one) ts.swap(all), tc.swap(cost), tr.swap(region);
         for (size_t i = 0; i < all.size(); i++)
             if (group[i] == q)
             {
@@ -1367,8 +1408,11 @@ bool gather_tables(const std::vector<PanelGemm>& gemms, int family, int tile, Pa
             }
         if (ts.empty()) continue;
         ts = xcd_order(ts, tc, tr, nregions);
-        T.tasks.insert(T.tasks.end(), ts.begin(), ts.end());
         T.group_n[q] = T.sched.group_n[0][q] = (int64_t)ts.size();
+        if (T.tasks.empty())
+            T.tasks = std::move(ts);
+        else
+            T.tasks.insert(T.tasks.end(), ts.begin(), ts.end());
     }
     T.task_stage.assign(T.tasks.size(), 0);
     T.direct[0] = T.direct[1] = true;
@@ -1998,7 +2042,7 @@ uint64_t tune_key(const std::vector<PanelGemm>& gemms, int family, bool real)
     return h;
 }
 
-int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bool swap,
+int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int dtype, bool swap,
                   const std::vector<int>& cands_in, int model_tile)
 {
     const std::vector<int>& cands0 = cands_in;
@@ -2048,12 +2092,12 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
     std::vector<PanelTables> tabs;
     for (int c : cands0)
     {
-        if (!real && panel_tile_lds(family, c)) continue;
+        if ((!real || !work) && panel_tile_lds(family, c)) continue;
         // with tensors: grouped as the plan will be; without: both operands
         // in panels
         const bool none[2] = {false, false};
         PanelTables T1;
-        if (real ? !tables_uniform(gemms, family, c, T1, dtype == 0 ? 8 : 4)
+        if (real ? !tables_uniform(gemms, work, family, c, T1, dtype == 0 ? 8 : 4)
                  : !tables_for_tile(gemms, family, c, T1, none, dtype == 0 ? 8 : 4))
             return -1;
         const bool reads = panel_tile_lds(family, c) || T1.group_n[1] + T1.group_n[2] + T1.group_n[3] > 0;
@@ -2062,7 +2106,7 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, int family, int dtype, bo
         if (real && reads && !t_direct_all && !panel_tile_lds(family, c))
         {
             PanelTables T2;
-            if (!tables_uniform(gemms, family, c, T2, dtype == 0 ? 8 : 4, true)) return -1;
+            if (!tables_uniform(gemms, work, family, c, T2, dtype == 0 ? 8 : 4, true)) return -1;
             if ((size_t)T2.ws_panel * eb <= free_bytes / 4)
             {
                 cands.push_back(c + kPackedBit);

@@ -8,6 +8,7 @@ import itertools
 import os
 import subprocess
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -254,3 +255,28 @@ def test_remembered_panel_tile_against_a_gather_tile(data, tmp_path):
     [[tile, gather, key]] = _plans_with(path, [], program)
     assert gather
     assert _plans_with(path, [(key, 1, 3)], program) == [[3, 0, key] if data else [tile, gather, key]]
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+def test_planning_time_of_long_sums(dtype, monkeypatch):
+    """Planning a gather tile makes each operand's tables once: 32 x 32 x
+    131072 takes as long as some passes over tables of its length (FP64 15 of
+    them; 60 when its models and its plan each made the tables anew)."""
+    ext = dict(a=32, b=32, k=131072)
+    form = [_tensor(ext, s) for s in ("ak", "kb", "ab")]
+    words = np.arange(2 * ext["k"])
+
+    def best(f):
+        t = []
+        for _ in range(9):
+            t0 = time.perf_counter()
+            f()
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    d = [_HostDesc(x[0], x[1], dtype) for x in form]
+    args = [y for t, x in zip(d, form) for y in (C.byref(t.d), x[2].encode("latin1"))]
+    out = (C.c_int64 * HEADER)()  # too small: the plan is made, not copied out
+    plan = best(lambda: T.lib().tblis_hip_debug_plan(None, *args, 1, out, HEADER))
+    one = best(lambda: (words[1:] - words[:-1]).sum() + words.copy()[0])
+    assert plan <= 30 * one, (plan, one)
