@@ -55,6 +55,16 @@ __device__ __forceinline__ uint32_t round_pair(float& a, float& b)
     return w;
 }
 
+// Orders this wave's LDS accesses before and after it, for lanes that read
+// what other lanes of the wave wrote.  A wave's LDS accesses are carried out
+// in order, so that only the compiler has to keep it: no instruction.
+__device__ __forceinline__ void wave_exchange()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int kNT = 256;  // threads per workgroup: one unit of A' and of B' per stage
 
 // One operand of a task.
@@ -145,10 +155,12 @@ struct UnitSide
             };
 #pragma unroll
             for (int j = 0; j < 8; j++) at(64 / BK * j + (int)threadIdx.x % 64 / BK)[kk] = f[j];
+            wave_exchange();  // the wave's lanes read one another's values
             const f32x4* p = (const f32x4*)(at(row - wrow) + 8 * oct);
             const f32x4 a = p[0], b = p[1];
 #pragma unroll
             for (int j = 0; j < 4; j++) f[j] = a[j], f[4 + j] = b[j];
+            wave_exchange();  // before the units overwrite them
         }
         u32x4 h, m, l;
 #pragma unroll
