@@ -299,59 +299,92 @@ int64_t total_k(const PanelGemm& g)
     return k;
 }
 
-// Best split-BF16 panel tile of GEMMs that are packed, and its us.  A 16-k
-// step of the 256 x 128 tile (one workgroup to a CU) takes 0.95 us a round
-// and more the more CUs draw power, of the 128 x 128 tile 0.86 us a round; the
-// 64 x 64 ones, cut along k over two or four waves, fill the chip evenly.
-// Model / measured: 2401^3 (190 tiles) 0 215 / 205, 2809^3 (242) 0 268 / 272,
-// 3025^3 (288) 0 484 / 458, 3969^3 (512) 0 732 / 748, 2304^3 2 280 / 281;
-// complex 30^4 4 104 / 98, 40^4 0 264 / 269.  Against the rates of kModelsBf16
-// (us, rate / this): complex 30^4 126 / 98, 40^4 397 / 269, permuted 45/21
-// 268 / 215; 2601^3 350 / 240.
+// 128-byte lines that neighbouring offsets (bytes) touch, over those that
+// their elements would fill: 1 for long runs, about 2 for runs of 29 floats,
+// 16 for pairs of floats far apart.
+double line_share(const std::vector<int64_t>& at, int elem)
+{
+    int64_t lines = 1;
+    for (size_t i = 1; i < at.size(); i++) lines += at[i] / 128 != at[i - 1] / 128;
+    return at.empty() ? 1.0 : std::max(1.0, (double)lines * 128.0 / ((double)at.size() * elem));
+}
+
+// Lines that the results of one row of C touch, as line_share.
+double result_share(const PanelGemm& g, int elem)
+{
+    std::vector<int64_t> at;
+    append_offsets(g.c[0].cols, 0, elem, at);
+    return line_share(at, elem);
+}
+
+// Best split-BF16 panel tile of GEMMs that are packed, and its us: the pack,
+// dearer for short runs (runs: a line_share per operand), the k steps, whole
+// rounds of tiles over the CUs with their first loads and results, and the
+// results' bytes, dearer where a row of C has short runs.  The constants are
+// fitted to 1789 contractions of 1e6 to 2.5e10 products with extents of 1 to
+// 64, in every order of their labels; median error 5% (0, 1) to 10%, 90th
+// percentile 18 to 30%.  Short k and scattered results are where the tiles
+// differ most: 28500 x 160 x 96 floats 0 46, 2 38, 3 33 us; 5220 x 5120 x 174
+// 0 153, 1 132, 3 102; 11264 x 24400 x 58 0 931, 1 768, 3 545.
 struct SplitTile
 {
     int tile;
     double us;
 };
-SplitTile split_tile(const std::vector<PanelGemm>& gemms, int cus)
+SplitTile split_tile(const std::vector<PanelGemm>& gemms, const double runs[2], int cus)
 {
     struct Step
     {
         int tile;
         int64_t bm, bn;
-        double round, share;  // us of 16 k: per round of tiles, and per CU's share of the tiles
-        double base;
+        double base, pack;           // us, and of the pack at its rate
+        double share, round, first;  // us of 16 k: of a CU's share of the tiles, of a round of tiles, of a GEMM
+        double tile_us, round_us;    // us of a CU's share of the tiles and of a round besides their k
+        double out, scatter;         // of the results at 4.9 TB/s, and for each further line they touch
     };
-    constexpr Step steps[] = {{0, 256, 128, 0.95, 0.33, 0.0}, {2, 128, 128, 0.86, 0.0, 0.0},
-                              {4, 64, 64, 0.0, 0.26, 0.30},   {5, 64, 64, 0.0, 0.28, 0.27}};
-    double packed = 9.0;
+    constexpr Step steps[] = {{0, 256, 128, 12.5, 1.4, 0.22, 0.75, 0.0, 0.7, 15.0, 1.2, 0.074},
+                              {1, 128, 256, 9.0, 1.5, 0.20, 0.79, 0.0, 2.6, 13.0, 0.55, 0.06},
+                              {2, 128, 128, 13.0, 1.4, 0.17, 0.56, 0.0, 2.3, 4.6, 0.4, 0.073},
+                              {3, 64, 64, 9.0, 1.2, 0.0, 0.29, 0.44, 0.16, 0.23, 0.7, 0.076},
+                              {4, 64, 64, 8.5, 1.55, 0.025, 0.22, 0.035, 0.0, 2.0, 0.0, 0.065},
+                              {5, 64, 64, 9.0, 1.65, 0.025, 0.225, 0.0, 0.5, 2.0, 0.5, 0.12}};
+    double packed = 0, slow = 0, results = 0;
     int64_t klo = -1, khi = 0;
+    const PanelGemm* big = &gemms[0];
+    auto rows = [](const std::vector<int64_t>& len) {
+        int64_t n = 0;
+        for (auto x : len) n += x;
+        return n;
+    };
     for (const PanelGemm& g : gemms)
     {
-        int64_t m = 0, n = 0;
-        for (auto x : g.mlen) m += x;
-        for (auto x : g.nlen) n += x;
-        const int64_t k = ceil_div(total_k(g), 16);
+        const int64_t m = rows(g.mlen), n = rows(g.nlen), k = ceil_div(total_k(g), 16);
         packed += 10.0 * (double)(m + n) * (double)total_k(g) / 3.83e6;
+        slow += 10.0 * ((double)m * (std::sqrt(runs[0]) - 1.0) + (double)n * (std::sqrt(runs[1]) - 1.0)) *
+                (double)total_k(g) / 3.83e6;
+        results += 4.0 * (double)m * (double)n;
         klo = klo < 0 ? k : std::min(klo, k);
         khi = std::max(khi, k);
+        if (m * n > rows(big->mlen) * rows(big->nlen)) big = &g;
     }
+    const double lines = std::min(32.0, result_share(*big, 4)) - 1.0;
     SplitTile best{-1, 0};
     for (const Step& st : steps)
     {
-        double share = 0;  // 16-k steps of a CU's share of the tiles
+        double share = 0, tiles = 0;  // 16-k steps, tiles of a CU's share
         for (const PanelGemm& g : gemms)
         {
-            int64_t m = 0, n = 0;
-            for (auto x : g.mlen) m += x;
-            for (auto x : g.nlen) n += x;
-            share += (double)(ceil_div(m, st.bm) * ceil_div(n, st.bn) * ceil_div(total_k(g), 16)) / (double)cus;
+            const double nt = (double)(ceil_div(rows(g.mlen), st.bm) * ceil_div(rows(g.nlen), st.bn)) / (double)cus;
+            tiles += nt;
+            share += nt * (double)ceil_div(total_k(g), 16);
         }
         // rounds: whole ones of equal tiles; those of several lengths fill
         // one another's
-        const double rounds = klo == khi && khi > 0 ? std::ceil(share / (double)khi - 1e-9) * (double)khi
-                                                    : std::max((double)khi, share + 0.5 * (double)khi);
-        const double us = packed + st.round * rounds + st.share * share + st.base * (double)khi;
+        const bool equal = klo == khi;
+        const double rounds = equal ? std::ceil(tiles - 1e-9) : std::max(1.0, tiles + 0.5);
+        const double steps_k = equal ? rounds * (double)khi : std::max((double)khi, share + 0.5 * (double)khi);
+        const double us = st.base + st.pack * packed + 0.28 * slow + st.share * share + st.round * steps_k + st.first * (double)khi +
+                          st.tile_us * tiles + st.round_us * rounds + results * (st.out + st.scatter * lines) / 4.9e6;
         if (best.tile < 0 || us < best.us) best = SplitTile{st.tile, us};
     }
     return best;
@@ -395,7 +428,9 @@ struct RegisterTile
 };
 
 // The FP64 register-fed tiles.  128 x 64 tiles (two waves) alone on a CU
-// share a SIMD.
+// share a SIMD.  Tile 6 (64 x 64, k over two wave sets) beat all others by
+// over 3% in 1.3% of 1411 contractions (median 12% behind): the autotuner
+// times it, the model does not ask for it.
 constexpr RegisterTile kRegisterTiles[] = {{0, 1.0, 0.77},  {1, 0.95, 0.60},  {2, 0.95, 0.94}, {3, 0.97, 0.50},
                                            {4, 0.95, 0.82}, {5, 0.965, 0.90}, {7, 0.92, 0.75}, {8, 0.97, 0.85}};
 
@@ -404,16 +439,20 @@ constexpr RegisterTile kRegisterTiles[] = {{0, 1.0, 0.77},  {1, 0.95, 0.60},  {2
 // several lengths fill one another's: half the longest wave).  Model /
 // measured: 1225^3 tile 5 93 / 92, 8 78 / 75; 1521^3 5 165 / 158, 8 132 /
 // 127; 1849^3 1 263 / 244, 2 264 / 250, 8 233 / 222; 4489 x 1225 x 4489
-// 0 1160 / 1186, 8 862 / 873; 8-irrep DPD 8 55 / 56.  Against a choice by
+// 0 1160 / 1186, 8 862 / 873; 8-irrep DPD 8 55 / 56.  A third of the results'
+// time at the write rate adds to the waves' (20480 x 1140 x 495, tile 5 441,
+// 0 401); short runs slow the pack (runs: a line_share per operand); 32 x 32
+// tiles read panels past the 256 MiB cache 15% slower (2160 x 1376 x 15360: 8
+// 2073, 5 1714).  Against a choice by
 // each tile's rate alone (us, rate / rounds): 2304^2 x 942 (48^4 with a
 // sparse index) 219 / 156, 1521^3 158 / 127, 4489 x 1225 x 4489 1176 / 872,
 // 41^4 complex 880 / 674.
-double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, int cus)
+double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, const double runs[2], int cus)
 {
     const int64_t BM = panel_tile_m(FAMILY_F64, rt.tile), BN = panel_tile_n(FAMILY_F64, rt.tile);
     const int64_t W = panel_tile_waves(FAMILY_F64, rt.tile), simds = 4LL * cus;
     int64_t waves = 0, ngemm = 0;
-    double work = 0, longest = 0, shortest = 0, packed = 0, results = 0;
+    double work = 0, longest = 0, shortest = 0, packed = 0, slow = 0, results = 0;
     for (const PanelGemm& g : gemms)
     {
         const int64_t k = total_k(g);
@@ -428,6 +467,7 @@ double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, in
         longest = std::max(longest, wave);
         shortest = ngemm ? std::min(shortest, wave) : wave;
         packed += 16.0 * (double)(m + n) * (double)k;
+        slow += 16.0 * ((double)m * (std::sqrt(runs[0]) - 1.0) + (double)n * (std::sqrt(runs[1]) - 1.0)) * (double)k;
         results += 8.0 * (double)m * (double)n;
         ngemm++;
     }
@@ -439,7 +479,9 @@ double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, in
         cyc = (double)ceil_div(waves, simds) * (longest / rt.eff + kTask);
     else
         cyc = (work / (double)simds + 0.5 * longest) / rt.eff + (double)waves / (double)simds * kTask;
-    return std::max(cyc / 2150.0, results / 5.0e6) + packed / 5.0e6 + 6.3 + 0.08 * (double)(ngemm - 1);
+    const double us = std::max(cyc / 2150.0 + 0.3 * results / 5.0e6, results / 5.0e6) +
+                      (packed + 0.45 * slow) / 5.0e6 + (ngemm == 1 ? 7.0 : 6.3 + 0.08 * (double)(ngemm - 1));
+    return BM == 32 && BN == 32 && packed / 2 > 256.0e6 ? 1.15 * us : us;
 }
 
 // Adding the k slices of a plan up: one launch, and the C panels written
@@ -524,16 +566,6 @@ GatherOperand gather_operand(const std::vector<PBlock>& bl, int src_elem)
     return o;
 }
 
-// 128-byte lines that an operand's loads touch, over those its elements
-// would fill: 1 for long runs, about 2 for runs of 29 floats.
-double line_share(const GatherOperand& o, int src_elem)
-{
-    const std::vector<int64_t>& v = o.lanes_k ? o.ks : o.rows;
-    int64_t lines = 1;
-    for (size_t i = 1; i < v.size(); i++) lines += v[i] / 128 != v[i - 1] / 128;
-    return std::max(1.0, (double)lines * 128.0 / ((double)v.size() * src_elem));
-}
-
 // Index in a side's dimensions of its unit stride one, or -1.
 int unit_dim(const Side& s)
 {
@@ -548,18 +580,31 @@ void move_first(Side& s, int d)
     std::rotate(s.stride.begin(), s.stride.begin() + d, s.stride.begin() + d + 1);
 }
 
-// The order in which the gather kernels walk the dimensions of m, n and k.
-// The planner's order follows C, and may leave an operand read with a stride
-// along its rows and along k, a line per element, on each of its re-reads.
-// Moving its unit stride dimension first costs scattered writes of C, once;
-// it is done from k = 256, where the operand has more elements than that.
-// 1517 x 713 x 1247 floats in runs of 41 and 23, one operand read across its
-// runs: 53.4 -> 42.1 us; another order of six odd extents 79 -> 50 us.
+bool same_side(const Side& a, const Side& b) { return a.len == b.len && a.stride == b.stride && a.offs == b.offs; }
+
+bool same_blocks(const std::vector<PBlock>& a, const std::vector<PBlock>& b)
+{
+    for (size_t i = 0; i < a.size() && a.size() == b.size(); i++)
+        if (a[i].base != b[i].base || !same_side(a[i].rows, b[i].rows) || !same_side(a[i].k, b[i].k)) return false;
+    return a.size() == b.size();
+}
+
+// Is an operand read with a stride along its rows and along k, a line per
+// element?
+bool strided(const PBlock& b)
+{
+    return first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1;
+}
+
+// Another order in which the gather kernels may walk the dimensions of m, n
+// and k.  The planner's order follows C, and may leave an operand strided on
+// each of its re-reads.  Moving its unit stride dimension first costs
+// scattered writes of C, once: 1517 x 713 x 1247 floats in runs of 41 and 23,
+// one operand read across its runs, 53.4 -> 42.1 us, but 40320 x 2976 x 256
+// doubles 1043 -> 1695.  From k = 256 on; single GEMMs weigh both orders
+// (GatherWalks).
 std::vector<PanelGemm> coalesced(std::vector<PanelGemm> gemms)
 {
-    const auto strided = [](const PBlock& b) {
-        return first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1;
-    };
     for (PanelGemm& g : gemms)
     {
         if (g.c.size() != 1 || g.a.empty() || g.b.empty() || total_k(g) < 256) continue;
@@ -596,15 +641,16 @@ struct GatherChoice
     int slices = 1;
     double us = 0;
     bool pieces = false;
+    int walk = 0;  // of GatherWalks
 };
 
-// What the gather tiles' plan and its models read of a plan's GEMMs, made
-// once: the GEMMs in the order in which the kernels walk them and, for those
-// with k, both operands' offsets.
+// What the gather tiles' plan and its models read of a plan's GEMMs, in the
+// order in which the kernels walk them, made once: for those with k, both
+// operands' offsets.
 struct GatherWork
 {
-    GatherWork(const std::vector<PanelGemm>& planned, int family, int src_elem)
-        : gemms(coalesced(planned)), family(family), src_elem(src_elem), ops(2 * gemms.size())
+    GatherWork(std::vector<PanelGemm> walk, int family, int src_elem)
+        : gemms(std::move(walk)), family(family), src_elem(src_elem), ops(2 * gemms.size())
     {
         const PanelGemm* big = &gemms[0];
         for (const PanelGemm& g : gemms)
@@ -616,9 +662,18 @@ struct GatherWork
             if (total_k(g) == 0) continue;
             ops[2 * i] = gather_operand(g.a, src_elem);
             ops[2 * i + 1] = gather_operand(g.b, src_elem);
-            if (family == FAMILY_F64 || &g != big) continue;
-            for (int o = 0; o < 2; o++) share = std::max(share, std::min(2.0, line_share(ops[2 * i + o], src_elem)));
+            for (const std::vector<PBlock>* bl : {&g.a, &g.b})
+                for (const PBlock& b : *bl) across = across || strided(b);
+            if (&g != big) continue;
+            for (int o = 0; o < 2; o++)
+            {
+                const GatherOperand& x = ops[2 * i + o];
+                const double r = line_share(x.rows, src_elem), k = line_share(x.ks, src_elem);
+                share[o] = x.lanes_k ? k : r;
+                runs[o] = std::min(r, k);
+            }
         }
+        if (gemms.size() == 1) out_share = result_share(gemms[0], src_elem);
     }
     // Do kernels with stages of bk k read every operand in 16-byte pieces?
     bool pieces(int64_t bk)
@@ -636,8 +691,10 @@ struct GatherWork
     int family, src_elem;
     std::vector<GatherOperand> ops;  // A and B of each GEMM
     bool scaled = false;             // some k block is scaled
-    double share = 1.0;              // split-BF16: line_share of the largest GEMM's worse operand
-    GatherChoice best;               // of all tiles (plan_panel_tables)
+    bool across = false;             // some operand is strided
+    double share[2] = {1.0, 1.0};    // line_share of the largest GEMM's operands along their lanes
+    double runs[2] = {1.0, 1.0};     // along whichever of rows and k has the longer runs
+    double out_share = 1.0;          // single GEMMs: result_share
 
   private:
     std::vector<std::pair<int64_t, bool>> pieces_;  // by stage length
@@ -647,16 +704,27 @@ struct GatherWork
 // number of k slices for these GEMMs, from a model of a CU that holds up to
 // occ workgroups.  A workgroup's stage takes `stage` cycles of the CU, a
 // round of resident workgroups at least `latency` per stage, and a task
-// `fill` cycles for its chain of table loads, first stage and epilogue.  us,
-// model / measured.  FP64 in pieces: 10^4 6 / 6.1, 16^4 7.5 / 7.4, 22^4 11 /
-// 10.4, 24^4 17 / 15.7, 30^4 39 / 37.6, 36^4 82 / 84.8, 42^4 202 / 202 on the
-// 32 x 32 tile, permuted 64/32 508 / 508 on the 64 x 64 one; element-wise:
-// 17^4 10.3 / 10.2, 25^4 23 / 23.5, 31^4 59 / 60.  Split-BF16: 24^4 17 / 17.7
-// and 36^4 44 / 44.3 on the 64 x 64 tile, permuted 64/32 233 / 237 whole and
-// 214 / 210 in two slices on the 128 x 128 one; its stages are bound by L2
-// where short runs make it fetch lines that it uses a part of (line_share: runs
-// of 29 and 31 floats, 2.0, took the 64 x 64 tile 1.7-2.1 times the cycles and
-// the 128 x 128 one 1.5-1.8; runs of 49 and 51, 1.6, the latter 1.07-1.17).
+// `fill` cycles for its chain of table loads, first stage and epilogue.
+//
+// Single GEMMs: a stage takes `lines` of itself longer for each step of the
+// square roots of the operands' line_share; results are written at `out` of 5
+// TB/s and `scatter` more for each further line that a row of C touches; the
+// sum of slices takes `sum` us and `again` of their bytes at 4.2 TB/s.  Fitted
+// to 443 contractions in 1 to 512 slices and, for short runs and scattered
+// results, to 3200 in the planner's slices (1e6 to 2.5e10 products, extents
+// of 1 to 64, every order of the labels): median error 5% (pieces), 5-7%
+// (element-wise) and 7-8% (split-BF16), 90th percentile 14-18 and 18-23%.  The
+// slices and tile that it picks take 1.0% (split-BF16) and 1.9% (FP64) longer
+// than the best.  Loads of pairs (two elements to a line; FP64: from operands
+// past the L2s, 32 MiB) are up to twice as long as modelled, hence `pairs`.
+//
+// Several GEMMs: split-BF16's stages are bound by L2 where short runs make it
+// fetch lines that it uses a part of (line_share: runs of 29 and 31 floats,
+// 2.0, took the 64 x 64 tile 1.7-2.1 times the cycles and the 128 x 128 one
+// 1.5-1.8; runs of 49 and 51, 1.6, the latter 1.07-1.17).
+//
+// FP64 tile 0 (128 x 64) is behind the 64 x 64 one wherever both were timed
+// (permuted 64/32 546 / 508 us): only the autotuner and the knob ask for it.
 GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
 {
     const std::vector<PanelGemm>& gemms = w.gemms;
@@ -666,17 +734,19 @@ GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
         int family, lt;
         bool pieces;
         int occ;
-        double stage, latency, fill;
+        double stage, latency, fill;                         // several GEMMs
+        double stage1, latency1, fill1, lines, out, scatter, base, sum, again;  // one GEMM
     };
-    constexpr Model models[] = {{FAMILY_F64, 1, true, 4, 1050, 1500, 5000},
-                                {FAMILY_F64, 2, true, 4, 567, 1000, 5000},
-                                {FAMILY_F64, 0, false, 2, 2500, 2600, 6000},
-                                {FAMILY_F64, 1, false, 4, 1260, 2000, 6000},
-                                {FAMILY_F64, 2, false, 3, 960, 1300, 6000},
-                                {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000},
-                                {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000}};
-    const bool f64 = family == FAMILY_F64;
-    const double share = w.share;
+    constexpr Model models[] = {
+        {FAMILY_F64, 1, true, 4, 1050, 1500, 5000, 1060, 1400, 3000, 0.030, 0.9, 0.060, 2.50, 3.5, 2.0},
+        {FAMILY_F64, 2, true, 4, 567, 1000, 5000, 590, 930, 4500, 0.096, 1.0, 0.030, 2.20, 3.5, 2.0},
+        {FAMILY_F64, 0, false, 2, 2500, 2600, 6000, 2500, 2600, 3000, 0.030, 0.9, 0.060, 2.50, 3.5, 2.0},
+        {FAMILY_F64, 1, false, 4, 1260, 2000, 6000, 1214, 1717, 3000, 0.045, 0.9, 0.060, 2.60, 3.5, 2.0},
+        {FAMILY_F64, 2, false, 3, 960, 1300, 6000, 900, 1220, 4500, 0.055, 1.0, 0.012, 2.20, 3.5, 2.0},
+        {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000, 1455, 2095, 3800, 0.150, 1.5, 0.080, 7.10, 2.2, 2.1},
+        {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000, 1040, 1683, 5500, 0.200, 1.5, 0.045, 3.45, 2.0, 3.1}};
+    const bool f64 = family == FAMILY_F64, single = gemms.size() == 1;
+    const double share = std::max(w.share[0], w.share[1]), most = 128.0 / src_elem;
     constexpr double kGHz = 2.15;
     GatherChoice best;
     const int first = panel_num_tiles(family) - (f64 ? lds_num_tiles() : gather_bf16_num_tiles());
@@ -689,14 +759,19 @@ GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
         const int64_t bk = panel_tile_k(family, tile);
         const bool pieces = f64 && w.pieces(bk);
         if (f64 && md.pieces != pieces && md.lt != 0) continue;
-        const double over = std::max(0.0, share - 1.3);
-        const double lines = f64 ? 1.0 : md.lt == 0 ? 1.0 + 1.6 * over * over : std::max(1.0, 0.9 * share);
+        const double over = std::max(0.0, std::min(2.0, share) - 1.3);
+        double lines = f64 ? 1.0 : md.lt == 0 ? 1.0 + 1.6 * over * over : std::max(1.0, 0.9 * std::min(2.0, share));
+        if (single)
+            lines = 1.0 + md.lines * (std::sqrt(std::min(most, w.share[0])) + std::sqrt(std::min(most, w.share[1])) - 2.0);
+        const double stage = single ? md.stage1 : md.stage, latency = single ? md.latency1 : md.latency;
+        const double fill = single ? md.fill1 : md.fill;
         int64_t kmax = 1;
-        double bytes = 0;
+        double bytes = 0, results = 0;
         for (const PanelGemm& g : gemms)
         {
             const int64_t k = total_k(g);
             kmax = std::max(kmax, k);
+            results += (double)src_elem * (double)g.mlen[0] * (double)g.nlen[0];
             bytes += (double)src_elem * ((double)g.mlen[0] * k + (double)g.nlen[0] * k + (double)g.mlen[0] * g.nlen[0]);
         }
         for (int64_t S = 1; S <= std::min<int64_t>(std::max<int64_t>(1, ceil_div(kmax, 2 * bk)), 1024);
@@ -710,34 +785,89 @@ GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
                 const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g), s = std::max<int64_t>(1, ceil_div(k, kslice));
                 const int64_t nt = ceil_div(m, BM) * ceil_div(n, BN) * s;
                 ntask += nt;
-                work += (double)nt * std::ceil(std::min((double)kslice, (double)k) / (double)bk) * md.stage * lines;
+                work += (double)nt * std::ceil(std::min((double)kslice, (double)k) / (double)bk) * stage * lines;
                 if (s > 1) panels += (f64 ? 8.0 : 4.0) * (double)s * (double)m * (double)n;
             }
             if (S > 1 && (panels > (double)(128 << 20) || ntask > 8 * cus)) break;
             const double st = (double)(std::min(kslice, ceil_div(kmax, bk) * bk) / bk);
             const int64_t per = ceil_div(ntask, cus);
-            double cyc;
-            if (per <= md.occ)
-                cyc = md.fill + st * lines * std::max((double)per * md.stage, md.latency);
-            else if (gemms.size() == 1)  // 64 x 64 split-BF16 tiles in several rounds: bound by L2
-                cyc = (double)ceil_div(per, md.occ) * md.fill +
-                      (double)per * st * md.stage * lines * (!f64 && md.lt == 1 ? 1.16 : 1.0);
+            double us;
+            if (single)
+            {
+                const double cyc =
+                    (double)ceil_div(per, md.occ) * fill + st * lines * std::max((double)per * stage, latency);
+                us = cyc / (kGHz * 1e3);
+                if (panels == 0)
+                    us += results * (md.out + md.scatter * (std::min(most, w.out_share) - 1.0)) / 5.0e6;
+                // (where both take as long, neither hides the other whole)
+                const double mem = bytes / 5.5e6;
+                us = std::pow(std::pow(us, 6) + std::pow(mem, 6), 1.0 / 6.0);
+                const double slow = pieces ? 1.4 : 1.2;
+                const double pairs = share * src_elem < 63.5 || (f64 && bytes - results < 32.0e6) ? 1.0 : slow;
+                us = (us + md.base + (panels > 0 ? md.sum + md.again * panels / 4.2e6 : 0.0)) *
+                     pairs;
+            }
             else
-                cyc = (double)ceil_div(per, md.occ) * md.fill + std::max(1.05 * work / cus, st * md.stage * lines * md.occ);
-            double us = std::max(cyc / (kGHz * 1e3), bytes / 5.5e6) + 1.5;
-            if (panels > 0) us += reduce_us(panels);
-            if (best.tile < 0 || us < best.us) best = GatherChoice{tile, (int)S, us, pieces};
+            {
+                double cyc;
+                if (per <= md.occ)
+                    cyc = fill + st * lines * std::max((double)per * stage, latency);
+                else
+                    cyc = (double)ceil_div(per, md.occ) * fill +
+                          std::max(1.05 * work / cus, st * stage * lines * md.occ);
+                us = std::max(cyc / (kGHz * 1e3), bytes / 5.5e6) + 1.5 + (panels > 0 ? reduce_us(panels) : 0.0);
+            }
+            if (best.tile < 0 || us < best.us) best = GatherChoice{tile, (int)S, us, pieces, 0};
         }
     }
     return best;
 }
 
+// The orders that a plan's gather tile may walk, and the best choice of one,
+// a tile and a number of slices.
+struct GatherWalks
+{
+    GatherWalks(const std::vector<PanelGemm>& planned, int family, int src_elem)
+    {
+        std::vector<PanelGemm> other = coalesced(planned);
+        if (planned.size() > 1)
+        {
+            walks.emplace_back(std::move(other), family, src_elem);
+            return;
+        }
+        walks.emplace_back(planned, family, src_elem);
+        const PanelGemm &a = planned[0], &b = other[0];
+        if (a.a.empty() || (same_blocks(a.a, b.a) && same_blocks(a.b, b.b))) return;
+        walks.emplace_back(std::move(other), family, src_elem);
+    }
+    // only: for that tile
+    GatherChoice choose(int cus, int only = -1)
+    {
+        if (only < 0 ? best_.tile >= 0 : best_.tile == only) return best_;
+        GatherChoice c;
+        for (size_t i = 0; i < walks.size(); i++)
+        {
+            GatherChoice x = gather_choice(walks[i], cus, only);
+            x.walk = (int)i;
+            // a strided operand, a line per element: the last choice
+            const bool last = walks[i].across && !x.pieces, clast = c.tile >= 0 && walks[c.walk].across && !c.pieces;
+            if (c.tile < 0 || (last == clast ? x.us < c.us : clast)) c = x;
+        }
+        if (only < 0) best_ = c;
+        return c;
+    }
+    std::vector<GatherWork> walks;
+
+  private:
+    GatherChoice best_;
+};
+
 // Does a plan take its best gather tile (us by the model) without a
-// measurement?  packed: the best register-fed tile's us (FP64).
+// measurement?  packed: the best register-fed tile's us.
 // FP64:
-//   Operands in 16-byte pieces: always (no pack, no panels).  10^4 6.7 / 6.1,
-//   16^4 9.6 / 7.4, 24^4 27.3 / 15.7, 36^4 95 / 85, permuted 64/32 575 / 508
-//   (us, packed / gathered).
+//   Operands in 16-byte pieces: single GEMMs where that costs less (no pack,
+//   no panels: 10^4 6.7 / 6.1, 16^4 9.6 / 7.4, 24^4 27.3 / 15.7, 36^4 95 / 85,
+//   permuted 64/32 575 / 508 us, packed / gathered), others always.
 //   Batches: packing leaves each register tile a short loop of scattered
 //   reads.  4096-instance mix (1024 of them) 5478 / 4862, 1000 of extents
 //   12-24 1495 / 1224, 200 of 12-40 2949 / 2427.
@@ -747,28 +877,33 @@ GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
 //   21, 91 x 91 x 357 42 / 8.1), short k (33 x 14553 x 21 13.1 / 7.8, 70 x
 //   112000 x 40 75 / 59), small DPD blocks (27.5 / 17.9), 4489 x 225 x 4489
 //   254 / 203.
-// Split-BF16: always, but for GEMMs with both sides from 2048 on, where the
-// 256 x 128 panel tiles (packed: their us) may fill their rounds better.
-// 8^4 12.5 / 6.8, 24^4 22.4 / 15.7, 36^4 81 / 44, 8-irrep DPD 48.7 / 29.7,
-// 1024-instance batch 3494 / 2246, 48^4 281 / 171, permuted 67/35 608 / 383;
-// 53^4 (242 tiles) 272 / 284, 55^4 (288) 458 / 419, 59^4 (392) 569 / 638,
-// 61^4 657 / 718, 80^4 2562 / 2856.
-bool gather_preferred(const std::vector<PanelGemm>& gemms, int family, const GatherChoice& c, double packed)
+// Split-BF16: single GEMMs where that costs less (8^4 12.5 / 6.8, 24^4 22.4 /
+// 15.7, 36^4 81 / 44, 48^4 281 / 171; 6480 x 1824 x 3328 with a stride of two
+// along k 567 / 1164, 1972 x 1920 x 4560 in pairs 266 / 530).  Several: always
+// (8-irrep DPD 48.7 / 29.7, 1024-instance batch 3494 / 2246), but for GEMMs
+// with both sides from 2048 on, where the 256 x 128 panel tiles may fill their
+// rounds better.
+bool gather_preferred(const GatherWork& w, const GatherChoice& c, double packed)
 {
+    const bool f64 = w.family == FAMILY_F64;
+    if (w.gemms.size() == 1 && !(f64 && t_direct_all))
+    {
+        // (the packed model is 10% short below 30 us, the pieces' one long)
+        if (c.pieces) return 0.85 * c.us < packed;
+        const bool large = !f64 && std::min(w.gemms[0].mlen[0], w.gemms[0].nlen[0]) >= 2048;
+        return !w.across && (large ? 1.06 : 1.0) * c.us < packed;
+    }
     if (c.pieces) return true;
+    if (w.across) return false;
+    if (f64) return t_direct_all || c.us < packed;
     double large = 0, all = 0;
-    for (const PanelGemm& g : gemms)
+    for (const PanelGemm& g : w.gemms)
     {
         const double f = (double)g.mlen[0] * (double)g.nlen[0] * (double)total_k(g);
         all += f;
         if (std::min(g.mlen[0], g.nlen[0]) >= 2048) large += f;
-        for (const std::vector<PBlock>* bl : {&g.a, &g.b})
-            for (const PBlock& b : *bl)
-                if (first_step(b.rows) != 1 && first_step(b.k) != 1 && side_count(b.rows) > 1 && side_count(b.k) > 1)
-                    return false;
     }
-    if (family != FAMILY_F64) return large <= 0.5 * all || 1.06 * c.us < packed;
-    return t_direct_all || c.us < packed;
+    return large <= 0.5 * all || 1.06 * c.us < packed;
 }
 
 }  // namespace
@@ -959,8 +1094,8 @@ int ksplit_forced();
 bool gather_tables(GatherWork& w, int tile, PanelTables& T, int64_t kslice);
 // tables_for_tile with the tasks grouped by which operands they read
 // directly (one kernel variant per launch); packed: every operand packed
-// (gather tiles: from work)
-bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int tile, PanelTables& T,
+// (gather tiles: from walks)
+bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWalks* walks, int family, int tile, PanelTables& T,
                     int src_elem, bool packed = false);
 // Autotuner candidates: a tile, or with kPackedBit the same tile with every
 // operand packed (timed next to the planner's direct reads)
@@ -968,7 +1103,7 @@ constexpr int kPackedBit = 256;
 // model_tile: the cost model's pick, preferred among finalists that tie.
 // Returns the measured choice (a tile, + kPackedBit for its every-operand-
 // packed variant) or -1.
-int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int dtype, bool swap,
+int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWalks* walks, int family, int dtype, bool swap,
                   const std::vector<int>& cands, int model_tile);
 uint64_t tune_key(const std::vector<PanelGemm>& gemms, int family, bool real);
 // Do the tuner's candidates run on the tensors?
@@ -1054,16 +1189,20 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
             tile = tm.tile;
         }
     }
+    std::unique_ptr<GatherWalks> walks;
+    if (rounds && gathers) walks.reset(new GatherWalks(gemms, family, src_elem));
+    double runs[2] = {1.0, 1.0};
+    if (walks && gemms.size() == 1) std::copy(walks->walks[0].runs, walks->walks[0].runs + 2, runs);
     if (rounds && family == FAMILY_BF16X3)
     {
-        const SplitTile st = split_tile(gemms, cus);
+        const SplitTile st = split_tile(gemms, runs, cus);
         best = st.us;
         tile = st.tile;
     }
     for (const RegisterTile& rt : kRegisterTiles)
     {
         if (!rounds || family != FAMILY_F64) break;
-        const double us = packed_us(gemms, rt, cus);
+        const double us = packed_us(gemms, rt, runs, cus);
         if (best < 0 || us < best)
         {
             best = us;
@@ -1071,15 +1210,13 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
         }
     }
     // Gather tiles: by their own model, against the best register-fed tile.
-    std::unique_ptr<GatherWork> work;
-    if (rounds && gathers)
+    if (walks)
     {
-        work.reset(new GatherWork(gemms, family, src_elem));
-        work->best = gather_choice(*work, cus);
-        if (gather_preferred(work->gemms, family, work->best, best)) tile = work->best.tile;
+        const GatherChoice c = walks->choose(cus);
+        if (gather_preferred(walks->walks[c.walk], c, best)) tile = c.tile;
     }
     bool packed = false;
-    const int tuned = autotune_tile(gemms, work.get(), family, dtype, swap, cands, tile);
+    const int tuned = autotune_tile(gemms, walks.get(), family, dtype, swap, cands, tile);
     if (tuned >= 0)
     {
         tile = tuned % kPackedBit;
@@ -1096,8 +1233,8 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
             packed = false;
         }
     }
-    if (panel_tile_lds(family, tile) && !work) work.reset(new GatherWork(gemms, family, src_elem));
-    if (!tables_uniform(gemms, work.get(), family, tile, T, src_elem, packed)) return false;
+    if (panel_tile_lds(family, tile) && !walks) walks.reset(new GatherWalks(gemms, family, src_elem));
+    if (!tables_uniform(gemms, walks.get(), family, tile, T, src_elem, packed)) return false;
     T.swap = swap;
     if (t_tune_recall) T.tune_key = tune_key(gemms, family, tune_real(family));
     return true;
@@ -1109,7 +1246,7 @@ namespace
 // Tasks grouped by which operands they read straight from the tensors
 // (GEMMs of one batch may differ): the groups become separate launches of
 // the matching kernel variant.
-bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int tile, PanelTables& T,
+bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWalks* walks, int family, int tile, PanelTables& T,
                     int src_elem, bool packed)
 {
     const bool allow[2] = {!packed, !packed};
@@ -1119,9 +1256,9 @@ bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWork* work, int f
         int64_t kmax = 1;
         for (const PanelGemm& g : gemms) kmax = std::max(kmax, total_k(g));
         const int64_t bk = panel_tile_k(family, tile);
-        int64_t S = ksplit_forced();
-        if (!S) S = (work->best.tile == tile ? work->best : gather_choice(*work, device_cu_count(), tile)).slices;
-        return gather_tables(*work, tile, T, ceil_div(ceil_div(kmax, S), bk) * bk);
+        const GatherChoice c = walks->choose(device_cu_count(), tile);
+        const int64_t S = ksplit_forced() ? ksplit_forced() : c.slices;
+        return gather_tables(walks->walks[c.walk], tile, T, ceil_div(ceil_div(kmax, S), bk) * bk);
     }
     if (!tables_for_tile(gemms, family, tile, T, allow, src_elem)) return false;
     auto group = [](const PanelTask& t) {
@@ -1148,7 +1285,6 @@ bool tables_uniform(const std::vector<PanelGemm>& gemms, GatherWork* work, int f
     return true;
 }
 
-bool same_side(const Side& a, const Side& b) { return a.len == b.len && a.stride == b.stride && a.offs == b.offs; }
 
 }  // namespace
 
@@ -1431,10 +1567,7 @@ bool same_operand(const PanelGemm& x, const PanelGemm& y, int o)
 {
     if (x.share != o + 1 || y.share != o + 1 || x.klen != y.klen) return false;
     if ((o == 0 ? x.mlen : x.nlen) != (o == 0 ? y.mlen : y.nlen)) return false;
-    const std::vector<PBlock>&p = o == 0 ? x.a : x.b, &q = o == 0 ? y.a : y.b;
-    for (size_t i = 0; i < p.size() && p.size() == q.size(); i++)
-        if (p[i].base != q[i].base || !same_side(p[i].rows, q[i].rows) || !same_side(p[i].k, q[i].k)) return false;
-    return p.size() == q.size();
+    return o == 0 ? same_blocks(x.a, y.a) : same_blocks(x.b, y.b);
 }
 
 bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, PanelTables& T,
@@ -2042,7 +2175,7 @@ uint64_t tune_key(const std::vector<PanelGemm>& gemms, int family, bool real)
     return h;
 }
 
-int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWork* work, int family, int dtype, bool swap,
+int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWalks* walks, int family, int dtype, bool swap,
                   const std::vector<int>& cands_in, int model_tile)
 {
     const std::vector<int>& cands0 = cands_in;
@@ -2092,12 +2225,12 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWork* work, int fam
     std::vector<PanelTables> tabs;
     for (int c : cands0)
     {
-        if ((!real || !work) && panel_tile_lds(family, c)) continue;
+        if ((!real || !walks) && panel_tile_lds(family, c)) continue;
         // with tensors: grouped as the plan will be; without: both operands
         // in panels
         const bool none[2] = {false, false};
         PanelTables T1;
-        if (real ? !tables_uniform(gemms, work, family, c, T1, dtype == 0 ? 8 : 4)
+        if (real ? !tables_uniform(gemms, walks, family, c, T1, dtype == 0 ? 8 : 4)
                  : !tables_for_tile(gemms, family, c, T1, none, dtype == 0 ? 8 : 4))
             return -1;
         const bool reads = panel_tile_lds(family, c) || T1.group_n[1] + T1.group_n[2] + T1.group_n[3] > 0;
@@ -2106,7 +2239,7 @@ int autotune_tile(const std::vector<PanelGemm>& gemms, GatherWork* work, int fam
         if (real && reads && !t_direct_all && !panel_tile_lds(family, c))
         {
             PanelTables T2;
-            if (!tables_uniform(gemms, work, family, c, T2, dtype == 0 ? 8 : 4, true)) return -1;
+            if (!tables_uniform(gemms, walks, family, c, T2, dtype == 0 ? 8 : 4, true)) return -1;
             if ((size_t)T2.ws_panel * eb <= free_bytes / 4)
             {
                 cands.push_back(c + kPackedBit);
