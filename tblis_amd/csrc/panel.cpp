@@ -325,7 +325,10 @@ double result_share(const PanelGemm& g, int elem)
 // 64, in every order of their labels; median error 5% (0, 1) to 10%, 90th
 // percentile 18 to 30%.  Short k and scattered results are where the tiles
 // differ most: 28500 x 160 x 96 floats 0 46, 2 38, 3 33 us; 5220 x 5120 x 174
-// 0 153, 1 132, 3 102; 11264 x 24400 x 58 0 931, 1 768, 3 545.
+// 0 153, 1 132, 3 102; 11264 x 24400 x 58 0 931, 1 768, 3 545.  GEMMs of
+// several lengths (complex batches and DPD) keep to four tiles and the rates
+// of their k steps, where the constants of equal ones cost 20% (382 complex
+// instances of 12-22: 0 1864, 3 2337).
 struct SplitTile
 {
     int tile;
@@ -341,13 +344,15 @@ SplitTile split_tile(const std::vector<PanelGemm>& gemms, const double runs[2], 
         double share, round, first;  // us of 16 k: of a CU's share of the tiles, of a round of tiles, of a GEMM
         double tile_us, round_us;    // us of a CU's share of the tiles and of a round besides their k
         double out, scatter;         // of the results at 4.9 TB/s, and for each further line they touch
+        double share_n, round_n, first_n;  // share, round, first of GEMMs of several lengths (0: not for them)
     };
-    constexpr Step steps[] = {{0, 256, 128, 12.5, 1.4, 0.22, 0.75, 0.0, 0.7, 15.0, 1.2, 0.074},
-                              {1, 128, 256, 9.0, 1.5, 0.20, 0.79, 0.0, 2.6, 13.0, 0.55, 0.06},
-                              {2, 128, 128, 13.0, 1.4, 0.17, 0.56, 0.0, 2.3, 4.6, 0.4, 0.073},
-                              {3, 64, 64, 9.0, 1.2, 0.0, 0.29, 0.44, 0.16, 0.23, 0.7, 0.076},
-                              {4, 64, 64, 8.5, 1.55, 0.025, 0.22, 0.035, 0.0, 2.0, 0.0, 0.065},
-                              {5, 64, 64, 9.0, 1.65, 0.025, 0.225, 0.0, 0.5, 2.0, 0.5, 0.12}};
+    constexpr Step steps[] = {
+        {0, 256, 128, 12.5, 1.4, 0.22, 0.75, 0.0, 0.7, 15.0, 1.2, 0.074, 0.33, 0.95, 0.0},
+        {1, 128, 256, 9.0, 1.5, 0.20, 0.79, 0.0, 2.6, 13.0, 0.55, 0.06, 0.0, 0.0, 0.0},
+        {2, 128, 128, 13.0, 1.4, 0.17, 0.56, 0.0, 2.3, 4.6, 0.4, 0.073, 0.0, 0.86, 0.0},
+        {3, 64, 64, 9.0, 1.2, 0.0, 0.29, 0.44, 0.16, 0.23, 0.7, 0.076, 0.0, 0.0, 0.0},
+        {4, 64, 64, 8.5, 1.55, 0.025, 0.22, 0.035, 0.0, 2.0, 0.0, 0.065, 0.26, 0.0, 0.30},
+        {5, 64, 64, 9.0, 1.65, 0.025, 0.225, 0.0, 0.5, 2.0, 0.5, 0.12, 0.28, 0.0, 0.27}};
     double packed = 0, slow = 0, results = 0;
     int64_t klo = -1, khi = 0;
     const PanelGemm* big = &gemms[0];
@@ -378,13 +383,20 @@ SplitTile split_tile(const std::vector<PanelGemm>& gemms, const double runs[2], 
             tiles += nt;
             share += nt * (double)ceil_div(total_k(g), 16);
         }
-        // rounds: whole ones of equal tiles; those of several lengths fill
-        // one another's
-        const bool equal = klo == khi;
-        const double rounds = equal ? std::ceil(tiles - 1e-9) : std::max(1.0, tiles + 0.5);
-        const double steps_k = equal ? rounds * (double)khi : std::max((double)khi, share + 0.5 * (double)khi);
-        const double us = st.base + st.pack * packed + 0.28 * slow + st.share * share + st.round * steps_k + st.first * (double)khi +
-                          st.tile_us * tiles + st.round_us * rounds + results * (st.out + st.scatter * lines) / 4.9e6;
+        double us;
+        if (klo == khi)
+        {
+            const double rounds = std::ceil(tiles - 1e-9);  // whole ones of equal tiles
+            us = st.base + st.pack * packed + 0.28 * slow + st.share * share + st.round * rounds * (double)khi +
+                 st.first * (double)khi + st.tile_us * tiles + st.round_us * rounds +
+                 results * (st.out + st.scatter * lines) / 4.9e6;
+        }
+        else  // tiles of several lengths fill one another's rounds
+        {
+            if (st.share_n == 0.0 && st.round_n == 0.0) continue;
+            us = 9.0 + packed + st.share_n * share + st.round_n * std::max((double)khi, share + 0.5 * (double)khi) +
+                 st.first_n * (double)khi;
+        }
         if (best.tile < 0 || us < best.us) best = SplitTile{st.tile, us};
     }
     return best;
@@ -443,7 +455,8 @@ constexpr RegisterTile kRegisterTiles[] = {{0, 1.0, 0.77},  {1, 0.95, 0.60},  {2
 // time at the write rate adds to the waves' (20480 x 1140 x 495, tile 5 441,
 // 0 401); short runs slow the pack (runs: a line_share per operand); 32 x 32
 // tiles read panels past the 256 MiB cache 15% slower (2160 x 1376 x 15360: 8
-// 2073, 5 1714).  Against a choice by
+// 2073, 5 1714); these three for single GEMMs (594 strided instances of 4-28:
+// 5 2105, which they would make 1 2380).  Against a choice by
 // each tile's rate alone (us, rate / rounds): 2304^2 x 942 (48^4 with a
 // sparse index) 219 / 156, 1521^3 158 / 127, 4489 x 1225 x 4489 1176 / 872,
 // 41^4 complex 880 / 674.
@@ -479,8 +492,10 @@ double packed_us(const std::vector<PanelGemm>& gemms, const RegisterTile& rt, co
         cyc = (double)ceil_div(waves, simds) * (longest / rt.eff + kTask);
     else
         cyc = (work / (double)simds + 0.5 * longest) / rt.eff + (double)waves / (double)simds * kTask;
+    if (ngemm > 1)
+        return std::max(cyc / 2150.0, results / 5.0e6) + packed / 5.0e6 + 6.3 + 0.08 * (double)(ngemm - 1);
     const double us = std::max(cyc / 2150.0 + 0.3 * results / 5.0e6, results / 5.0e6) +
-                      (packed + 0.45 * slow) / 5.0e6 + (ngemm == 1 ? 7.0 : 6.3 + 0.08 * (double)(ngemm - 1));
+                      (packed + 0.45 * slow) / 5.0e6 + 7.0;
     return BM == 32 && BN == 32 && packed / 2 > 256.0e6 ? 1.15 * us : us;
 }
 
