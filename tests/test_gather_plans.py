@@ -306,3 +306,59 @@ def test_gathered_or_packed(labels, ext, dtype, gather):
     A, rest = labels.split(",")
     B, C_ = rest.split("->")
     assert bool(Plan(*[_tensor(ext, s) for s in (A, B, C_)], dtype=dtype).gather) == gather
+
+
+def _matrix(m, n, row_major, labels):
+    return [m, n], [n, 1] if row_major else [1, m], labels
+
+
+SHAPES = [(32, 64, 16), (34, 66, 18), (130, 2, 130), (66, 34, 31), (33, 64, 98), (64, 130, 162), (129, 127, 47),
+          (200, 8, 80), (8, 264, 1100)]
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("ra", [False, True])
+@pytest.mark.parametrize("rb", [False, True])
+def test_load_modes(ra, rb, aligned, monkeypatch):
+    """FP64 pieces run where both operands' contiguous extent and the other
+    stride are even and the tensors start on 16 bytes; split-BF16 loads
+    aligned eights of k in mode 2, other contiguous k in mode 1, rows in
+    mode 0."""
+    for m, n, k in SHAPES:
+        A, B, C_ = _matrix(m, k, ra, "ak"), _matrix(k, n, rb, "kb"), _matrix(m, n, True, "ab")
+        even = (k if ra else m) % 2 == 0 and (n if rb else k) % 2 == 0
+        for tile in ("9", "10", "11"):
+            monkeypatch.setenv("TBLIS_HIP_PANEL_TILE", tile)
+            p = Plan(A, B, C_, F64, aligned=aligned)
+            assert (p.tile, p.pieces) == (int(tile), aligned and even), (m, n, k)
+            assert list(p.groups) == [ra + 2 * (not rb)]
+        eights = 2 if aligned and k % 8 == 0 else 1
+        for tile in ("6", "7"):
+            monkeypatch.setenv("TBLIS_HIP_PANEL_TILE", tile)
+            p = Plan(A, B, C_, F32, aligned=aligned)
+            assert p.tile == int(tile)
+            assert list(p.groups) == [(eights if ra else 0) + 3 * (0 if rb else eights)], (m, n, k)
+
+
+@pytest.mark.parametrize("dtype,elem", [(F64, 8), (F32, 4)])
+@pytest.mark.parametrize("back", [1, -1])
+def test_reach_of_four_gib(back, dtype, elem):
+    """Offsets are 32-bit bytes: an operand that spans 4 GiB is packed, one
+    that ends just below is gathered, in either direction of its stride."""
+    for gather, span in ((True, (1 << 32) // elem - 2), (False, (1 << 32) // elem)):
+        A = [64, 8], [1, back * ((span - 64) // 7)], "ak"
+        A[1][1] += back * (0 if gather else 1)
+        reach = (63 + 7 * abs(A[1][1]) + 1) * elem
+        assert (reach < 1 << 32) == gather
+        plan = Plan(A, _matrix(8, 64, False, "kb"), _matrix(64, 64, False, "ab"), dtype)
+        assert bool(plan.gather) == gather
+
+
+@pytest.mark.parametrize("m,n,k,dtype,tile", [
+    (1225, 1225, 120, F64, 10), (33, 4489, 225, F64, 11), (2500, 31, 2499, F64, 11), (4489, 1225, 4489, F64, 8),
+    (2025, 2025, 2025, F64, 5), (1296, 1296, 1296, F32, 7), (2561, 2049, 1700, F32, 6), (4096, 4096, 2048, F32, 1),
+    (8192, 8192, 8192, F32, 0)])
+def test_tiles_picked(m, n, k, dtype, tile):
+    """One size of each side of the lines between tiles."""
+    plan = Plan(_matrix(m, k, False, "ak"), _matrix(k, n, False, "kb"), _matrix(m, n, dtype == F32, "ab"), dtype)
+    assert plan.tile == tile
