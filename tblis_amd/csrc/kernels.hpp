@@ -28,8 +28,8 @@ int panel_num_tiles(int family);
 int panel_tile_m(int family, int tile);
 int panel_tile_n(int family, int tile);
 int panel_tile_waves(int family, int tile);
-// FP64 tiles that stage both operands through LDS (every operand read from
-// the tensors, single-block GEMMs only)
+// Gather tiles of either family: both operands read from the tensors through
+// LDS (one row block per operand, any number of k blocks, one C block)
 bool panel_tile_lds(int family, int tile);
 int panel_tile_k(int family, int tile);  // gather tiles: k per stage
 struct PanelLaunch

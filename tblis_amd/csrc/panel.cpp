@@ -287,9 +287,9 @@ struct TileModel
 // dense 24^4 GEMM (8).  Split-BF16: per tile of the BF16 table.
 const TileModel kModelsF64[] = {{0, 0.85, 2}, {2, 0.70, 2}, {3, 0.82, 2}, {4, 0.80, 2},
                                 {1, 0.62, 6}, {5, 0.72, 6}, {6, 0.62, 4}, {7, 0.62, 4},
-                                {8, 0.50, 4}, {9, 0.88, 1}, {10, 0.55, 2}, {11, 0.80, 1}};
+                                {8, 0.50, 4}};
 const TileModel kModelsBf16[] = {{0, 0.55, 1}, {1, 0.55, 1}, {2, 0.45, 2}, {3, 0.35, 4},
-                                 {4, 0.30, 4}, {5, 0.25, 4}, {6, 0, 2},    {7, 0, 3}};
+                                 {4, 0.30, 4}, {5, 0.25, 4}};
 const TileModel kModelsOzaki[] = {{0, 0.30, 1}};
 
 int64_t total_k(const PanelGemm& g)
@@ -1191,11 +1191,8 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
     for (int mi = 0; mi < nmodels; mi++)
     {
         const TileModel& tm = models[mi];
-        if (tm.tile >= panel_num_tiles(family)) continue;
-        if (family == FAMILY_BF16X3 && !panel_tile_lds(family, tm.tile) && panel_bf16_tile_fast_only(tm.tile)) continue;
-        if (panel_tile_lds(family, tm.tile) && !gathers) continue;
+        if (family == FAMILY_BF16X3 && panel_bf16_tile_fast_only(tm.tile)) continue;
         cands.push_back(tm.tile);
-        if (panel_tile_lds(family, tm.tile)) continue;  // gather tiles have a model of their own
         if (rounds) continue;
         double c = tile_cost(gemms, tm, cus, family);
         if (best < 0 || c < best)
@@ -1204,6 +1201,9 @@ bool plan_panel_tables(std::vector<PanelGemm> gemms, PanelTables& T, int family,
             tile = tm.tile;
         }
     }
+    // gather tiles have a model of their own
+    for (int t = 0; gathers && t < panel_num_tiles(family); t++)
+        if (panel_tile_lds(family, t)) cands.push_back(t);
     std::unique_ptr<GatherWalks> walks;
     if (rounds && gathers) walks.reset(new GatherWalks(gemms, family, src_elem));
     double runs[2] = {1.0, 1.0};
@@ -2046,13 +2046,14 @@ bool tables_for_tile(const std::vector<PanelGemm>& gemms, int family, int tile, 
 // ------------------------------------------------------------------ autotuner
 //
 // Times every candidate tile of the panel GEMM on the device for this list
-// of GEMM shapes and keeps the fastest.  The measurement never touches the
-// caller's data: the GEMM runs on scratch panels of pseudo-random values
+// of GEMM shapes and keeps the fastest.  The measurement never writes the
+// caller's data: with the tensors it packs and gathers from them as the plan
+// would; without, the GEMM runs on scratch panels of pseudo-random values
 // laid out for the candidate (all-zero operands would time the MFMA units at
-// an unrealistically low power draw) and writes C tiles into a scratch
-// buffer (1024 tile slots, reused round-robin).  Pack and unpack costs do not depend on the tile and
-// are not timed.  Results are cached per (family, GEMM shapes) for the
-// process and, with TBLIS_HIP_TUNE_FILE, in a JSON-lines file that later
+// an unrealistically low power draw) and neither packs nor gathers.  C tiles go
+// to a scratch buffer (1024 tile slots, reused round-robin).  Results are
+// cached for the process by family, GEMM shapes and, with the tensors, layout
+// (tune_key) and, with TBLIS_HIP_TUNE_FILE, in a JSON-lines file that later
 // processes read back.
 
 std::atomic<int> g_autotune{-1};  // -1: not yet read from TBLIS_HIP_AUTOTUNE
