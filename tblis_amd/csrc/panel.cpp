@@ -1312,6 +1312,7 @@ bool lds_applicable(const std::vector<PanelGemm>& gemms, int family, int src_ele
             for (double x : g.kscale)
                 if (x != 1.0) return false;
         if (g.mlen.size() != 1 || g.nlen.size() != 1 || g.c.size() != 1) return false;
+        if (total_k(g) > INT32_MAX / 2) return false;  // (their k counters run past the end)
         if (g.a.size() != g.klen.size() || g.b.size() != g.klen.size()) return false;
         for (const std::vector<PBlock>* bl : {&g.a, &g.b})
         {
@@ -1429,7 +1430,7 @@ bool gather_tables(GatherWork& w, int tile, PanelTables& T, int64_t kslice)
         const PanelGemm& g = w.gemms[gi];
         const int64_t m = g.mlen[0], n = g.nlen[0], k = total_k(g);
         const int64_t MT = ceil_div(m, BM), NT = ceil_div(n, BN), mp = MT * BM, np = NT * BN;
-        if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX / 2) fail("contraction too large for one GEMM");
+        if (m > INT32_MAX || n > INT32_MAX) fail("contraction too large for one GEMM");
         T.useful_flops += 2 * m * n * k;
         T.mfma_flops += 2 * mp * np * (ceil_div(k, 4) * 4);
         if (k > 0) T.reads_ab = true;

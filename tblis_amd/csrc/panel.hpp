@@ -101,8 +101,8 @@ struct PanelTables
 };
 
 // Can the gather tiles (gemm_lds.hip) run these GEMMs: direct reads enabled,
-// one row block per operand, one C block, the same rows in every k block, and
-// each operand's offsets within 4 GiB?  Split-BF16 (gemm_gather_bf16.hip):
+// one row block per operand, one C block, the same rows in every k block,
+// fewer than 2^30 k and each operand's offsets within 4 GiB?  Split-BF16 (gemm_gather_bf16.hip):
 // also no scaled k block.  src_elem: bytes per tensor element.
 bool lds_applicable(const std::vector<PanelGemm>& gemms, int family, int src_elem);
 
