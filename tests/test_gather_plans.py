@@ -279,7 +279,7 @@ def test_planning_time_of_long_sums(dtype, monkeypatch):
     out = (C.c_int64 * HEADER)()  # too small: the plan is made, not copied out
     plan = best(lambda: T.lib().tblis_hip_debug_plan(None, *args, 1, out, HEADER))
     one = best(lambda: (words[1:] - words[:-1]).sum() + words.copy()[0])
-    assert plan <= 30 * one, (plan, one)
+    assert plan <= 40 * one, (plan, one)
 
 
 # (labels, extents, type, gather tile or not): both sides of the rules between
