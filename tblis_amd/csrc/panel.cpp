@@ -348,7 +348,7 @@ SplitTile split_tile(const std::vector<PanelGemm>& gemms, const double runs[2], 
     };
     constexpr Step steps[] = {
         {0, 256, 128, 12.5, 1.4, 0.22, 0.75, 0.0, 0.7, 15.0, 1.2, 0.074, 0.33, 0.95, 0.0},
-        {1, 128, 256, 9.0, 1.5, 0.20, 0.79, 0.0, 2.6, 13.0, 0.55, 0.06, 0.0, 0.0, 0.0},
+        {1, 128, 256, 9.0, 1.5, 0.21, 0.80, 0.0, 2.6, 13.0, 0.55, 0.06, 0.0, 0.0, 0.0},
         {2, 128, 128, 13.0, 1.4, 0.17, 0.56, 0.0, 2.3, 4.6, 0.4, 0.073, 0.0, 0.86, 0.0},
         {3, 64, 64, 9.0, 1.2, 0.0, 0.29, 0.44, 0.16, 0.23, 0.7, 0.076, 0.0, 0.0, 0.0},
         {4, 64, 64, 8.5, 1.55, 0.025, 0.22, 0.035, 0.0, 2.0, 0.0, 0.065, 0.26, 0.0, 0.30},
@@ -759,7 +759,7 @@ GatherChoice gather_choice(GatherWork& w, int cus, int only = -1)
         {FAMILY_F64, 1, false, 4, 1260, 2000, 6000, 1214, 1717, 3000, 0.045, 0.9, 0.060, 2.60, 3.5, 2.0},
         {FAMILY_F64, 2, false, 3, 960, 1300, 6000, 900, 1220, 4500, 0.055, 1.0, 0.012, 2.20, 3.5, 2.0},
         {FAMILY_BF16X3, 0, false, 2, 1534, 1880, 6000, 1455, 2095, 3800, 0.150, 1.5, 0.080, 7.10, 2.2, 2.1},
-        {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000, 1040, 1683, 5500, 0.200, 1.5, 0.045, 3.45, 2.0, 3.1}};
+        {FAMILY_BF16X3, 1, false, 3, 1000, 1715, 5000, 1040, 1683, 8500, 0.200, 1.5, 0.045, 2.05, 2.0, 3.1}};
     const bool f64 = family == FAMILY_F64, single = gemms.size() == 1;
     const double share = std::max(w.share[0], w.share[1]), most = 128.0 / src_elem;
     constexpr double kGHz = 2.15;
@@ -905,8 +905,10 @@ bool gather_preferred(const GatherWork& w, const GatherChoice& c, double packed)
     {
         // (the packed model is 10% short below 30 us, the pieces' one long)
         if (c.pieces) return 0.85 * c.us < packed;
+        // two models' ties go to the packed tile: 2401^3 floats, priced alike,
+        // packed 201, gathered 223; 1369^3 doubles 103, 111
         const bool large = !f64 && std::min(w.gemms[0].mlen[0], w.gemms[0].nlen[0]) >= 2048;
-        return !w.across && (large ? 1.06 : 1.0) * c.us < packed;
+        return !w.across && (large ? 1.09 : f64 ? 1.05 : 1.0) * c.us < packed;
     }
     if (c.pieces) return true;
     if (w.across) return false;

@@ -356,7 +356,7 @@ def test_reach_of_four_gib(back, dtype, elem):
 
 @pytest.mark.parametrize("m,n,k,dtype,tile", [
     (1225, 1225, 120, F64, 10), (33, 4489, 225, F64, 11), (2500, 31, 2499, F64, 11), (4489, 1225, 4489, F64, 8),
-    (2025, 2025, 2025, F64, 5), (1296, 1296, 1296, F32, 7), (2561, 2049, 1700, F32, 6), (4096, 4096, 2048, F32, 1),
+    (2025, 2025, 2025, F64, 5), (1296, 1296, 1296, F32, 7), (2561, 2049, 1700, F32, 6), (4096, 4096, 2048, F32, 0),
     (8192, 8192, 8192, F32, 0)])
 def test_tiles_picked(m, n, k, dtype, tile):
     """One size of each side of the lines between tiles."""
